@@ -276,6 +276,11 @@ int m2l_valu_parts(const DevicePlan& d, int K);
 int device_cu_count(int device);
 template <class S>
 void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s);
+// The vector-ALU near field (near_lanes.hip): any K, FP32 and FP64.
+template <class S>
+void launch_p2p_lanes(const DevicePlan& d, int K, bool potential, hipStream_t s);
+template <class S>
+void launch_p2p_grad_lanes(const DevicePlan& d, int K, hipStream_t s);
 // Leaf order of `count` points (device arrays; tree.hip): the stable sort by
 // leaf Morton index into permutation[sorted] = input index, and leaf_ranges
 // [2 * leaf] = {begin, end} (count, count for an empty leaf).

@@ -1,20 +1,17 @@
-// List-1 P2P (near field) and the FP64 direct sum.
+// List-1 P2P (near field) on the matrix cores, and the FP64 direct sum; the
+// vector-ALU near field is near_lanes.hip.
 //
 // Reference: the list-1 pair set of src/uniform_fmm.cpp:678-710 (every
 // source of the clipped 3x3x3 leaf neighbourhood of the target's leaf, the
 // identity pair skipped, coincident non-identity pairs giving NaN:
 // src/static_operators.cpp:435-446) with the point-dipole tensor
 // D = (3 r r^T/|r|^5 - I/|r|^3)/(4 pi) of src/cuboid.cpp:293-307.  The
-// reference stores one tensor per pair (37 GB at 2^20 points); here each
-// workgroup owns one target leaf, streams the neighbour leaves' sources
-// through LDS and evaluates the tensor on the fly, reusing every staged
-// source for all K moment states.
+// reference stores one tensor per pair (37 GB at 2^20 points); here the
+// tensor is evaluated on the fly and reused for all K moment states.
 //
 // FP32 plans carry positions as hi+lo float pairs of the FP64 operator-frame
 // coordinates, so r = (t_hi - s_hi) + (t_lo - s_lo) keeps FP32 relative
-// accuracy even for pairs far closer than a leaf width.  The field is formed
-// as f*(3(u.m)u - m) with u = r/|r| and f = |r|^-3/(4 pi), which avoids the
-// |r|^-5 overflow of close pairs in FP32.
+// accuracy even for pairs far closer than a leaf width.
 #include "common.hpp"
 #include "bf16_split.hpp"
 
@@ -23,7 +20,6 @@ namespace hipfmm {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSlots = 32;  // target slots per pass; 8 thread groups per slot
 
 template <class S>
 struct PairPos;
@@ -42,133 +38,7 @@ struct PairPos<float> {
   }
 };
 
-template <>
-struct PairPos<double> {
-  double4 hi;
-  __device__ static PairPos load(const void* pos, int, int i) { return {static_cast<const double4*>(pos)[i]}; }
-  __device__ inline void diff(const PairPos& s, double& x, double& y, double& z) const {
-    x = hi.x - s.hi.x;
-    y = hi.y - s.hi.y;
-    z = hi.z - s.hi.z;
-  }
-};
-
 __device__ inline float inv_sqrt(float x) { return __frsqrt_rn(x); }
-__device__ inline double inv_sqrt(double x) { return 1.0 / sqrt(x); }
-
-// Workgroup per target leaf.  Thread = (slot, group); group g handles the k
-// range [kg*KPT, kg*KPT+KPT) and the sources j with j % SP == sp, where
-// KG = number of k groups and SP = 8 / KG source splits.  With kPot the
-// potential phi += (m.r)|r|^-3/(4 pi) (src/static_operators.cpp:455-463,
-// src/near_field.cpp:30-80) is accumulated beside the field into Pn[t][k].
-template <class S, int KPT, bool kPot>
-__global__ void __launch_bounds__(kThreads) p2p_kernel(const DevicePlan d, int K, int KG, int chunk) {
-  extern __shared__ unsigned char smem_raw[];
-  auto* spos = reinterpret_cast<PairPos<S>*>(smem_raw);       // chunk
-  S* smom = reinterpret_cast<S*>(spos + chunk);                // chunk x 3 x K
-  S* red = smom;                                               // reused for the split reduction
-  const int leaf = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x));
-  const int2 trange = d.leaf_tgt[leaf];
-  if (trange.x == trange.y) return;
-  const int slot = threadIdx.x % kSlots, g = threadIdx.x / kSlots;
-  const int SP = 8 / KG;
-  const int kg = g % KG, sp = g / KG;
-  const int nb = 1 << d.L;
-  int lx, ly, lz;
-  demorton3(uint32_t(leaf), d.L, lx, ly, lz);
-  const S c4pi = S(0.079577471545947667884441881686257181);  // 1/(4 pi)
-  const S* sm = static_cast<const S*>(d.sm);
-  S* Hn = static_cast<S*>(d.Hn);
-  constexpr int C = kPot ? 4 : 3;  // accumulated rows per (target, state)
-  for (int t0 = trange.x; t0 < trange.y; t0 += kSlots) {
-    const int t = t0 + slot;
-    const bool active = t < trange.y;
-    const PairPos<S> tp = PairPos<S>::load(d.tgt_pos, d.nt, active ? t : trange.x);
-    const int self = active ? d.self[t] : -2;
-    S acc[KPT][C];
-#pragma unroll
-    for (int q = 0; q < KPT; ++q)
-#pragma unroll
-      for (int c = 0; c < C; ++c) acc[q][c] = S(0);
-    for (int dz = -1; dz <= 1; ++dz)
-      for (int dy = -1; dy <= 1; ++dy)
-        for (int dx = -1; dx <= 1; ++dx) {
-          const int x = lx + dx, y = ly + dy, z = lz + dz;
-          if (x < 0 || y < 0 || z < 0 || x >= nb || y >= nb || z >= nb) continue;
-          const int2 sr = d.leaf_src[morton3(uint32_t(x), uint32_t(y), uint32_t(z), d.L)];
-          for (int j0 = sr.x; j0 < sr.y; j0 += chunk) {
-            const int cnt = min(chunk, sr.y - j0);
-            __syncthreads();
-            for (int w = threadIdx.x; w < cnt; w += kThreads) spos[w] = PairPos<S>::load(d.src_pos, d.ns, j0 + w);
-            for (int w = threadIdx.x; w < cnt * 3 * K; w += kThreads) smom[w] = sm[int64_t(j0) * 3 * K + w];
-            __syncthreads();
-            if (active) {
-              for (int j = sp; j < cnt; j += SP) {
-                if (j0 + j == self) continue;
-                S rx, ry, rz;
-                tp.diff(spos[j], rx, ry, rz);
-                const S r2 = rx * rx + ry * ry + rz * rz;
-                const S rinv = inv_sqrt(r2);
-                const S f = rinv * rinv * rinv * c4pi;
-                const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
-                const S* mj = smom + j * 3 * K + kg * KPT;
-#pragma unroll
-                for (int q = 0; q < KPT; ++q) {
-                  if (kg * KPT + q < K) {
-                    const S mx = mj[q], my = mj[K + q], mz = mj[2 * K + q];
-                    const S mu3 = S(3) * (ux * mx + uy * my + uz * mz);
-                    acc[q][0] += f * (mu3 * ux - mx);
-                    acc[q][1] += f * (mu3 * uy - my);
-                    acc[q][2] += f * (mu3 * uz - mz);
-                    if constexpr (kPot) acc[q][C - 1] += f * (rx * mx + ry * my + rz * mz);
-                  }
-                }
-              }
-            }
-          }
-        }
-    // Reduce the SP source splits (fixed order) and store Hn[t][c][k].
-    __syncthreads();
-    if (SP > 1) {
-      for (int q = 0; q < KPT; ++q)
-        for (int c = 0; c < C; ++c) red[((g * kSlots + slot) * KPT + q) * C + c] = acc[q][c];
-      __syncthreads();
-      if (sp == 0 && active) {
-        for (int s2 = 1; s2 < SP; ++s2) {
-          const int g2 = s2 * KG + kg;
-          for (int q = 0; q < KPT; ++q)
-            for (int c = 0; c < C; ++c) acc[q][c] += red[((g2 * kSlots + slot) * KPT + q) * C + c];
-        }
-      }
-    }
-    if (sp == 0 && active) {
-      for (int q = 0; q < KPT; ++q) {
-        const int k = kg * KPT + q;
-        if (k < K) {
-          for (int c = 0; c < 3; ++c) Hn[(int64_t(t) * 3 + c) * K + k] = acc[q][c];
-          if constexpr (kPot) static_cast<S*>(d.Pn)[int64_t(t) * K + k] = acc[q][C - 1];
-        }
-      }
-    }
-  }
-}
-
-template <class S, int KPT>
-void launch_p2p_t(const DevicePlan& d, int K, bool potential, hipStream_t s) {
-  int KG = (K + KPT - 1) / KPT;
-  int kg = 1;
-  while (kg < KG) kg *= 2;  // 1, 2, 4 or 8 k groups
-  const int chunk = sizeof(S) == 4 ? 64 : 32;
-  const size_t stage = size_t(chunk) * sizeof(PairPos<S>) + size_t(chunk) * 3 * K * sizeof(S);
-  // The cross-group reduction runs only when several groups share a state
-  // group (kg < 8).
-  const size_t reduce = kg < 8 ? size_t(8) * kSlots * KPT * 4 * sizeof(S) + size_t(chunk) * sizeof(PairPos<S>) : 0;
-  if (potential)
-    p2p_kernel<S, KPT, true><<<unsigned(d.leaves), kThreads, std::max(stage, reduce), s>>>(d, K, kg, chunk);
-  else
-    p2p_kernel<S, KPT, false><<<unsigned(d.leaves), kThreads, std::max(stage, reduce), s>>>(d, K, kg, chunk);
-  HIPFMM_CHECK(hipGetLastError());
-}
 
 // FP64 direct field, one thread per target, sources staged through LDS.
 // validation.cpp:71-111 / operators.cpp:178-220; model kernel
@@ -752,127 +622,10 @@ void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s) {
       return;
     }
   }
-  if (K <= 8)
-    launch_p2p_t<S, 1>(d, K, potential, s);
-  else if (K <= 32)
-    launch_p2p_t<S, 4>(d, K, potential, s);
-  else
-    launch_p2p_t<S, 8>(d, K, potential, s);
+  launch_p2p_lanes<S>(d, K, potential, s);
 }
 template void launch_p2p<float>(const DevicePlan&, int, bool, hipStream_t);
 template void launch_p2p<double>(const DevicePlan&, int, bool, hipStream_t);
-
-namespace {
-
-// Near-field gradient of the field, G_cj = dH_c/dx_j of every target over
-// its list-1 sources (no counterpart in the reference; the derivative of its
-// pair tensor, src/cuboid.cpp:293-307): with r = x_t - x_s, u = r/|r|,
-// w = u.m and g = 3/(4 pi |r|^4),
-//   G_cj += g (delta_cj w + u_c m_j + m_c u_j - 5 u_c u_j w),
-// symmetric and traceless; entries xx xy xz yy yz zz.  Identity pair skipped,
-// coincident pairs NaN.  Workgroup per target leaf as the field kernel:
-// thread (slot, state group), sources staged in LDS, into Gn[t][6][K].
-template <class S, int KPT>
-__global__ void __launch_bounds__(kThreads) p2p_grad_kernel(const DevicePlan d, int K, int KG, int chunk) {
-  extern __shared__ unsigned char smem_raw[];
-  auto* spos = reinterpret_cast<PairPos<S>*>(smem_raw);  // chunk
-  S* smom = reinterpret_cast<S*>(spos + chunk);           // chunk x 3 x K
-  const int leaf = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x));
-  const int2 trange = d.leaf_tgt[leaf];
-  if (trange.x == trange.y) return;
-  const int slot = threadIdx.x % kSlots, g = threadIdx.x / kSlots;
-  const int kg = g % KG, sp = g / KG, SP = 8 / KG;
-  const int nb = 1 << d.L;
-  int lx, ly, lz;
-  demorton3(uint32_t(leaf), d.L, lx, ly, lz);
-  const S c34pi = S(0.23873241463784300365332564505877154);  // 3/(4 pi)
-  const S* sm = static_cast<const S*>(d.sm);
-  S* Gn = static_cast<S*>(d.Gn);
-  S* red = smom;
-  for (int t0 = trange.x; t0 < trange.y; t0 += kSlots) {
-    const int t = t0 + slot;
-    const bool active = t < trange.y;
-    const PairPos<S> tp = PairPos<S>::load(d.tgt_pos, d.nt, active ? t : trange.x);
-    const int self = active ? d.self[t] : -2;
-    S acc[KPT][6];
-#pragma unroll
-    for (int q = 0; q < KPT; ++q)
-#pragma unroll
-      for (int e = 0; e < 6; ++e) acc[q][e] = S(0);
-    for (int dz = -1; dz <= 1; ++dz)
-      for (int dy = -1; dy <= 1; ++dy)
-        for (int dx = -1; dx <= 1; ++dx) {
-          const int x = lx + dx, y = ly + dy, z = lz + dz;
-          if (x < 0 || y < 0 || z < 0 || x >= nb || y >= nb || z >= nb) continue;
-          const int2 sr = d.leaf_src[morton3(uint32_t(x), uint32_t(y), uint32_t(z), d.L)];
-          for (int j0 = sr.x; j0 < sr.y; j0 += chunk) {
-            const int cnt = min(chunk, sr.y - j0);
-            __syncthreads();
-            for (int w = threadIdx.x; w < cnt; w += kThreads) spos[w] = PairPos<S>::load(d.src_pos, d.ns, j0 + w);
-            for (int w = threadIdx.x; w < cnt * 3 * K; w += kThreads) smom[w] = sm[int64_t(j0) * 3 * K + w];
-            __syncthreads();
-            if (active) {
-              for (int j = sp; j < cnt; j += SP) {
-                if (j0 + j == self) continue;
-                S rx, ry, rz;
-                tp.diff(spos[j], rx, ry, rz);
-                const S r2 = rx * rx + ry * ry + rz * rz;
-                const S rinv = inv_sqrt(r2);
-                const S gg = c34pi * rinv * rinv * rinv * rinv;
-                const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
-                const S* mj = smom + j * 3 * K + kg * KPT;
-#pragma unroll
-                for (int q = 0; q < KPT; ++q) {
-                  if (kg * KPT + q < K) {
-                    const S mx = mj[q], my = mj[K + q], mz = mj[2 * K + q];
-                    const S w = ux * mx + uy * my + uz * mz;
-                    const S w5 = S(5) * w;
-                    acc[q][0] += gg * (w + S(2) * ux * mx - w5 * ux * ux);
-                    acc[q][1] += gg * (ux * my + mx * uy - w5 * ux * uy);
-                    acc[q][2] += gg * (ux * mz + mx * uz - w5 * ux * uz);
-                    acc[q][3] += gg * (w + S(2) * uy * my - w5 * uy * uy);
-                    acc[q][4] += gg * (uy * mz + my * uz - w5 * uy * uz);
-                    acc[q][5] += gg * (w + S(2) * uz * mz - w5 * uz * uz);
-                  }
-                }
-              }
-            }
-          }
-        }
-    __syncthreads();
-    if (SP > 1) {
-      for (int q = 0; q < KPT; ++q)
-        for (int e = 0; e < 6; ++e) red[((g * kSlots + slot) * KPT + q) * 6 + e] = acc[q][e];
-      __syncthreads();
-      if (sp == 0 && active)
-        for (int s2 = 1; s2 < SP; ++s2) {
-          const int g2 = s2 * KG + kg;
-          for (int q = 0; q < KPT; ++q)
-            for (int e = 0; e < 6; ++e) acc[q][e] += red[((g2 * kSlots + slot) * KPT + q) * 6 + e];
-        }
-    }
-    if (sp == 0 && active)
-      for (int q = 0; q < KPT; ++q) {
-        const int k = kg * KPT + q;
-        if (k < K)
-          for (int e = 0; e < 6; ++e) Gn[(int64_t(t) * 6 + e) * K + k] = acc[q][e];
-      }
-  }
-}
-
-template <class S, int KPT>
-void launch_p2p_grad_t(const DevicePlan& d, int K, hipStream_t s) {
-  int KG = (K + KPT - 1) / KPT;
-  int kg = 1;
-  while (kg < KG) kg *= 2;
-  const int chunk = sizeof(S) == 4 ? 64 : 32;
-  const size_t stage = size_t(chunk) * sizeof(PairPos<S>) + size_t(chunk) * 3 * K * sizeof(S);
-  const size_t reduce = kg < 8 ? size_t(8) * kSlots * KPT * 6 * sizeof(S) + size_t(chunk) * sizeof(PairPos<S>) : 0;
-  p2p_grad_kernel<S, KPT><<<unsigned(d.leaves), kThreads, std::max(stage, reduce), s>>>(d, K, kg, chunk);
-  HIPFMM_CHECK(hipGetLastError());
-}
-
-}  // namespace
 
 // acc[E] += W m_D over both state halves, for one entry of W (its pieces)
 // and the moments' component D.
@@ -1117,12 +870,7 @@ void launch_p2p_grad(const DevicePlan& d, int K, hipStream_t s) {
       return;
     }
   }
-  if (K <= 8)
-    launch_p2p_grad_t<S, 1>(d, K, s);
-  else if (K <= 32)
-    launch_p2p_grad_t<S, 4>(d, K, s);
-  else
-    launch_p2p_grad_t<S, 8>(d, K, s);
+  launch_p2p_grad_lanes<S>(d, K, s);
 }
 template void launch_p2p_grad<float>(const DevicePlan&, int, hipStream_t);
 template void launch_p2p_grad<double>(const DevicePlan&, int, hipStream_t);

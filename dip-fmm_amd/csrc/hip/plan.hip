@@ -1125,13 +1125,17 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   } else if (mfma) {
     hipfmm::launch_m2l_split(d, K, P->m2l_mode, s);
   }
-  // From K = 32 on, the matrix-core M2L starts once the near field is done.
-  // Both kernels then fill the chip and are bound by instruction issue, so
-  // one after the other they take as long as side by side (measured within
-  // noise), and the M2L runs alone; the upward pass before this point still
-  // runs beside the near field.  A smaller batch gives the M2L too few
-  // workgroups to fill the chip, and it keeps running beside the near field.
-  if (mfma && K >= 32) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
+  // From K = 32 on, the matrix-core M2L starts once the near field is done,
+  // and the vector-ALU M2L always does.  Both kernels then fill the chip and
+  // are bound by instruction issue, so one after the other they take as long
+  // as side by side (measured within noise), and the M2L runs alone; the
+  // upward pass before this point still runs beside the near field.  The
+  // vector-ALU M2L's few, long workgroups must start on an empty chip: placed
+  // around the near field's last workgroups they crowd some CUs (2^20 points,
+  // p = 6, one state: M2L 2.04 ms beside the near field's tail, 1.24 ms after
+  // it).  A smaller matrix-core batch has too few workgroups to fill the chip
+  // and keeps running beside the near field.
+  if (!mfma || K >= 32) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
   mark(kEvM2LKernel0, s);
   const int ring_slot = int(P->m2l_launch_count % hipfmm_plan::kRing);
   drain_m2l_slot(P, ring_slot);
