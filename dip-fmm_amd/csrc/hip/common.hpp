@@ -198,7 +198,6 @@ struct DevicePlan {
   void* Pn = nullptr;          // near-field potential Pn[target][K] (allocated once a potential is asked for)
   void* Gn = nullptr;          // near-field field gradient Gn[target][6][K] (allocated once asked for)
   void* gradients_out = nullptr;  // host-path staging: K x nt x 6
-  int* grad_tab = nullptr;     // [n][6]: index of b - e_c - e_j (xx xy xz yy yz zz), or -1
   int* grad_up = nullptr;      // [g][8], g of degree <= p - 2: index of g + e_c + e_j (6 used)
   double potential_scale = 1.0;  // frame factor of the potential (root width W for FP32 plans)
   // Harmonic-subspace M2L: L = Q sum_o C_o P M with the level scalings folded
@@ -321,12 +320,29 @@ template <class S>
 void launch_l2p_unsort(const DevicePlan& d, S* fields, S* potentials, int K, hipStream_t s);
 template <class S>
 void launch_zero(S* ptr, size_t count, hipStream_t s);
+// The same operations for any number of states, FP32 and FP64 (columns.hip):
+// what the launchers above use where the batch is no multiple of 32 FP32
+// states.
+template <class S>
+void launch_p2m_columns(const DevicePlan& d, int K, hipStream_t s);
+template <class S>
+void launch_m2m_columns(const DevicePlan& d, int parent_level, int K, hipStream_t s);
+template <class S>
+void launch_l2l_columns(const DevicePlan& d, int child_level, int K, hipStream_t s);
+template <class S>
+void launch_compress_columns(const DevicePlan& d, int level, int K, hipStream_t s);
+template <class S>
+void launch_expand_columns(const DevicePlan& d, int level, int K, hipStream_t s);
+template <class S>
+void launch_l2p_columns(const DevicePlan& d, S* fields, S* potentials, int K, hipStream_t s);
+template <class S>
+void launch_l2p_grad_columns(const DevicePlan& d, S* gradients, int K, hipStream_t s);
 
 void launch_m2l_split(const DevicePlan& d, int K, int mode, hipStream_t s);  // all levels 2..L
 // Harmonic-subspace transforms around the M2L, levels first_level..L (at
-// least 2): M -> Mc (or the MFMA split layout when `split`), and Lcc -> Lc.
+// least 2): M -> Mc, and Lcc -> Lc.
 template <class S>
-void launch_m2l_compress(const DevicePlan& d, int K, bool split, int first_level, hipStream_t s);
+void launch_m2l_compress(const DevicePlan& d, int K, int first_level, hipStream_t s);
 template <class S>
 void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t s);
 // bf16 hi/lo split of the compressed multipoles (levels 2..L) into the MFMA

@@ -1,14 +1,10 @@
-// Far-field kernels of the HipFull path: moment gather, leaf P2M, level-wise
-// M2M and L2L, and leaf L2P fused with the near-field combine and the unsort
-// to user target order.  One workgroup owns one box (P2M, L2P) or one parent
-// box (M2M, L2L), reads its inputs once and writes its outputs once, with no
-// atomics.
-//
-// Each operation is a small dense product per box, computed as a register-
-// tiled GEMM on the vector ALUs (FP32 or FP64 FMA, no reduced precision):
-// a thread owns an 8-row x 4-state tile of the output and, per depth step,
-// reads 8 operator entries and 4 state values as 16-byte vectors from LDS or
-// L2 (3 vector loads per 32 FMAs at FP32).
+// Far-field kernels of the HipFull path on the matrix cores for FP32 plans with
+// a multiple of 32 moment states: leaf P2M, level-wise M2M and L2L, the
+// harmonic compression and expansion, and leaf L2P with the near-field
+// combine; the moment gather and the unsorts; and the dispatch between these
+// and the kernels of columns.hip, which serve every other number of states and
+// FP64.  One workgroup owns one box (P2M, L2P) or one parent box (M2M, L2L),
+// reads its inputs once and writes its outputs once, with no atomics.
 //
 // Reference operations restated here:
 //   permute_moments / prepare_moments_float   src/cuda_fmm.cu:56-64, src/far_field.cpp:334-365
@@ -19,8 +15,6 @@
 //   L2P   H_c = -sum_{b: b_c>0} L_b dx^(b-e_c)/(b-e_c)!
 //         src/static_operators.cpp:300-335
 //   combine + unsort  src/cuda_fmm.cu:503-516, src/uniform_fmm.cpp:1439-1452
-#include <type_traits>
-
 #include "common.hpp"
 #include "bf16_split.hpp"
 
@@ -29,90 +23,8 @@ namespace hipfmm {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRA = 8;  // output rows per thread tile
-constexpr int kRK = 4;  // moment states per thread tile
 
 __host__ __device__ inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
-__host__ __device__ inline size_t align16(size_t bytes) { return (bytes + 15) & ~size_t(15); }
-
-// d^g/g! for one axis, g <= p, by the recurrence x^i/i! = x^(i-1)/(i-1)! * x / i.
-template <class S>
-__device__ inline S axis_power(S x, int g) {
-  S v = S(1);
-  for (int i = 1; i <= g; ++i) v = v * x / S(i);
-  return v;
-}
-
-// bf16 bits of x, round to nearest even (inf / nan keep their class).
-__device__ inline uint16_t bf16_round(float x) {
-  uint32_t u = __builtin_bit_cast(uint32_t, x);
-  if ((u & 0x7f800000u) == 0x7f800000u) return uint16_t(u >> 16);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return uint16_t(u >> 16);
-}
-
-// R consecutive scalars from 16-byte aligned memory (LDS or global).
-template <class S, int R>
-__device__ __forceinline__ void load_vec(const S* p, S (&out)[R]) {
-  if constexpr (sizeof(S) == 4) {
-#pragma unroll
-    for (int i = 0; i < R; i += 4) {
-      const float4 t = *reinterpret_cast<const float4*>(p + i);
-      out[i] = t.x;
-      out[i + 1] = t.y;
-      out[i + 2] = t.z;
-      out[i + 3] = t.w;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < R; i += 2) {
-      const double2 t = *reinterpret_cast<const double2*>(p + i);
-      out[i] = t.x;
-      out[i + 1] = t.y;
-    }
-  }
-}
-
-// acc[i][j] += sum_d A[d*lda + i] * B[d*ldb + j]: A and B already point at
-// the thread's first row / state; both 16-byte aligned per depth step.
-template <class S>
-__device__ __forceinline__ void tile_gemm(const S* __restrict__ A, int lda, const S* __restrict__ B, int ldb,
-                                          int depth, S (&acc)[kRA][kRK]) {
-#pragma unroll 4
-  for (int dd = 0; dd < depth; ++dd) {
-    S a[kRA], b[kRK];
-    load_vec<S, kRA>(A + size_t(dd) * lda, a);
-    load_vec<S, kRK>(B + size_t(dd) * ldb, b);
-#pragma unroll
-    for (int i = 0; i < kRA; ++i)
-#pragma unroll
-      for (int j = 0; j < kRK; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-  }
-}
-
-// Rows [n_rows) x columns [KCn) of a box's coefficient block C[row][ld]
-// (C offset to the first column) from a tile accumulator; kAdd accumulates
-// into the existing values.
-template <class S, bool kAdd>
-__device__ __forceinline__ void store_tile(S* __restrict__ C, int row0, int n_rows, int k0, int KCn, int ld,
-                                           const S (&acc)[kRA][kRK]) {
-#pragma unroll
-  for (int i = 0; i < kRA; ++i) {
-    const int row = row0 + i;
-    if (row >= n_rows) break;
-    S* dst = C + size_t(row) * ld + k0;
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) {
-      if (k0 + j >= KCn) break;
-      const S v = acc[i][j];
-      if constexpr (kAdd)
-        dst[j] += v;
-      else
-        dst[j] = v;
-    }
-  }
-}
-
 // Moments from the user layout [k][user][3] into the sorted state layout
 // sm[sorted][3][K], times the frame factor.  A workgroup owns `points`
 // consecutive user points: it reads their rows of every state (3 * points
@@ -223,123 +135,6 @@ __global__ void __launch_bounds__(kThreads) scatter_potentials_kernel(const floa
   }
 }
 
-// Shared LDS layout of the monomial-based kernels (P2M, L2P).
-struct MonoLayout {
-  int NP, KP, JC, TCP;
-  size_t off_tab, off_ex, off_px, off_mono, off_a, off_b, bytes;
-};
-
-// P2M layout: tab[n] int4, ex[nm] int4, px[JC][3][p], mono[JC][nm],
-// A[3*JC][NP] (row = (source, component), column = alpha), B[3*JC][KP].
-template <class S>
-MonoLayout p2m_layout(const DevicePlan& d, int KC) {
-  MonoLayout l{};
-  l.NP = round_up(d.n, kRA);
-  l.KP = round_up(KC, kRK);
-  l.JC = sizeof(S) == 4 ? 16 : 8;
-  size_t o = 0;
-  l.off_tab = o;
-  o += align16(size_t(d.n) * sizeof(int4));
-  l.off_ex = o;
-  o += align16(size_t(std::max(d.nm, 1)) * sizeof(int4));
-  l.off_px = o;
-  o += align16(size_t(l.JC) * 3 * std::max(d.p, 1) * sizeof(S));
-  l.off_mono = o;
-  o += align16(size_t(l.JC) * std::max(d.nm, 1) * sizeof(S));
-  l.off_a = o;
-  o += align16(size_t(3 * l.JC) * l.NP * sizeof(S));
-  l.off_b = o;
-  o += align16(size_t(3 * l.JC) * l.KP * sizeof(S));
-  l.bytes = o;
-  return l;
-}
-
-// One workgroup per (leaf, chunk of KC states):
-//   M[alpha][k] = sign(alpha) sum_{(j,c)} A[(j,c)][alpha] B[(j,c)][k]
-// with A[(j,c)][alpha] = d_j^(alpha-e_c)/(alpha-e_c)! (0 unless alpha_c > 0)
-// and B[(j,c)][k] = m_jc (state k); sources in chunks of JC.
-template <class S>
-__global__ void __launch_bounds__(1024) p2m_kernel(const DevicePlan d, int K, int KC, MonoLayout l) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  int4* tab = reinterpret_cast<int4*>(smem_raw + l.off_tab);
-  int4* ex = reinterpret_cast<int4*>(smem_raw + l.off_ex);
-  S* px = reinterpret_cast<S*>(smem_raw + l.off_px);
-  S* mono = reinterpret_cast<S*>(smem_raw + l.off_mono);
-  S* A = reinterpret_cast<S*>(smem_raw + l.off_a);
-  S* B = reinterpret_cast<S*>(smem_raw + l.off_b);
-  const int n = d.n, nm = d.nm, p = d.p, NP = l.NP, KP = l.KP, JC = l.JC;
-  const int tid = threadIdx.x, T = blockDim.x;
-  const int KT = KP / kRK;
-  const int at = tid / KT, kt = tid % KT;
-  const bool active = at < NP / kRA;
-  const int leaf = blockIdx.x;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  const int2 range = d.leaf_src[leaf];
-  const int64_t node = level_offset(d.L) + leaf;
-  for (int i = tid; i < n; i += T) tab[i] = d.p2m_tab[i];
-  for (int i = tid; i < nm; i += T) ex[i] = d.p2m_tab[n + i];
-  S acc[kRA][kRK];
-#pragma unroll
-  for (int i = 0; i < kRA; ++i)
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) acc[i][j] = S(0);
-  const auto* rel = static_cast<const typename Vec4<S>::type*>(d.src_rel);
-  const S* sm = static_cast<const S*>(d.sm);
-  for (int j0 = range.x; j0 < range.y; j0 += JC) {
-    const int cnt = min(JC, range.y - j0);
-    __syncthreads();  // previous chunk's products done; tables visible
-    if (tid < 3 * JC) {
-      const int j = tid / 3, a = tid % 3;
-      S x = S(0);
-      if (j < cnt) {
-        const auto r = rel[j0 + j];
-        x = a == 0 ? r.x : (a == 1 ? r.y : r.z);
-      }
-      S* row = px + (j * 3 + a) * p;
-      for (int i = 0; i < p; ++i) row[i] = axis_power<S>(x, i);
-    }
-    for (int w = tid; w < 3 * JC * KP; w += T) {
-      const int row = w / KP, k = w - row * KP;
-      const int j = row / 3, c = row - 3 * j;
-      B[w] = (j < cnt && k < KCn) ? sm[(int64_t(j0 + j) * 3 + c) * K + kc0 + k] : S(0);
-    }
-    __syncthreads();
-    for (int g = tid; g < nm; g += T) {
-      const int4 e = ex[g];
-      for (int j = 0; j < JC; ++j) {
-        const S* pj = px + j * 3 * p;
-        mono[j * nm + g] = pj[e.x] * pj[p + e.y] * pj[2 * p + e.z];
-      }
-    }
-    __syncthreads();
-    for (int alpha = tid; alpha < NP; alpha += T) {
-      const int4 t = alpha < n ? tab[alpha] : int4{-1, -1, -1, 0};
-      for (int j = 0; j < JC; ++j) {
-        const S* mj = mono + j * nm;
-        const bool ok = j < cnt;
-        A[(3 * j + 0) * NP + alpha] = ok && t.x >= 0 ? mj[t.x] : S(0);
-        A[(3 * j + 1) * NP + alpha] = ok && t.y >= 0 ? mj[t.y] : S(0);
-        A[(3 * j + 2) * NP + alpha] = ok && t.z >= 0 ? mj[t.z] : S(0);
-      }
-    }
-    __syncthreads();
-    if (active) tile_gemm<S>(A + at * kRA, NP, B + kt * kRK, KP, 3 * min(cnt, JC), acc);
-  }
-  if (!active) return;
-  S* M = static_cast<S*>(d.M) + node * int64_t(n) * K + kc0;
-#pragma unroll
-  for (int i = 0; i < kRA; ++i) {
-    const int alpha = at * kRA + i;
-    if (alpha >= n) break;
-    const S sign = d.p2m_tab[alpha].w > 0 ? S(1) : S(-1);
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) {
-      const int k = kt * kRK + j;
-      if (k < KCn) M[int64_t(alpha) * K + k] = sign * acc[i][j];
-    }
-  }
-}
-
 // Dense transposed shift operators: T[(level*8 + class)][col][NP], row
 // (output coefficient) contiguous, rows n..NP-1 zero.
 template <class S>
@@ -347,373 +142,10 @@ __device__ __forceinline__ const S* shift_operator(const void* dense, int level,
   return static_cast<const S*>(dense) + (size_t(level) * 8 + cls) * size_t(n) * NP;
 }
 
-// Copy columns [0, KCn) of box coefficients C[n][ld] (global; C already
-// offset to the first column) into LDS B[n][KP], zero-padded.
-template <class S>
-__device__ __forceinline__ void stage_box(S* __restrict__ B, const S* __restrict__ C, int n, int ld, int KCn,
-                                          int KP) {
-  const int tid = threadIdx.x, T = blockDim.x;
-  constexpr int V = 16 / sizeof(S);
-  if (KCn == KP && ld % V == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0) {
-    using V4 = typename std::conditional<sizeof(S) == 4, float4, double2>::type;
-    const int vpr = KP / V;  // vectors per row
-    for (int w = tid; w < n * vpr; w += T) {
-      const int row = w / vpr, v = w - row * vpr;
-      reinterpret_cast<V4*>(B)[w] = *reinterpret_cast<const V4*>(C + size_t(row) * ld + v * V);
-    }
-  } else {
-    for (int w = tid; w < n * KP; w += T) {
-      const int row = w / KP, k = w - row * KP;
-      B[w] = k < KCn ? C[size_t(row) * ld + k] : S(0);
-    }
-  }
-}
-
-// One workgroup per parent at `level`: M_parent = sum_c T_c M_child(c).
-template <class S>
-__global__ void __launch_bounds__(1024) m2m_kernel(const DevicePlan d, int level, int K, int KC, int KP) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  S* B = reinterpret_cast<S*>(smem_raw);  // [n][KP]
-  const int n = d.n, NP = round_up(n, kRA), KT = KP / kRK;
-  const int tid = threadIdx.x;
-  const int at = tid / KT, kt = tid % KT;
-  const bool active = at < NP / kRA;
-  const int64_t parent = blockIdx.x;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  const int64_t cnode0 = level_offset(level + 1) + parent * 8;
-  const S* M = static_cast<const S*>(d.M) + kc0;
-  S acc[kRA][kRK];
-#pragma unroll
-  for (int i = 0; i < kRA; ++i)
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) acc[i][j] = S(0);
-  for (int c = 0; c < 8; ++c) {
-    __syncthreads();
-    stage_box<S>(B, M + (cnode0 + c) * int64_t(n) * K, n, K, KCn, KP);
-    __syncthreads();
-    if (active) tile_gemm<S>(shift_operator<S>(d.m2m_dense, level + 1, c, n, NP) + at * kRA, NP, B + kt * kRK, KP, n, acc);
-  }
-  if (active)
-    store_tile<S, false>(static_cast<S*>(d.M) + (level_offset(level) + parent) * int64_t(n) * K + kc0, at * kRA, n,
-                         kt * kRK, KCn, K, acc);
-}
-
-// One workgroup per parent at child_level - 1: L_child(c) += T_c L_parent.
-template <class S>
-__global__ void __launch_bounds__(1024) l2l_kernel(const DevicePlan d, int child_level, int K, int KC, int KP) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  S* B = reinterpret_cast<S*>(smem_raw);  // [n][KP]
-  const int n = d.n, NP = round_up(n, kRA), KT = KP / kRK;
-  const int tid = threadIdx.x;
-  const int at = tid / KT, kt = tid % KT;
-  const bool active = at < NP / kRA;
-  const int64_t parent = blockIdx.x;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  S* Lc = static_cast<S*>(d.Lc) + kc0;
-  stage_box<S>(B, Lc + (level_offset(child_level - 1) + parent) * int64_t(n) * K, n, K, KCn, KP);
-  __syncthreads();
-  if (!active) return;
-  for (int c = 0; c < 8; ++c) {
-    S acc[kRA][kRK];
-#pragma unroll
-    for (int i = 0; i < kRA; ++i)
-#pragma unroll
-      for (int j = 0; j < kRK; ++j) acc[i][j] = S(0);
-    tile_gemm<S>(shift_operator<S>(d.l2l_dense, child_level, c, n, NP) + at * kRA, NP, B + kt * kRK, KP, n, acc);
-    const int64_t child = level_offset(child_level) + parent * 8 + c;
-    store_tile<S, true>(Lc + child * int64_t(n) * K, at * kRA, n, kt * kRK, KCn, K, acc);
-  }
-}
-
-constexpr int kL2PTargets = 32;  // targets per chunk
-constexpr int kL2PRT = 2;        // targets per thread tile
-
-// L2P layout: tab[n] int4, ex[NM] int4, px[TC][3][PW], monoT[NM][TC],
-// Lb[n][KP] (the leaf local).  Fields need the NM = nm monomials of degree
-// < p (powers up to p-1); the potential needs all n (powers up to p).
-template <class S>
-MonoLayout l2p_layout(const DevicePlan& d, int KC, bool potential) {
-  MonoLayout l{};
-  l.NP = round_up(d.n, kRA);
-  l.KP = round_up(KC, kRK);
-  l.TCP = kL2PTargets;
-  const int NM = potential ? d.n : d.nm, PW = potential ? d.p + 1 : d.p;
-  size_t o = 0;
-  l.off_tab = o;
-  o += align16(size_t(d.n) * sizeof(int4));
-  l.off_ex = o;
-  o += align16(size_t(std::max(NM, 1)) * sizeof(int4));
-  l.off_px = o;
-  o += align16(size_t(l.TCP) * 3 * std::max(PW, 1) * sizeof(S));
-  l.off_mono = o;
-  o += align16(size_t(std::max(NM, 1)) * l.TCP * sizeof(S));
-  l.off_b = o;
-  o += align16(size_t(d.n) * l.KP * sizeof(S));
-  l.bytes = o;
-  return l;
-}
-
-// One workgroup per target leaf: far field from the leaf local,
-//   H[t][c][k] = -sum_b L[b][k] d_t^(b-e_c)/(b-e_c)!
-// (src/static_operators.cpp:300-335), a thread owning 2 targets x 4 states x
-// 3 components; plus the near field, written to out[k][user target][3].
-// With kPot also the potential phi[t][k] = sum_b L[b][k] d_t^b/b! plus the
-// near-field potential, times the frame factor, to pot[k][user target]
-// (out may then be null).
-template <class S, bool kPot>
-__global__ void __launch_bounds__(1024) l2p_kernel(const DevicePlan d, S* __restrict__ out, S* __restrict__ pot, int K,
-                                                   int KC, MonoLayout l) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  int4* tab = reinterpret_cast<int4*>(smem_raw + l.off_tab);
-  int4* ex = reinterpret_cast<int4*>(smem_raw + l.off_ex);
-  S* px = reinterpret_cast<S*>(smem_raw + l.off_px);
-  S* monoT = reinterpret_cast<S*>(smem_raw + l.off_mono);
-  S* Lb = reinterpret_cast<S*>(smem_raw + l.off_b);
-  const int n = d.n, KP = l.KP;
-  const int nm = kPot ? d.n : d.nm, p = kPot ? d.p + 1 : d.p;  // monomial count and axis powers held
-  constexpr int TC = kL2PTargets;
-  const int tid = threadIdx.x, T = blockDim.x;
-  const int KT = KP / kRK;
-  const int tt = tid / KT, kt = tid % KT;
-  const int leaf = blockIdx.x;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  const int2 range = d.leaf_tgt[leaf];
-  if (range.x == range.y) return;
-  const int64_t node = level_offset(d.L) + leaf;
-  for (int i = tid; i < n; i += T) tab[i] = d.p2m_tab[i];
-  for (int i = tid; i < nm; i += T) ex[i] = d.p2m_tab[n + i];
-  stage_box<S>(Lb, static_cast<const S*>(d.Lc) + node * int64_t(n) * K + kc0, n, K, KCn, KP);
-  const auto* rel = static_cast<const typename Vec4<S>::type*>(d.tgt_rel);
-  const S* Hn = static_cast<const S*>(d.Hn);
-  const int k0 = kt * kRK, tl = tt * kL2PRT;
-  for (int t0 = range.x; t0 < range.y; t0 += TC) {
-    const int cnt = min(TC, range.y - t0);
-    __syncthreads();
-    if (tid < 3 * TC) {
-      const int t = tid / 3, a = tid % 3;
-      S x = S(0);
-      if (t < cnt) {
-        const auto r = rel[t0 + t];
-        x = a == 0 ? r.x : (a == 1 ? r.y : r.z);
-      }
-      S* row = px + (t * 3 + a) * p;
-      for (int i = 0; i < p; ++i) row[i] = axis_power<S>(x, i);
-    }
-    __syncthreads();
-    for (int w = tid; w < nm * TC; w += T) {
-      const int g = w / TC, t = w - g * TC;
-      const int4 e = ex[g];
-      const S* pt = px + t * 3 * p;
-      monoT[w] = pt[e.x] * pt[p + e.y] * pt[2 * p + e.z];
-    }
-    __syncthreads();
-    if (tl >= cnt) continue;
-    constexpr int C = kPot ? 4 : 3;
-    S acc[C][kL2PRT][kRK];
-#pragma unroll
-    for (int c = 0; c < C; ++c)
-#pragma unroll
-      for (int i = 0; i < kL2PRT; ++i)
-#pragma unroll
-        for (int j = 0; j < kRK; ++j) acc[c][i][j] = S(0);
-    for (int b = 0; b < n; ++b) {
-      const int4 t4 = tab[b];
-      S lv[kRK];
-      load_vec<S, kRK>(Lb + b * KP + k0, lv);
-      const int idx[4] = {t4.x, t4.y, t4.z, b};
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        if (idx[c] < 0) continue;
-        const S* mrow = monoT + idx[c] * TC + tl;
-        S mv[kL2PRT];
-#pragma unroll
-        for (int i = 0; i < kL2PRT; ++i) mv[i] = mrow[i];
-#pragma unroll
-        for (int i = 0; i < kL2PRT; ++i)
-#pragma unroll
-          for (int j = 0; j < kRK; ++j) acc[c][i][j] = fma(mv[i], lv[j], acc[c][i][j]);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kL2PRT; ++i) {
-      if (tl + i >= cnt) break;
-      const int ts = t0 + tl + i;
-      const int user = d.tgt_perm[ts];
-      const S* hn = Hn + int64_t(ts) * 3 * K;
-#pragma unroll
-      for (int j = 0; j < kRK; ++j) {
-        if (k0 + j >= KCn) break;
-        const int k = kc0 + k0 + j;
-        if (!kPot || out != nullptr) {
-          S* o = out + (int64_t(k) * d.nt + user) * 3;
-          o[0] = hn[k] - acc[0][i][j];
-          o[1] = hn[K + k] - acc[1][i][j];
-          o[2] = hn[2 * K + k] - acc[2][i][j];
-        }
-        if constexpr (kPot) {
-          const S pn = static_cast<const S*>(d.Pn)[int64_t(ts) * K + k];
-          pot[int64_t(k) * d.nt + user] = S(d.potential_scale) * (pn + acc[C - 1][i][j]);
-        }
-      }
-    }
-  }
-}
-
-// Harmonic-subspace compression of the multipoles of one box at `level`:
-//   Mc[r][k] = sum_alpha cmp[level][alpha][r] M[alpha][k],  r < NPc,
-// written as plain scalars (Mc) or, for the MFMA M2L, split into bf16 hi/lo
-// halves in its operand layout mt[node][ks][k][16] (r = 16 ks + position;
-// rows nc..NPc-1 are zero because the operator's padding columns are).
-template <class S, bool kSplit>
-__global__ void __launch_bounds__(1024) compress_kernel(const DevicePlan d, int level, int K, int KC, int KP) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  S* B = reinterpret_cast<S*>(smem_raw);  // [n][KP]
-  const int n = d.n, NPc = round_up(d.nc, 16), KT = KP / kRK;
-  const int tid = threadIdx.x;
-  const int at = tid / KT, kt = tid % KT;
-  const bool active = at < NPc / kRA;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  const int64_t node = level_offset(level) + blockIdx.x;
-  stage_box<S>(B, static_cast<const S*>(d.M) + node * int64_t(n) * K + kc0, n, K, KCn, KP);
-  __syncthreads();
-  if (!active) return;
-  S acc[kRA][kRK];
-#pragma unroll
-  for (int i = 0; i < kRA; ++i)
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) acc[i][j] = S(0);
-  const S* A = static_cast<const S*>(d.cmp_op) + size_t(level) * n * NPc + at * kRA;
-  tile_gemm<S>(A, NPc, B + kt * kRK, KP, n, acc);
-  if constexpr (kSplit) {
-    // FP32 only: 8 consecutive rows of one 16-deep step -> one 16-byte store
-    // per state and half.
-    const int r0 = at * kRA, ks = r0 / 16, pos = r0 % 16, KS = NPc / 16;
-    uint4* hi = static_cast<uint4*>(d.mt_hi);
-    uint4* lo = static_cast<uint4*>(d.mt_lo);
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) {
-      const int k = kt * kRK + j;
-      if (k >= KCn) break;
-      uint16_t h[kRA], l[kRA];
-#pragma unroll
-      for (int i = 0; i < kRA; ++i) {
-        const float x = float(acc[i][j]);
-        h[i] = bf16_round(x);
-        l[i] = bf16_round(x - __builtin_bit_cast(float, uint32_t(h[i]) << 16));
-      }
-      const int64_t at16 = (((node * KS + ks) * K + kc0 + k) * 16 + pos) / 8;  // uint4 index
-      hi[at16] = uint4{uint32_t(h[0]) | (uint32_t(h[1]) << 16), uint32_t(h[2]) | (uint32_t(h[3]) << 16),
-                       uint32_t(h[4]) | (uint32_t(h[5]) << 16), uint32_t(h[6]) | (uint32_t(h[7]) << 16)};
-      lo[at16] = uint4{uint32_t(l[0]) | (uint32_t(l[1]) << 16), uint32_t(l[2]) | (uint32_t(l[3]) << 16),
-                       uint32_t(l[4]) | (uint32_t(l[5]) << 16), uint32_t(l[6]) | (uint32_t(l[7]) << 16)};
-    }
-  } else {
-    store_tile<S, false>(static_cast<S*>(d.Mc) + node * int64_t(d.nc) * K + kc0, at * kRA, d.nc, kt * kRK, KCn, K,
-                         acc);
-  }
-}
-
-// Expansion of the compressed locals of one box at `level`:
-//   Lc[beta][k] = sum_r exp[level][r][beta] Lcc[r][k]   (overwrites Lc).
-template <class S>
-__global__ void __launch_bounds__(1024) expand_kernel(const DevicePlan d, int level, int K, int KC, int KP) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  S* B = reinterpret_cast<S*>(smem_raw);  // [nc][KP]
-  const int n = d.n, nc = d.nc, NP = round_up(n, kRA), KT = KP / kRK;
-  const int tid = threadIdx.x;
-  const int at = tid / KT, kt = tid % KT;
-  const bool active = at < NP / kRA;
-  const int kc0 = blockIdx.y * KC, KCn = min(KC, K - kc0);
-  const int64_t node = level_offset(level) + blockIdx.x;
-  stage_box<S>(B, static_cast<const S*>(d.Lcc) + node * int64_t(nc) * K + kc0, nc, K, KCn, KP);
-  __syncthreads();
-  if (!active) return;
-  S acc[kRA][kRK];
-#pragma unroll
-  for (int i = 0; i < kRA; ++i)
-#pragma unroll
-    for (int j = 0; j < kRK; ++j) acc[i][j] = S(0);
-  const S* A = static_cast<const S*>(d.exp_op) + size_t(level) * nc * NP + at * kRA;
-  tile_gemm<S>(A, NP, B + kt * kRK, KP, nc, acc);
-  store_tile<S, false>(static_cast<S*>(d.Lc) + node * int64_t(n) * K + kc0, at * kRA, n, kt * kRK, KCn, K, acc);
-}
-
 template <class S>
 __global__ void zero_kernel(S* p, size_t count) {
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += size_t(gridDim.x) * blockDim.x)
     p[i] = S(0);
-}
-
-// Threads for a tile grid of (row tiles) x (state tiles), whole waves.
-inline unsigned tile_threads(int row_tiles, int KP) {
-  const int t = row_tiles * (KP / kRK);
-  const int threads = std::max(64, round_up(t, 64));
-  if (threads > 1024) throw invalid_argument("expansion order and batch too large for one workgroup per box");
-  return unsigned(threads);
-}
-
-// Far-field gradient of the field from the leaf local (no counterpart in
-// the reference): the derivative of its L2P polynomial,
-//   G_cj(t) = -sum_b L[b] d_t^(b - e_c - e_j) / (b - e_c - e_j)!,
-// entries xx xy xz yy yz zz (grad_tab[b][e]: index of b - e_c - e_j, or -1),
-// plus the near-field gradient Gn, times the frame factor, unsorted to
-// out[k][user target][6].  One workgroup per target leaf, targets in
-// chunks of 32; thread per (target, state).
-template <class S>
-__global__ void __launch_bounds__(256) l2p_grad_kernel(const DevicePlan d, S* __restrict__ out, int K, int nm2,
-                                                       S scale) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int n = d.n, PW = max(d.p - 1, 1);
-  int* gt = reinterpret_cast<int*>(smem_raw);                      // [n][6]
-  S* pw = reinterpret_cast<S*>(smem_raw + align16(size_t(n) * 6 * sizeof(int)));  // [32][3][PW]
-  S* mono = pw + 32 * 3 * PW;                                       // [32][nm2]
-  const int leaf = blockIdx.x, tid = threadIdx.x;
-  const int2 range = d.leaf_tgt[leaf];
-  if (range.x == range.y) return;
-  const int64_t node = level_offset(d.L) + leaf;
-  for (int i = tid; i < n * 6; i += 256) gt[i] = d.grad_tab[i];
-  const auto* rel = static_cast<const typename Vec4<S>::type*>(d.tgt_rel);
-  const S* Lb = static_cast<const S*>(d.Lc) + node * int64_t(n) * K;
-  const S* Gn = static_cast<const S*>(d.Gn);
-  for (int t0 = range.x; t0 < range.y; t0 += 32) {
-    const int cnt = min(32, range.y - t0);
-    __syncthreads();
-    if (tid < 96) {
-      const int t = tid / 3, a = tid % 3;
-      S x = S(0);
-      if (t < cnt) {
-        const auto r = rel[t0 + t];
-        x = a == 0 ? r.x : (a == 1 ? r.y : r.z);
-      }
-      for (int i = 0; i < PW; ++i) pw[tid * PW + i] = axis_power<S>(x, i);
-    }
-    __syncthreads();
-    for (int w = tid; w < 32 * nm2; w += 256) {
-      const int t = w / nm2, g = w - t * nm2;
-      const int4 e = d.p2m_tab[n + g];
-      const S* pt = pw + t * 3 * PW;
-      mono[w] = pt[e.x] * pt[PW + e.y] * pt[2 * PW + e.z];
-    }
-    __syncthreads();
-    for (int item = tid; item < cnt * K; item += 256) {
-      const int t = item / K, k = item - t * K;
-      S G[6] = {S(0), S(0), S(0), S(0), S(0), S(0)};
-      const S* mt = mono + t * nm2;
-      for (int b = 0; b < n; ++b) {
-        const S lv = Lb[int64_t(b) * K + k];
-#pragma unroll
-        for (int e = 0; e < 6; ++e) {
-          const int i = gt[b * 6 + e];
-          if (i >= 0) G[e] -= lv * mt[i];
-        }
-      }
-      const int ts = t0 + t;
-      const int user = d.tgt_perm[ts];
-      S* o = out + (int64_t(k) * d.nt + user) * 6;
-#pragma unroll
-      for (int e = 0; e < 6; ++e) o[e] = scale * (Gn[(int64_t(ts) * 6 + e) * K + k] + G[e]);
-    }
-  }
 }
 
 // P2M on the matrix cores (FP32 plans, K a multiple of 32).  With
@@ -1023,15 +455,6 @@ void launch_gather(const DevicePlan& d, const S* user_moments, S scale, int K, h
   HIPFMM_CHECK(hipGetLastError());
 }
 
-// Widest state chunk (a multiple of 4, or K) whose LDS layout fits 64 KiB.
-template <class F>
-int state_chunk(int K, F bytes_for) {
-  int kc = K;
-  while (kc > kRK && bytes_for(kc) > 65536) kc = round_up(kc / 2, kRK);
-  if (bytes_for(kc) > 65536) throw invalid_argument("expansion order too large for the box kernels' LDS");
-  return kc;
-}
-
 template <class S>
 void launch_p2m(const DevicePlan& d, int K, hipStream_t s) {
   if (d.leaves == 0) return;
@@ -1052,12 +475,7 @@ void launch_p2m(const DevicePlan& d, int K, hipStream_t s) {
       return;
     }
   }
-  const int kc = state_chunk(K, [&](int c) { return p2m_layout<S>(d, c).bytes; });
-  const MonoLayout l = p2m_layout<S>(d, kc);
-  const unsigned threads = std::max(tile_threads(l.NP / kRA, l.KP), unsigned(round_up(3 * l.JC, 64)));
-  const dim3 grid(unsigned(d.leaves), unsigned((K + kc - 1) / kc));
-  p2m_kernel<S><<<grid, threads, l.bytes, s>>>(d, K, kc, l);
-  HIPFMM_CHECK(hipGetLastError());
+  launch_p2m_columns<S>(d, K, s);
 }
 
 // Far-field gradient on the matrix cores (FP32 plans, K a multiple of 32),
@@ -1159,7 +577,7 @@ __global__ void __launch_bounds__(256) l2p_grad_mfma_kernel(const DevicePlan d, 
 template <class S>
 void launch_l2p_grad_unsort(const DevicePlan& d, S* gradients, int K, hipStream_t s) {
   if (d.leaves == 0 || d.nt == 0) return;
-  if (d.Gn == nullptr || d.grad_tab == nullptr) throw invalid_argument("field-gradient buffers are not allocated");
+  if (d.Gn == nullptr) throw invalid_argument("field-gradient buffers are not allocated");
   const int nm2 = d.p >= 2 ? coefficient_count(d.p - 2) : 0;
   if constexpr (sizeof(S) == 4) {
     const size_t lds_m = size_t(4) * 48 * std::max(d.p - 1, 1) * sizeof(float) + size_t(nm2) * sizeof(int4) +
@@ -1171,11 +589,7 @@ void launch_l2p_grad_unsort(const DevicePlan& d, S* gradients, int K, hipStream_
       return;
     }
   }
-  const size_t lds = align16(size_t(d.n) * 6 * sizeof(int)) + (size_t(32) * 3 * std::max(d.p - 1, 1) + size_t(32) * std::max(nm2, 1)) * sizeof(S);
-  if (lds > 65536) throw invalid_argument("expansion order too large for the field-gradient kernel's LDS");
-  const S scale = S(1.0 / d.potential_scale);
-  l2p_grad_kernel<S><<<unsigned(d.leaves), 256, lds, s>>>(d, gradients, K, nm2, scale);
-  HIPFMM_CHECK(hipGetLastError());
+  launch_l2p_grad_columns<S>(d, gradients, K, s);
 }
 
 // Box GEMMs on the matrix cores (FP32 plans, K a multiple of 32): M2M, L2L,
@@ -1488,7 +902,7 @@ __global__ void __launch_bounds__(256)
 m2m_mfma_kernel(const DevicePlan d, int level, int K) {
   extern __shared__ __align__(16) float box_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
-  const int n = d.n, NP = round_up(n, kRA), D4 = (n + 3) / 4 * 4, RT = (n + 15) / 16;
+  const int n = d.n, NP = round_up(n, 8), D4 = (n + 3) / 4 * 4, RT = (n + 15) / 16;
   const int kc0 = int(blockIdx.y) * 32;
   const int64_t parent = blockIdx.x, cnode0 = level_offset(level + 1) + parent * 8;
   const float* M = static_cast<const float*>(d.M) + kc0;
@@ -1528,7 +942,7 @@ __global__ void __launch_bounds__(256)
 l2l_mfma_kernel(const DevicePlan d, int child_level, int K) {
   extern __shared__ __align__(16) float box_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
-  const int n = d.n, NP = round_up(n, kRA), D4 = (n + 3) / 4 * 4, RT = (n + 15) / 16;
+  const int n = d.n, NP = round_up(n, 8), D4 = (n + 3) / 4 * 4, RT = (n + 15) / 16;
   const int kc0 = int(blockIdx.y) * 32;
   const int64_t parent = blockIdx.x;
   float* Lc = static_cast<float*>(d.Lc) + kc0;
@@ -1600,12 +1014,7 @@ void launch_m2m(const DevicePlan& d, int parent_level, int K, hipStream_t s) {
       return;
     }
   }
-  const int NP = round_up(d.n, kRA);
-  const int kc = state_chunk(K, [&](int c) { return size_t(d.n) * round_up(c, kRK) * sizeof(S); });
-  const int KP = round_up(kc, kRK);
-  const dim3 grid(unsigned(int64_t(1) << (3 * parent_level)), unsigned((K + kc - 1) / kc));
-  m2m_kernel<S><<<grid, tile_threads(NP / kRA, KP), size_t(d.n) * KP * sizeof(S), s>>>(d, parent_level, K, kc, KP);
-  HIPFMM_CHECK(hipGetLastError());
+  launch_m2m_columns<S>(d, parent_level, K, s);
 }
 
 template <class S>
@@ -1628,12 +1037,7 @@ void launch_l2l(const DevicePlan& d, int child_level, int K, hipStream_t s) {
       return;
     }
   }
-  const int NP = round_up(d.n, kRA);
-  const int kc = state_chunk(K, [&](int c) { return size_t(d.n) * round_up(c, kRK) * sizeof(S); });
-  const int KP = round_up(kc, kRK);
-  const dim3 grid(unsigned(int64_t(1) << (3 * (child_level - 1))), unsigned((K + kc - 1) / kc));
-  l2l_kernel<S><<<grid, tile_threads(NP / kRA, KP), size_t(d.n) * KP * sizeof(S), s>>>(d, child_level, K, kc, KP);
-  HIPFMM_CHECK(hipGetLastError());
+  launch_l2l_columns<S>(d, child_level, K, s);
 }
 
 template <class S>
@@ -1675,34 +1079,15 @@ void launch_l2p_unsort(const DevicePlan& d, S* fields, S* potentials, int K, hip
       return;
     }
   }
-  const int kc = state_chunk(K, [&](int c) { return l2p_layout<S>(d, c, pot).bytes; });
-  const MonoLayout l = l2p_layout<S>(d, kc, pot);
-  const unsigned threads = std::max(tile_threads(l.TCP / kL2PRT, l.KP), unsigned(round_up(3 * l.TCP, 64)));
-  const dim3 grid(unsigned(d.leaves), unsigned((K + kc - 1) / kc));
-  if (pot)
-    l2p_kernel<S, true><<<grid, threads, l.bytes, s>>>(d, fields, potentials, K, kc, l);
-  else
-    l2p_kernel<S, false><<<grid, threads, l.bytes, s>>>(d, fields, nullptr, K, kc, l);
-  HIPFMM_CHECK(hipGetLastError());
+  launch_l2p_columns<S>(d, fields, potentials, K, s);
 }
 
 template <class S>
-void launch_m2l_compress(const DevicePlan& d, int K, bool split, int first_level, hipStream_t s) {
-  const int NPc = round_up(d.nc, 16);
-  const int kc = state_chunk(K, [&](int c) { return size_t(d.n) * round_up(c, kRK) * sizeof(S); });
-  const int KP = round_up(kc, kRK);
+void launch_m2l_compress(const DevicePlan& d, int K, int first_level, hipStream_t s) {
   for (int level = std::max(first_level, 2); level <= d.L; ++level) {
-    const dim3 grid(unsigned(int64_t(1) << (3 * level)), unsigned((K + kc - 1) / kc));
-    const unsigned threads = tile_threads(NPc / kRA, KP);
-    const size_t lds = size_t(d.n) * KP * sizeof(S);
     if constexpr (sizeof(S) == 4) {
-      if (split) {
-        compress_kernel<S, true><<<grid, threads, lds, s>>>(d, level, K, kc, KP);
-        HIPFMM_CHECK(hipGetLastError());
-        continue;
-      }
       if (const int rtw = box_mfma_rtw(d.nc, d.n, K)) {
-        const dim3 g2(grid.x, unsigned(K / 32));
+        const dim3 g2(unsigned(int64_t(1) << (3 * level)), unsigned(K / 32));
         const int64_t node0 = level_offset(level);
         const float* in = static_cast<const float*>(d.M) + node0 * d.n * K;
         float* out = static_cast<float*>(d.Mc) + node0 * d.nc * K;
@@ -1715,6 +1100,7 @@ void launch_m2l_compress(const DevicePlan& d, int K, bool split, int first_level
 #undef HIPFMM_CMP
         } else {
           const size_t l2 = size_t((d.n + 3) / 4 * 4) * kBoxLd * sizeof(float);
+          const int NPc = round_up(d.nc, 16);
           const float* A = static_cast<const float*>(d.cmp_op) + size_t(level) * d.n * NPc;
 #define HIPFMM_CMP(R) box_mfma_kernel<R, false><<<g2, 256, l2, s>>>(A, NPc, d.nc, d.n, in, int64_t(d.n) * K, out, \
                                                                      int64_t(d.nc) * K, K)
@@ -1725,22 +1111,16 @@ void launch_m2l_compress(const DevicePlan& d, int K, bool split, int first_level
         continue;
       }
     }
-    if (split) throw invalid_argument("the split compressed layout is an FP32 operand");
-    compress_kernel<S, false><<<grid, threads, lds, s>>>(d, level, K, kc, KP);
-    HIPFMM_CHECK(hipGetLastError());
+    launch_compress_columns<S>(d, level, K, s);
   }
 }
 
 template <class S>
 void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t s) {
-  const int NP = round_up(d.n, kRA);
-  const int kc = state_chunk(K, [&](int c) { return size_t(d.nc) * round_up(c, kRK) * sizeof(S); });
-  const int KP = round_up(kc, kRK);
   for (int level = std::max(first_level, 2); level <= d.L; ++level) {
-    const dim3 grid(unsigned(int64_t(1) << (3 * level)), unsigned((K + kc - 1) / kc));
     if constexpr (sizeof(S) == 4) {
       if (const int rtw = box_mfma_rtw(d.n, d.nc, K)) {
-        const dim3 g2(grid.x, unsigned(K / 32));
+        const dim3 g2(unsigned(int64_t(1) << (3 * level)), unsigned(K / 32));
         const int64_t node0 = level_offset(level);
         const float* in = static_cast<const float*>(d.Lcc) + node0 * d.nc * K;
         float* out = static_cast<float*>(d.Lc) + node0 * d.n * K;
@@ -1753,6 +1133,7 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
 #undef HIPFMM_EXP
         } else {
           const size_t l2 = size_t((d.nc + 3) / 4 * 4) * kBoxLd * sizeof(float);
+          const int NP = round_up(d.n, 8);
           const float* A = static_cast<const float*>(d.exp_op) + size_t(level) * d.nc * NP;
 #define HIPFMM_EXP(R) box_mfma_kernel<R, false><<<g2, 256, l2, s>>>(A, NP, d.n, d.nc, in, int64_t(d.nc) * K, out, \
                                                                      int64_t(d.n) * K, K)
@@ -1763,8 +1144,7 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
         continue;
       }
     }
-    expand_kernel<S><<<grid, tile_threads(NP / kRA, KP), size_t(d.nc) * KP * sizeof(S), s>>>(d, level, K, kc, KP);
-    HIPFMM_CHECK(hipGetLastError());
+    launch_expand_columns<S>(d, level, K, s);
   }
 }
 
@@ -1783,7 +1163,7 @@ void launch_zero(S* ptr, size_t count, hipStream_t s) {
   template void launch_l2l<S>(const DevicePlan&, int, int, hipStream_t);           \
   template void launch_l2p_unsort<S>(const DevicePlan&, S*, S*, int, hipStream_t);     \
   template void launch_l2p_grad_unsort<S>(const DevicePlan&, S*, int, hipStream_t);    \
-  template void launch_m2l_compress<S>(const DevicePlan&, int, bool, int, hipStream_t); \
+  template void launch_m2l_compress<S>(const DevicePlan&, int, int, hipStream_t); \
   template void launch_m2l_expand<S>(const DevicePlan&, int, int, hipStream_t);    \
   template void launch_zero<S>(S*, size_t, hipStream_t);
 HIPFMM_INSTANTIATE(float)

@@ -438,28 +438,6 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   d.self = upload(P, self.data(), self.size());
   const auto tab = basis_tables(p);
   d.p2m_tab = upload(P, tab.data(), tab.size());
-  // Field-gradient table: b -> b - e_c - e_j for (c, j) = xx xy xz yy yz zz.
-  {
-    std::vector<int> gt(size_t(n) * 6, -1);
-    const int cj[6][2] = {{0, 0}, {0, 1}, {0, 2}, {1, 1}, {1, 2}, {2, 2}};
-    for (int b = 0; b < n; ++b) {
-      const int4 e = tab[n + b];
-      for (int q = 0; q < 6; ++q) {
-        int x[3] = {e.x, e.y, e.z};
-        --x[cj[q][0]];
-        --x[cj[q][1]];
-        if (x[0] < 0 || x[1] < 0 || x[2] < 0) continue;
-        for (int g = 0; g < n; ++g) {
-          const int4 f = tab[n + g];
-          if (f.x == x[0] && f.y == x[1] && f.z == x[2]) {
-            gt[size_t(b) * 6 + q] = g;
-            break;
-          }
-        }
-      }
-    }
-    d.grad_tab = upload(P, gt.data(), gt.size());
-  }
   // Raising table of the matrix-core L2P: g (degree < p) -> g + e_c.
   {
     std::vector<int4> up(std::max(d.nm, 1), int4{0, 0, 0, 0});
@@ -1090,7 +1068,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     dc.l2l_dense = d.l2l_dense_c;
     dc.m2m_x3 = d.m2m_x3_c;
     dc.l2l_x3 = d.l2l_x3_c;
-    hipfmm::launch_m2l_compress<S>(d, K, false, d.L, s);
+    hipfmm::launch_m2l_compress<S>(d, K, d.L, s);
     for (int level = d.L - 1; level >= 2; --level) hipfmm::launch_m2m<S>(dc, level, K, s);
   } else {
     for (int level = d.L - 1; level >= 2; --level) hipfmm::launch_m2m<S>(d, level, K, s);
@@ -1110,18 +1088,11 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     dm.Lc = d.Lcc;
     dm.ms = d.unit_scale;
     dm.ls = d.unit_scale;
-    // bf16 operands come straight out of the compression; FP16 operands need
-    // the level maxima of the compressed multipoles first.
-    const bool fp16 = mfma && P->m2l_mode == HIPFMM_M2L_MFMA_FP16X3;
-    if (harmonic) {
-      if (fp16)
-        hipfmm::launch_m2l_fp16_split(d, K, s);
-      else if (mfma)
-        hipfmm::launch_m2l_bf16_split(d, K, s);
-    } else {
-      hipfmm::launch_m2l_compress<S>(d, K, mfma && !fp16, 2, s);
-      if (fp16) hipfmm::launch_m2l_fp16_split(d, K, s);
-    }
+    if (!harmonic) hipfmm::launch_m2l_compress<S>(d, K, 2, s);
+    if (mfma && P->m2l_mode == HIPFMM_M2L_MFMA_FP16X3)
+      hipfmm::launch_m2l_fp16_split(d, K, s);
+    else if (mfma)
+      hipfmm::launch_m2l_bf16_split(d, K, s);
   } else if (mfma) {
     hipfmm::launch_m2l_split(d, K, P->m2l_mode, s);
   }
