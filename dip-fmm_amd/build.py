@@ -29,7 +29,7 @@ HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-Wall", "-Wno-unused-result",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-HIP_SOURCES = ["plan.hip", "far.hip", "columns.hip", "near.hip", "near_lanes.hip", "m2l_valu.hip", "m2l_mfma.hip", "m2l_basis.hip", "tree.hip", "lists.hip"]
+HIP_SOURCES = ["plan.hip", "far.hip", "columns.hip", "near.hip", "near_lanes.hip", "m2l_valu.hip", "m2l_full.hip", "m2l_mfma.hip", "m2l_basis.hip", "tree.hip", "lists.hip"]
 HOST_SOURCES = ["host/operators.cpp", "host/operator_tables.cpp", "host/uniform_fmm.cpp", "python/bindings.cpp"]
 
 

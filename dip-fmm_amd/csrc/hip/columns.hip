@@ -57,10 +57,20 @@ struct Mma<double> {
   __device__ __forceinline__ static int row(int q, int r) { return 4 * r + q; }
 };
 
+// How a box's coefficients lie: rows row values apart, states state apart.
+struct Strides {
+  uint32_t row, state;
+};
+// [coefficient][K], or (state_major) [K][count].
+inline Strides strides(bool state_major, int K, int count) {
+  return state_major ? Strides{1u, uint32_t(count)} : Strides{uint32_t(K), 1u};
+}
+
 // out[row][col] (+)= sum over segments g and depth d of A_g[d][row] in_g[d][col]
 // with the columns col = (box, state): in_g[d][col] = in[box * in_box +
-// g * in_seg + d * K + state], out likewise, A_g = A + g * a_seg.  blockIdx.z
-// offsets A and out by a_z and out_z (the 8 children of the L2L).
+// g * in_seg + d * in_at.row + state * in_at.state], out likewise,
+// A_g = A + g * a_seg.  blockIdx.z offsets A and out by a_z and out_z (the 8
+// children of the L2L).
 template <class S>
 struct Product {
   const S* A;
@@ -68,8 +78,10 @@ struct Product {
   int lda, R, D, segments;
   const S* in;
   int64_t in_box, in_seg;
+  Strides in_at;
   S* out;
   int64_t out_box, out_z;
+  Strides out_at;
   int K;
   int64_t cols;
   int row_waves;  // waves side by side over the rows; blockDim / 64 / row_waves groups share the segments
@@ -105,10 +117,10 @@ __global__ void __launch_bounds__(1024) product_kernel(const Product<S> p) {
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     const uint32_t x = rem + min(uint32_t(16 * c + i), left - 1), box = x / K, k = x - box * K;
-    in_at[c] = (box * uint32_t(p.in_box) + k) * uint32_t(sizeof(S));
-    out_at[c] = box * uint32_t(p.out_box) + k;
+    in_at[c] = (box * uint32_t(p.in_box) + k * p.in_at.state) * uint32_t(sizeof(S));
+    out_at[c] = box * uint32_t(p.out_box) + k * p.out_at.state;
   }
-  const uint32_t a_step = uint32_t(p.lda) * uint32_t(sizeof(S)), b_step = K * uint32_t(sizeof(S));  // per depth value
+  const uint32_t a_step = uint32_t(p.lda) * uint32_t(sizeof(S)), b_step = p.in_at.row * uint32_t(sizeof(S));  // per depth value
   uint32_t row[RTW];
 #pragma unroll
   for (int t = 0; t < RTW; ++t)
@@ -133,7 +145,7 @@ __global__ void __launch_bounds__(1024) product_kernel(const Product<S> p) {
           for (int t = 0; t < RTW; ++t) a[u][t] = load_at(A + int64_t(d0 + 4 * u) * p.lda, uint32_t(q) * a_step + row[t]);
 #pragma unroll
           for (int c = 0; c < CT; ++c)
-            b[u][c] = load_at(in + seg + int64_t(d0 + 4 * u) * p.K, uint32_t(q) * b_step + in_at[c]);
+            b[u][c] = load_at(in + seg + int64_t(d0 + 4 * u) * p.in_at.row, uint32_t(q) * b_step + in_at[c]);
         }
       } else {  // the last batch: depth values past D read the last one, times zero
 #pragma unroll
@@ -189,7 +201,7 @@ __global__ void __launch_bounds__(1024) product_kernel(const Product<S> p) {
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
         if (uint32_t(16 * c + i) >= left) continue;
-        S* o = out + uint32_t(orow) * K + out_at[c];
+        S* o = out + uint32_t(orow) * p.out_at.row + out_at[c];
         *o = p.add ? *o + acc[t][c][r] : acc[t][c][r];
       }
     }
@@ -567,6 +579,7 @@ void launch_m2m_columns(const DevicePlan& d, int parent_level, int K, hipStream_
   p.in_box = 8 * box, p.in_seg = box;
   p.out = M + level_offset(parent_level) * box;
   p.out_box = box;
+  p.in_at = p.out_at = strides(d.state_major, K, n);
   p.K = K, p.cols = parents * K;
   launch_product<S>(p, 1, s);
 }
@@ -584,6 +597,7 @@ void launch_l2l_columns(const DevicePlan& d, int child_level, int K, hipStream_t
   p.in_box = box;
   p.out = L + level_offset(child_level) * box;
   p.out_box = 8 * box, p.out_z = box;
+  p.in_at = p.out_at = strides(d.state_major, K, n);
   p.K = K, p.cols = parents * K;
   p.add = true;
   launch_product<S>(p, 8, s);
@@ -599,6 +613,7 @@ void launch_compress_columns(const DevicePlan& d, int level, int K, hipStream_t 
   p.in_box = int64_t(d.n) * K, p.out_box = int64_t(d.nc) * K;
   p.in = static_cast<const S*>(d.M) + node0 * p.in_box;
   p.out = static_cast<S*>(d.Mc) + node0 * p.out_box;
+  p.in_at = strides(false, K, d.n), p.out_at = strides(d.compressed_state_major, K, d.nc);
   p.K = K, p.cols = boxes * K;
   launch_product<S>(p, 1, s);
 }
@@ -613,6 +628,7 @@ void launch_expand_columns(const DevicePlan& d, int level, int K, hipStream_t s)
   p.in_box = int64_t(d.nc) * K, p.out_box = int64_t(d.n) * K;
   p.in = static_cast<const S*>(d.Lcc) + node0 * p.in_box;
   p.out = static_cast<S*>(d.Lc) + node0 * p.out_box;
+  p.in_at = strides(d.compressed_state_major, K, d.nc), p.out_at = strides(false, K, d.n);
   p.K = K, p.cols = boxes * K;
   launch_product<S>(p, 1, s);
 }

@@ -161,7 +161,13 @@ struct DevicePlan {
   int4* p2m_tab = nullptr;  // per alpha: index(alpha-e_c) or -1 for c=0..2, w = sign (+1/-1)
   int4* l2p_up = nullptr;   // per g of degree < p: index(g + e_c) for c = 0..2
   // operators
-  void* m2l_T = nullptr;     // FP32/FP64 class matrices, column-major [class][alpha][beta]
+  void* m2l_T = nullptr;     // FP32/FP64 class matrices, column-major [class][alpha][beta] (plans without harmonic form)
+  // Harmonic form: the class matrices C_o in fragment order (m2l_full.hip), the
+  // 189 offsets of each parity as dilated Morton steps (x, y, z, class), and a
+  // box of zeros at the largest batch (the source of columns without one).
+  void* m2l_fragments = nullptr;
+  int4* m2l_steps = nullptr;
+  void* m2l_zero_box = nullptr;
   int* m2l_slot = nullptr;   // 343 slot -> class index or -1
   int4* parity_offsets = nullptr;  // [8 parities][189] (ox, oy, oz, class) list-2 offsets
   // Order of the target parents over the tiles of the matrix-core M2L (one
@@ -205,7 +211,6 @@ struct DevicePlan {
   int nc = 0;
   void* cmp_op = nullptr;  // [(level)][alpha n][NPc] = P[r][alpha] * ms[level][alpha], NPc = nc rounded up to 16
   void* exp_op = nullptr;  // [(level)][r nc][NP]    = ls[level][beta] * Q[beta][r], NP = n rounded up to 8
-  void* unit_scale = nullptr;  // (L+1) x nc ones: the M2L's own scalings in compressed form
   // The box-product operators as three-piece bf16 A fragments of
   // v_mfma_f32_16x16x32_bf16 (FP32 harmonic plans; null otherwise): per
   // operator [piece][32-deep step][row, padded to 16][32], box_x3_elems
@@ -218,11 +223,13 @@ struct DevicePlan {
   void* l2l_x3 = nullptr;
   void* m2m_x3_c = nullptr;
   void* l2l_x3_c = nullptr;
-  // Partial sums of the vector-ALU M2L when its tiles' offsets are split in
-  // parts: [part][node][nc][K], room for parts * K <= m2l_part_capacity.
-  void* m2l_part = nullptr;
-  int m2l_part_capacity = 0;
-  void* Mc = nullptr;      // compressed multipoles [node][nc][K] (vector-ALU M2L input)
+  // Where no kernel of far.hip's K = 32 n forms runs, a node's compressed
+  // coefficients lie [K][nc] instead of [nc][K] (compressed_state_major): the
+  // depth of the M2L's columns is contiguous at every K.  state_major says the
+  // same of M and Lc as this view sees them (the compressed view).
+  bool compressed_state_major = false;
+  bool state_major = false;
+  void* Mc = nullptr;      // compressed multipoles [node][nc][K]
   void* Lcc = nullptr;     // compressed locals [node][nc][K] (M2L output)
   // MFMA operands
   void* mt_hi = nullptr;  // bf16/fp16 [node][K][apad]
@@ -265,14 +272,21 @@ template <class S>
 void launch_m2m(const DevicePlan& d, int parent_level, int K, hipStream_t s);
 template <class S>
 void launch_l2l(const DevicePlan& d, int child_level, int K, hipStream_t s);
+// M2L of all levels 2..L in the type's own precision: on the matrix cores for
+// the harmonic form (d seen through the compressed view: n = nc, M = Mc,
+// Lc = Lcc), on the vector ALUs otherwise.
 template <class S>
-void launch_m2l_valu(const DevicePlan& d, int K, hipStream_t s);  // all levels 2..L
-// Offset parts per tile of the FP32 vector-ALU M2L at K states (1: no split;
-// otherwise the launch needs parts * K <= m2l_part_capacity).
-constexpr int kValuMaxParts = 4;
-int m2l_valu_parts(const DevicePlan& d, int K);
-// CUs of a device (asked of the runtime once per device).
-int device_cu_count(int device);
+void launch_m2l_full(const DevicePlan& d, int K, hipStream_t s);
+template <class S>
+void launch_m2l_valu(const DevicePlan& d, int K, hipStream_t s);
+// The bf16 mode's M2L for small batches (same view, state-major; needs no
+// split operands).
+void launch_m2l_bf16_direct(const DevicePlan& d, int K, hipStream_t s);
+// Operands of launch_m2l_full, built with the plan: class matrices C[row + n * depth]
+// in fragment order, and one parity offset with its class.
+std::vector<float> m2l_fragments_f32(int n, const std::vector<double>& C, int classes);
+std::vector<double> m2l_fragments_f64(int n, const std::vector<double>& C, int classes);
+int4 m2l_step(int ox, int oy, int oz, int cls);
 template <class S>
 void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s);
 // The vector-ALU near field (near_lanes.hip): any K, FP32 and FP64.
@@ -349,6 +363,9 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
 // operand layout, for plans whose upper levels are formed in compressed form.
 void launch_m2l_bf16_split(const DevicePlan& d, int K, hipStream_t s);
 void launch_m2l_mfma(const DevicePlan& d, int K, int mode, hipStream_t s);   // all levels 2..L
+// Columns per box of the 16-bit M2L operands at K states (the mt buffers hold
+// this many at the largest batch).
+int m2l_operand_states(const DevicePlan& d, int K);
 void prepare_mfma_operators(DevicePlan& d, int n, const std::vector<double>& matrices, int classes,
                             const std::vector<double>& local_scaling, std::vector<void*>& allocations, size_t& bytes);
 // FP16 operators of the harmonic form (n = nc); call after prepare_mfma_operators.

@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(256) split_kernel(const DevicePlan d, int K, i
 
 struct LevelTable {
   int count;  // entries, each a run of blocks of one level
+  int states;  // moment states of the output; the operands may hold more columns
   int level[12];
   int block_begin[12];
   int blocks_per_parity[12];
@@ -512,13 +513,16 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
   for (int nb = 0; nb < NB; ++nb) {
     if (!c.valid[nb]) continue;
     const int64_t tnode = sg.lvl0 + morton3(uint32_t(c.tx[nb]), uint32_t(c.ty[nb]), uint32_t(c.tz[nb]), level);
-    float* out = Lc + tnode * int64_t(n) * K + c.kk[nb] + (kUniformBox ? col : 0);
+    const int state = c.kk[nb] + (kUniformBox ? col : 0);
+    if (state >= lt.states) continue;  // a column of the padding
+    float* out = Lc + tnode * int64_t(n) * lt.states + (d.state_major ? state * n : state);
+    const int64_t row_step = d.state_major ? 1 : lt.states;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = m * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-        if (row < n) out[int64_t(row) * K] = (lsp[row] * unscale) * acc[nb][m][r];
+        if (row < n) out[row * row_step] = (lsp[row] * unscale) * acc[nb][m][r];
       }
   }
 }
@@ -528,8 +532,9 @@ bool uniform_box(const DevicePlan& d, int K) {
   return K % 32 == 0 && d.mt_zero_offset + 1024 <= int64_t(0xffffffffu);
 }
 
-LevelTable level_table(const DevicePlan& d, int K, int nb) {
+LevelTable level_table(const DevicePlan& d, int states, int K, int nb) {
   LevelTable lt{};
+  lt.states = states;
   lt.count = d.L - 1;
   // With one box per tile, tiles follow the plan's boundary-class order of
   // the parents for this workgroup size (kM2LGroupTiles).
@@ -609,8 +614,9 @@ void launch_uniform(const DevicePlan& v, const LevelTable& lt, int K, hipStream_
 }
 
 template <int MT, int NB, int kStages>
-void launch_mfma_cfg(const DevicePlan& d, int K, bool f16, hipStream_t s) {
-  const LevelTable lt = level_table(d, K, NB);
+void launch_mfma_cfg(const DevicePlan& d, int states, bool f16, hipStream_t s) {
+  const int K = m2l_operand_states(d, states);
+  const LevelTable lt = level_table(d, states, K, NB);
   const unsigned blocks = unsigned(lt.block_begin[lt.count]);
   const bool uniform = uniform_box(d, K);
   DevicePlan v = d;
@@ -712,7 +718,7 @@ __global__ void __launch_bounds__(256) level_max_kernel(const DevicePlan d, int 
   const float* cs = static_cast<const float*>(d.col16_scale);
   unsigned mx = 0u;
   for (int i = threadIdx.x; i < d.nc * K; i += blockDim.x)
-    mx = max(mx, __builtin_bit_cast(unsigned, fabsf(Mc[i] * cs[i / K])));
+    mx = max(mx, __builtin_bit_cast(unsigned, fabsf(Mc[i] * cs[d.compressed_state_major ? i % d.nc : i / K])));
   red[threadIdx.x] = mx;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -723,50 +729,53 @@ __global__ void __launch_bounds__(256) level_max_kernel(const DevicePlan d, int 
 }
 
 // FP16 hi/lo split of 2^e_l Mc / sigma into the MFMA B layout
-// mt[node][ks][K][16]; each thread packs 8 consecutive coefficients of one
-// column (reads coalesced over the K columns, 16-byte stores).
-__global__ void __launch_bounds__(256) split_f16_kernel(const DevicePlan d, int K) {
+// mt[node][ks][KO][16] (KO >= K columns, zeros from K on); each thread packs 8
+// consecutive coefficients of one column (16-byte stores).
+__global__ void __launch_bounds__(256) split_f16_kernel(const DevicePlan d, int K, int KO) {
   const int nc = d.nc, AP = d.apad, KS = AP / 16;
   const int64_t node = level_offset(2) + blockIdx.x;
   const int level = level_of_node(node);
   const float scale = ldexpf(1.0f, fp16_level_exponent(d.lvl_max_bits[level]));
   const float* Mc = static_cast<const float*>(d.Mc) + node * int64_t(nc) * K;
   const float* cs = static_cast<const float*>(d.col16_scale);
-  for (int w = threadIdx.x; w < K * (AP / 8); w += blockDim.x) {
-    const int k = w % K, a0 = (w / K) * 8;
+  const int row = d.compressed_state_major ? 1 : K, state = d.compressed_state_major ? nc : 1;
+  for (int w = threadIdx.x; w < KO * (AP / 8); w += blockDim.x) {
+    const int k = w % KO, a0 = (w / KO) * 8;
     half8 hi, lo;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int a = a0 + e;
-      const float x = a < nc ? (scale * cs[a]) * Mc[int64_t(a) * K + k] : 0.0f;
+      const float x = a < nc && k < K ? (scale * cs[a]) * Mc[a * row + k * state] : 0.0f;
       const _Float16 h = _Float16(x);
       hi[e] = h;
       lo[e] = _Float16(x - float(h));
     }
-    const int64_t at = ((node * KS + a0 / 16) * K + k) * 16 + a0 % 16;
+    const int64_t at = ((node * KS + a0 / 16) * KO + k) * 16 + a0 % 16;
     *reinterpret_cast<uint4*>(static_cast<_Float16*>(d.mt_hi) + at) = __builtin_bit_cast(uint4, hi);
     *reinterpret_cast<uint4*>(static_cast<_Float16*>(d.mt_lo) + at) = __builtin_bit_cast(uint4, lo);
   }
 }
 
-// bf16 hi/lo split of Mc into the MFMA B layout mt[node][ks][K][16] (levels
-// 2..L); each thread packs 8 consecutive coefficients of one column.
-__global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int K) {
+// bf16 hi/lo split of Mc into the MFMA B layout mt[node][ks][KO][16] (levels
+// 2..L, KO as above); each thread packs 8 consecutive coefficients of one
+// column.
+__global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int K, int KO) {
   const int nc = d.nc, AP = d.apad, KS = AP / 16;
   const int64_t node = level_offset(2) + blockIdx.x;
   const float* Mc = static_cast<const float*>(d.Mc) + node * int64_t(nc) * K;
-  for (int w = threadIdx.x; w < K * (AP / 8); w += blockDim.x) {
-    const int k = w % K, a0 = (w / K) * 8;
+  const int row = d.compressed_state_major ? 1 : K, state = d.compressed_state_major ? nc : 1;
+  for (int w = threadIdx.x; w < KO * (AP / 8); w += blockDim.x) {
+    const int k = w % KO, a0 = (w / KO) * 8;
     uint32_t hi[4], lo[4];
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-      const float x0 = a0 + e < nc ? Mc[int64_t(a0 + e) * K + k] : 0.0f;
-      const float x1 = a0 + e + 1 < nc ? Mc[int64_t(a0 + e + 1) * K + k] : 0.0f;
+      const float x0 = a0 + e < nc && k < K ? Mc[(a0 + e) * row + k * state] : 0.0f;
+      const float x1 = a0 + e + 1 < nc && k < K ? Mc[(a0 + e + 1) * row + k * state] : 0.0f;
       const uint16_t h0 = bf16_bits(x0), h1 = bf16_bits(x1);
       hi[e / 2] = uint32_t(h0) | (uint32_t(h1) << 16);
       lo[e / 2] = uint32_t(bf16_bits(x0 - bf16_value(h0))) | (uint32_t(bf16_bits(x1 - bf16_value(h1))) << 16);
     }
-    const int64_t at = (((node * KS + a0 / 16) * K + k) * 16 + a0 % 16) / 8;  // uint4 index
+    const int64_t at = (((node * KS + a0 / 16) * KO + k) * 16 + a0 % 16) / 8;  // uint4 index
     static_cast<uint4*>(d.mt_hi)[at] = uint4{hi[0], hi[1], hi[2], hi[3]};
     static_cast<uint4*>(d.mt_lo)[at] = uint4{lo[0], lo[1], lo[2], lo[3]};
   }
@@ -774,10 +783,19 @@ __global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int
 
 }  // namespace
 
+// From 9 states on a box's operand columns are padded with zeros to a multiple
+// of 32, so that every 32-column tile is one box and its step runs on the
+// uniform-box path: at 4681 boxes of p = 6 a batch of 12 to 31 states takes
+// 0.41 ms padded and 0.77-1.38 ms with several boxes per tile; up to 8 states
+// (four or more boxes per tile) it takes 0.37 ms.
+int m2l_operand_states(const DevicePlan& d, int K) {
+  return d.nc == 0 || K < 9 ? K : (K + 31) / 32 * 32;
+}
+
 void launch_m2l_bf16_split(const DevicePlan& d, int K, hipStream_t s) {
   if (d.L < 2) return;
   const unsigned boxes = unsigned(d.nodes - level_offset(2));
-  split_bf16_kernel<<<boxes, 256, 0, s>>>(d, K);
+  split_bf16_kernel<<<boxes, 256, 0, s>>>(d, K, m2l_operand_states(d, K));
   HIPFMM_CHECK(hipGetLastError());
 }
 
@@ -787,7 +805,7 @@ void launch_m2l_fp16_split(const DevicePlan& d, int K, hipStream_t s) {
   launch_zero<float>(reinterpret_cast<float*>(d.lvl_max_bits), size_t(d.L + 1), s);
   level_max_kernel<<<boxes, 256, 0, s>>>(d, K);
   HIPFMM_CHECK(hipGetLastError());
-  split_f16_kernel<<<boxes, 256, 0, s>>>(d, K);
+  split_f16_kernel<<<boxes, 256, 0, s>>>(d, K, m2l_operand_states(d, K));
   HIPFMM_CHECK(hipGetLastError());
 }
 

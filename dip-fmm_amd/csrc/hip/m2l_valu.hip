@@ -1,4 +1,6 @@
-// Plain M2L on the vector ALUs (FP32 or FP64 FMA): the baseline path.
+// M2L on the vector ALUs (FP32 or FP64 FMA) for class matrices that do not
+// factor through the harmonic subspace (a descriptor with matrices of its own);
+// those that do run in m2l_full.hip.
 //
 // Reference: apply_static_m2l_plan / apply_scaled_m2l_rows_kernel
 // (src/static_operators.cpp:16-102, src/cuda_fmm.cu:142-189):
@@ -16,13 +18,8 @@
 // (column = target box x moment state); accumulation is in registers and
 // every local is written once, without atomics.  Empty source boxes carry
 // exact zero multipoles, so they need no test.  One launch covers every
-// level 2..L, so the small upper levels overlap the leaf level.  FP32 plans
-// with n = (p + 1)^2, p = 1..8 (the harmonic-subspace sizes), run the
-// register-tiled form below.
+// level 2..L, so the small upper levels overlap the leaf level.
 #include "common.hpp"
-
-#include <map>
-#include <mutex>
 
 namespace hipfmm {
 
@@ -37,7 +34,6 @@ struct ValuLevels {
   int boxes_per_tile;
   int k_per_tile;
   int kchunks;
-  int parts;  // offset parts per tile (register-tiled kernel; 1 elsewhere)
 };
 
 template <class S>
@@ -116,323 +112,30 @@ __global__ void m2l_valu_kernel(const DevicePlan d, const ValuLevels lv, int K) 
   }
 }
 
-// FP32 register-tiled form for the harmonic sizes n = (p + 1)^2, p = 1..8.
-// A workgroup of 16 * RG threads owns one parity class's tile of 64 columns
-// (target box x moment state) and all n output rows; thread (ty, tx)
-// accumulates rows RT * ty .. + RT - 1 (RG * RT >= n) and columns
-// 4 tx .. + 3, so each alpha step costs RT broadcast values of T_o and one
-// float4 of sources for 4 RT FMAs.  Per offset the class matrix T_o
-// (n x n, copied as stored: row alpha = the coefficients of source alpha)
-// and the gathered, scaled source coefficients are staged in LDS; the next
-// offset's values are loaded into registers while the current one is
-// multiplied, so the global latency hides behind the FMAs.  The product
-// order per output element (alpha ascending within each offset, offsets in
-// list order) is that of m2l_valu_kernel.
-constexpr int kTileCols = 64;
-
-// Rows per thread for n coefficients.  n = 49 and 81 (p = 6 and 8) take the
-// shapes that a sweep of RT = 1..6 on MI355X found fastest (2^20 uniform
-// points, depth 5; M2L kernel ms at one state / 32 states):
-//   n = 49: RT 1 1.78, 2 1.44, 3 2.52, 4 1.27, 5 2.15, 6 2.44 (one state)
-//   n = 81: RT 2 3.76 / 77.0, 3 3.03 / 61.4, 4 4.57 / 100.6, 5 4.71 / 104.9,
-//           6 3.94 / 69.7
-// The spread follows the registers: the prefetched values cost NT + NG
-// VGPRs per thread, and the shapes that keep two or three workgroups per CU
-// win (at one state the depth-5 grid is 592 workgroups, so three per CU run
-// it in one round).  Other sizes take the fewest wavefront issue slots per
-// alpha step, wavefronts x (2 RT + 1) (4 RT FMAs against RT + 1 LDS reads),
-// the larger RT on a tie, RT <= 6, at most 1024 threads.
-constexpr int tiled_rows_per_thread(int n) {
-  if (n == 49) return 4;
-  if (n == 81) return 3;
-  int best = 1, best_cost = 1 << 30;
-  for (int rt = 1; rt <= 6; ++rt) {
-    const int threads = 16 * ((n + rt - 1) / rt);
-    if (threads > 1024) continue;
-    const int cost = ((threads + 63) / 64) * (2 * rt + 1);
-    if (cost <= best_cost) best = rt, best_cost = cost;
-  }
-  return best;
-}
-
-template <int N, int RT_>
-struct TiledShape {
-  static constexpr int RT = RT_;
-  static constexpr int RG = (N + RT - 1) / RT;
-  static constexpr int THREADS = 16 * RG;
-  static constexpr int BR = RG * RT;  // rows computed; rows n..BR-1 read T's next row and are dropped
-  static constexpr int T_LDS = (N * N + (BR - N) + 3) / 4 * 4;
-  static constexpr int NT = (N * N + THREADS - 1) / THREADS;          // T values per thread and offset
-  static constexpr int NG = (N * kTileCols + THREADS - 1) / THREADS;  // gathered values per thread and offset
-};
-
-template <int N, int RT_>
-__global__ void __launch_bounds__(16 * ((N + RT_ - 1) / RT_))
-    m2l_valu_tiled_kernel(const DevicePlan d, const ValuLevels lv, int K) {
-  using Sh = TiledShape<N, RT_>;
-  constexpr int RT = Sh::RT, THREADS = Sh::THREADS;
-  static_assert(THREADS == 16 * ((N + RT_ - 1) / RT_), "launch bound");
-  __shared__ __align__(16) float tl[Sh::T_LDS];          // T_o[alpha][beta], then zero slack
-  __shared__ __align__(16) float ml[N * kTileCols];      // [alpha][column]: scaled sources
-  __shared__ int4 tbox[kTileCols];                       // target box coords + valid flag, per column
-  __shared__ int64_t src[kTileCols];                     // index of (source, alpha 0, state) in M, or -1
-  __shared__ float scale[N];                             // source scaling ms[level][alpha]
-  int li = lv.count - 1;
-  while (li > 0 && int(blockIdx.x) < lv.block_begin[li]) --li;
-  const int level = 2 + li;
-  const int lb = int(blockIdx.x) - lv.block_begin[li];
-  const int parity = lb & 7, rest = lb >> 3;
-  const int tile = rest % lv.tiles[li], kc = (rest / lv.tiles[li]) % lv.kchunks;
-  const int part = rest / lv.tiles[li] / lv.kchunks;
-  // This workgroup's share of the parity's offsets.
-  const int o_begin = part * 189 / lv.parts, o_end = (part + 1) * 189 / lv.parts;
-  const int px = parity & 1, py = (parity >> 1) & 1, pz = (parity >> 2) & 1;
-  const int nbox = 1 << level;
-  const int64_t parents = int64_t(1) << (3 * (level - 1));
-  const int bpt = lv.boxes_per_tile, kpt = lv.k_per_tile;
-  const int64_t q0 = int64_t(tile) * bpt;
-  const int k0 = kc * kpt;
-  const int64_t lvl0 = level_offset(level);
-  const int tid = threadIdx.x;
-  // The tables have 64 entries and a workgroup may have fewer threads.
-  for (int j = tid; j < kTileCols; j += THREADS) {
-    const int b = j / kpt;
-    int4 tb{0, 0, 0, 0};
-    if (b < bpt && q0 + b < parents && k0 + j % kpt < K) {
-      int x, y, z;
-      demorton3(uint32_t(q0 + b), level - 1, x, y, z);
-      tb = int4{2 * x + px, 2 * y + py, 2 * z + pz, 1};
-    }
-    tbox[j] = tb;
-  }
-  for (int w = N * N + tid; w < Sh::T_LDS; w += THREADS) tl[w] = 0.0f;
-  const float* M = static_cast<const float*>(d.M);
-  const float* msl = static_cast<const float*>(d.ms) + int64_t(level) * N;
-  const float* T = static_cast<const float*>(d.m2l_T);
-  const int4* offs = d.parity_offsets + parity * 189;
-  // Column j of the table: where source box t - o keeps its coefficients.
-  auto source_index = [&](int4 o, int j) {
-    const int4 tb = tbox[j];
-    const int sx = tb.x - o.x, sy = tb.y - o.y, sz = tb.z - o.z;
-    if (!tb.w || sx < 0 || sy < 0 || sz < 0 || sx >= nbox || sy >= nbox || sz >= nbox) return int64_t(-1);
-    const int64_t snode = lvl0 + morton3(uint32_t(sx), uint32_t(sy), uint32_t(sz), level);
-    return snode * N * K + k0 + j % kpt;
-  };
-  for (int a = tid; a < N; a += THREADS) scale[a] = msl[a];
-  // The loads go out unconditionally (absent sources read M[0]) and their
-  // validity is kept as a bit mask applied at the LDS store, so no use of a
-  // loaded value precedes the next offset's multiply loop.
-  float pt[Sh::NT], pm[Sh::NG];
-  uint32_t valid = 0;
-  static_assert(Sh::NG <= 32, "validity mask");
-  auto load = [&](int4 o) {
-    const float* To = T + int64_t(o.w) * N * N;
-#pragma unroll
-    for (int i = 0; i < Sh::NT; ++i) pt[i] = To[min(tid + THREADS * i, N * N - 1)];
-    valid = 0;
-#pragma unroll
-    for (int i = 0; i < Sh::NG; ++i) {
-      const int w = tid + THREADS * i;
-      const int64_t s0 = w < N * kTileCols ? src[w % kTileCols] : int64_t(-1);
-      valid |= uint32_t(s0 >= 0) << i;
-      pm[i] = M[s0 >= 0 ? s0 + int64_t(w / kTileCols) * K : 0];
-    }
-  };
-  __syncthreads();  // tbox, scale
-  for (int j = tid; j < kTileCols; j += THREADS) src[j] = source_index(offs[o_begin], j);
-  __syncthreads();
-  load(offs[o_begin]);
-  const int tx = tid & 15, ty = tid >> 4;
-  float acc[RT][4];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[i][c] = 0.0f;
-  for (int oi = o_begin; oi < o_end; ++oi) {
-    __syncthreads();  // every thread is done with the previous offset's tiles and table
-#pragma unroll
-    for (int i = 0; i < Sh::NT; ++i) {
-      const int w = tid + THREADS * i;
-      if (w < N * N) tl[w] = pt[i];
-    }
-#pragma unroll
-    for (int i = 0; i < Sh::NG; ++i) {
-      const int w = tid + THREADS * i;
-      if (w < N * kTileCols) ml[w] = (valid >> i) & 1 ? scale[w / kTileCols] * pm[i] : 0.0f;
-    }
-    if (oi + 1 < o_end)
-      for (int j = tid; j < kTileCols; j += THREADS) src[j] = source_index(offs[oi + 1], j);
-    __syncthreads();
-    if (oi + 1 < o_end) load(offs[oi + 1]);
-    const float* tr = tl + RT * ty;
-    const float4* mr = reinterpret_cast<const float4*>(ml) + tx;
-#pragma unroll 9
-    for (int a = 0; a < N; ++a) {
-      const float4 m4 = mr[a * (kTileCols / 4)];
-      const float mv[4] = {m4.x, m4.y, m4.z, m4.w};
-      float tv[RT];
-#pragma unroll
-      for (int i = 0; i < RT; ++i) tv[i] = tr[a * N + i];
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[i][c] += tv[i] * mv[c];
-    }
-  }
-  const float* lsl = static_cast<const float*>(d.ls) + int64_t(level) * N;
-  // One part writes the locals; several write their partial sums, which
-  // m2l_valu_sum_parts_kernel adds in part order.
-  float* Lc = lv.parts == 1 ? static_cast<float*>(d.Lc)
-                            : static_cast<float*>(d.m2l_part) + int64_t(part) * d.nodes * N * K;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int j = 4 * tx + c;
-    const int4 tb = tbox[j];
-    if (!tb.w) continue;
-    const int64_t tnode = lvl0 + morton3(uint32_t(tb.x), uint32_t(tb.y), uint32_t(tb.z), level);
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-      const int beta = RT * ty + i;
-      if (beta < N) Lc[(tnode * N + beta) * K + k0 + j % kpt] = lsl[beta] * acc[i][c];
-    }
-  }
-}
-
-template <int N>
-void launch_tiled(const DevicePlan& d, const ValuLevels& lv, int blocks, int K, hipStream_t s) {
-  constexpr int rt = tiled_rows_per_thread(N);
-  m2l_valu_tiled_kernel<N, rt><<<unsigned(blocks), TiledShape<N, rt>::THREADS, 0, s>>>(d, lv, K);
-}
-
-ValuLevels valu_levels(const DevicePlan& d, int K, int cols, int& blocks, int parts = 1) {
+ValuLevels valu_levels(const DevicePlan& d, int K, int cols, int& blocks) {
   ValuLevels lv{};
   lv.count = d.L - 1;
   lv.k_per_tile = K >= cols ? cols : K;
   lv.boxes_per_tile = cols / lv.k_per_tile;
   lv.kchunks = (K + lv.k_per_tile - 1) / lv.k_per_tile;
-  lv.parts = parts;
   int begin = 0;
   for (int i = 0; i < lv.count; ++i) {
     const int64_t parents = int64_t(1) << (3 * (i + 1));
     lv.tiles[i] = int((parents + lv.boxes_per_tile - 1) / lv.boxes_per_tile);
     lv.block_begin[i] = begin;
-    begin += 8 * lv.tiles[i] * lv.kchunks * parts;
+    begin += 8 * lv.tiles[i] * lv.kchunks;
   }
   lv.block_begin[lv.count] = begin;
   blocks = begin;
   return lv;
 }
 
-// Lc = the parts' partial sums added in part order, over the nodes of
-// levels 2..L.
-__global__ void __launch_bounds__(256) m2l_valu_sum_parts_kernel(const DevicePlan d, int K, int parts) {
-  const int64_t first = level_offset(2) * d.n * K, count = (level_offset(d.L + 1) - level_offset(2)) * d.n * K;
-  const int64_t stride = int64_t(d.nodes) * d.n * K;
-  const float* part = static_cast<const float*>(d.m2l_part);
-  float* Lc = static_cast<float*>(d.Lc);
-  for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < count; i += int64_t(gridDim.x) * 256) {
-    float v = part[first + i];
-    for (int p = 1; p < parts; ++p) v += part[int64_t(p) * stride + first + i];
-    Lc[first + i] = v;
-  }
-}
-
-// Resident workgroups per CU of the tiled kernel for N, asked of the runtime
-// once per device.
-template <int N>
-int tiled_workgroups_per_cu(int device) {
-  static std::mutex mutex;
-  static std::map<int, int> known;
-  std::lock_guard<std::mutex> lock(mutex);
-  const auto it = known.find(device);
-  if (it != known.end()) return it->second;
-  constexpr int rt = tiled_rows_per_thread(N);
-  int per_cu = 0;
-  HIPFMM_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, m2l_valu_tiled_kernel<N, rt>,
-                                                            TiledShape<N, rt>::THREADS, 0));
-  known[device] = per_cu;
-  return per_cu;
-}
-
 }  // namespace
-
-int device_cu_count(int device) {
-  static std::mutex mutex;
-  static std::map<int, int> known;
-  std::lock_guard<std::mutex> lock(mutex);
-  const auto it = known.find(device);
-  if (it != known.end()) return it->second;
-  int cus = 0;
-  HIPFMM_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  known[device] = cus;
-  return cus;
-}
-
-// Offset parts per tile of the register-tiled kernel at K states.  A grid of
-// few tiles leaves the last round of resident workgroups part-empty (at one
-// state the depth-5 grid is 592 workgroups for 512 resident slots at
-// p = 8); splitting every tile's 189 offsets into S parts runs the same work
-// in S times as many, S times shorter workgroups.  S in 1..kValuMaxParts
-// minimises ceil(S * blocks / slots) / S (the rounds, each 1/S as long),
-// the smaller S on a tie; a split must save at least a tenth of the rounds
-// to be taken (each part adds its partial sums' traffic).
-int m2l_valu_parts(const DevicePlan& d, int K) {
-  if (d.precision != 32 || d.L < 2) return 1;
-  int blocks = 0;
-  (void)valu_levels(d, K, kTileCols, blocks);
-  int device = 0, per_cu = 0;
-  HIPFMM_CHECK(hipGetDevice(&device));
-  switch (d.n) {
-    case 4: per_cu = tiled_workgroups_per_cu<4>(device); break;
-    case 9: per_cu = tiled_workgroups_per_cu<9>(device); break;
-    case 16: per_cu = tiled_workgroups_per_cu<16>(device); break;
-    case 25: per_cu = tiled_workgroups_per_cu<25>(device); break;
-    case 36: per_cu = tiled_workgroups_per_cu<36>(device); break;
-    case 49: per_cu = tiled_workgroups_per_cu<49>(device); break;
-    case 64: per_cu = tiled_workgroups_per_cu<64>(device); break;
-    case 81: per_cu = tiled_workgroups_per_cu<81>(device); break;
-    default: return 1;
-  }
-  const int cus = device_cu_count(device);
-  const int64_t slots = int64_t(std::max(per_cu, 1)) * std::max(cus, 1);
-  const double whole = double((blocks + slots - 1) / slots);
-  int best = 1;
-  double best_cost = whole;
-  for (int parts = 2; parts <= kValuMaxParts; ++parts) {
-    const double cost = double((int64_t(blocks) * parts + slots - 1) / slots) / parts;
-    if (cost < best_cost - 1e-9) best = parts, best_cost = cost;
-  }
-  return best_cost <= 0.9 * whole ? best : 1;
-}
 
 template <class S>
 void launch_m2l_valu(const DevicePlan& d, int K, hipStream_t s) {
   if (d.L < 2) return;
   int blocks = 0;
-  if constexpr (sizeof(S) == 4) {
-    int parts = m2l_valu_parts(d, K);
-    if (parts > 1 && (d.m2l_part == nullptr || int64_t(parts) * K > d.m2l_part_capacity)) parts = 1;
-    const ValuLevels lv = valu_levels(d, K, kTileCols, blocks, parts);
-    if (blocks >= 0) switch (d.n) {
-      case 4: launch_tiled<4>(d, lv, blocks, K, s); break;
-      case 9: launch_tiled<9>(d, lv, blocks, K, s); break;
-      case 16: launch_tiled<16>(d, lv, blocks, K, s); break;
-      case 25: launch_tiled<25>(d, lv, blocks, K, s); break;
-      case 36: launch_tiled<36>(d, lv, blocks, K, s); break;
-      case 49: launch_tiled<49>(d, lv, blocks, K, s); break;
-      case 64: launch_tiled<64>(d, lv, blocks, K, s); break;
-      case 81: launch_tiled<81>(d, lv, blocks, K, s); break;
-      default: blocks = -1;
-    }
-    if (blocks >= 0) {
-      HIPFMM_CHECK(hipGetLastError());
-      if (parts > 1) {
-        m2l_valu_sum_parts_kernel<<<2048, 256, 0, s>>>(d, K, parts);
-        HIPFMM_CHECK(hipGetLastError());
-      }
-      return;
-    }
-  }
   const ValuLevels lv = valu_levels(d, K, kCols, blocks);
   const int threads = ((d.n + 63) / 64) * 64;
   const size_t lds = size_t(d.n) * kCols * sizeof(S);

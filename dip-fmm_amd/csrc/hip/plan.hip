@@ -495,8 +495,6 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
             require(slot[hipfmm::offset_slot(x, y, z)] >= 0, "an M2L class matrix for a list-2 offset is missing");
   }
   const size_t nn = size_t(n) * n;
-  std::vector<S> T(std::max<size_t>(size_t(desc.m2l_class_count) * nn, 1));
-  for (size_t i = 0; i < size_t(desc.m2l_class_count) * nn; ++i) T[i] = S(desc.m2l_matrices[i]);
   // Harmonic-subspace form of the M2L (T_o = Q C_o P): class matrices of
   // size nc x nc and the level scalings folded into P and Q.
   hipfmm::HarmonicBasis hb;
@@ -504,10 +502,7 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   if (hb.nc > 0) {
     const int nc = hb.nc, NPc = (nc + 15) / 16 * 16, NP = (n + 7) / 8 * 8;
     d.nc = nc;
-    T.assign(std::max<size_t>(hb.C.size(), 1), S(0));
-    for (size_t i = 0; i < hb.C.size(); ++i) T[i] = S(hb.C[i]);
     std::vector<S> cmp(size_t(L + 1) * n * NPc, S(0)), expd(size_t(L + 1) * nc * NP, S(0));
-    std::vector<S> ones(size_t(L + 1) * nc, S(1));
     for (int l = 0; l <= L; ++l)
       for (int r = 0; r < nc; ++r) {
         for (int a = 0; a < n; ++a)
@@ -523,7 +518,15 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
       d.cmp_x3 = upload(P, c3.data(), c3.size());
       d.exp_x3 = upload(P, e3.data(), e3.size());
     }
-    d.unit_scale = upload(P, ones.data(), ones.size());
+    if constexpr (sizeof(S) == 4) {
+      const auto f = hipfmm::m2l_fragments_f32(nc, hb.C, desc.m2l_class_count);
+      d.m2l_fragments = upload(P, f.data(), f.size());
+    } else {
+      const auto f = hipfmm::m2l_fragments_f64(nc, hb.C, desc.m2l_class_count);
+      d.m2l_fragments = upload(P, f.data(), f.size());
+    }
+    const std::vector<S> zero_box(size_t(nc) * hipfmm::kMaxBatch, S(0));
+    d.m2l_zero_box = upload(P, zero_box.data(), zero_box.size());
     P->stats.m2l_reconstruction_error = hb.max_reconstruction_error;
     // FP32 plans run the upward and downward passes in the harmonic subspace
     // too.  A multipole with no harmonic part has no field, and neither has
@@ -604,7 +607,11 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
       P->stats.harmonic_pass_leak = leak;
     }
   }
-  d.m2l_T = upload(P, T.data(), T.size());
+  if (hb.nc == 0) {
+    std::vector<S> T(std::max<size_t>(size_t(desc.m2l_class_count) * nn, 1));
+    for (size_t i = 0; i < size_t(desc.m2l_class_count) * nn; ++i) T[i] = S(desc.m2l_matrices[i]);
+    d.m2l_T = upload(P, T.data(), T.size());
+  }
   d.m2l_slot = upload(P, slot.data(), slot.size());
   // The 189 list-2 offsets of each parity class (target coordinate parity
   // q per axis: offsets in [q-3, q+2] minus the near cube), ordered by the
@@ -627,6 +634,12 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
     }
   }
   d.parity_offsets = upload(P, parity_offsets.data(), parity_offsets.size());
+  std::vector<int4> parity_steps(parity_offsets.size());
+  for (size_t i = 0; i < parity_steps.size(); ++i) {
+    const int4 o = parity_offsets[i];
+    parity_steps[i] = hipfmm::m2l_step(o.x, o.y, o.z, o.w);
+  }
+  d.m2l_steps = upload(P, parity_steps.data(), parity_steps.size());
   // Tile order of the matrix-core M2L.  A workgroup applies every offset
   // that any of its boxes uses, so a box whose list 2 is cut by the grid
   // boundary multiplies zeros for the offsets it lacks.  Along each axis only
@@ -835,28 +848,8 @@ void ensure_capacity(hipfmm_plan* P, int K, bool potential, bool gradient = fals
     HIPFMM_CHECK(hipMemset(d.Mc, 0, cc * sizeof(S)));
     HIPFMM_CHECK(hipMemset(d.Lcc, 0, cc * sizeof(S)));
   }
-  // Partial sums of the split vector-ALU M2L, for the largest parts x K any
-  // batch up to the capacity asks for, within kValuPartBytes (batches
-  // beyond it run unsplit; none split at most sizes).
-  d.m2l_part = nullptr;
-  d.m2l_part_capacity = 0;
-  if (sizeof(S) == 4 && d.nc > 0 && d.L >= 2) {
-    DevicePlan dm = d;
-    dm.n = d.nc;
-    constexpr size_t kValuPartBytes = size_t(256) << 20;
-    const size_t per_state = size_t(d.nodes) * d.nc * sizeof(S);
-    int need = 0;
-    for (int k = 1; k <= cap; ++k) {
-      const int parts = hipfmm::m2l_valu_parts(dm, k);
-      if (parts > 1 && size_t(parts) * k * per_state <= kValuPartBytes) need = std::max(need, parts * k);
-    }
-    if (need > 0) {
-      d.m2l_part = alloc(size_t(d.nodes) * d.nc * need, sizeof(S));
-      d.m2l_part_capacity = need;
-    }
-  }
   if (sizeof(S) == 4 && P->mfma_ready) {
-    const size_t ms = size_t(d.nodes) * cap * d.apad;
+    const size_t ms = size_t(d.nodes) * hipfmm::m2l_operand_states(d, cap) * d.apad;
     // Each half is followed by a 1 KiB zero block (the operand of sources
     // outside the grid); zeroed once here.
     d.mt_zero_offset = int64_t(ms) * 2;
@@ -976,7 +969,8 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   // only when timings are asked for, so the host can enqueue ahead.
   (void)hipGetLastError();
   ensure_capacity<S>(P, K, want_pot, want_grad);
-  const DevicePlan d = adjoint ? role_exchanged(P) : P->d;
+  DevicePlan d = adjoint ? role_exchanged(P) : P->d;
+  d.compressed_state_major = d.nc > 0 && (sizeof(S) == 8 || K % 32 != 0);
   hipStream_t s = P->s_far;
   hipEvent_t* e = P->ev;
   auto mark = [&](int ev, hipStream_t on) {
@@ -1064,6 +1058,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     dc.n = d.nc;
     dc.M = d.Mc;
     dc.Lc = d.Lcc;
+    dc.state_major = d.compressed_state_major;
     dc.m2m_dense = d.m2m_dense_c;
     dc.l2l_dense = d.l2l_dense_c;
     dc.m2m_x3 = d.m2m_x3_c;
@@ -1078,16 +1073,35 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   hipfmm::launch_zero<S>(static_cast<S*>(d.M), top, s);
   hipfmm::launch_zero<S>(static_cast<S*>(d.Lc), d.L >= 2 ? top : size_t(d.nodes) * d.n * K, s);
   mark(kEvM2M, s);
-  const bool mfma = sizeof(S) == 4 && P->m2l_mode != HIPFMM_M2L_VALU && P->mfma_ready;
+  // The 16-bit modes split the multipoles in a pass of their own and run in
+  // workgroups of 256 columns whose chain of up to 189 offsets takes 0.23-0.6
+  // ms however few there are.  A small batch runs on the direct kernels
+  // instead, whose waves share the offsets and which need no split: the bf16
+  // mode in its own arithmetic, the FP16 mode in full FP32 (24 bits per
+  // operand against 22, and no pass over the level maxima).  The line is at
+  // the batch's size in boxes x states x coefficients.  Whole evaluates (ms,
+  // workgroups of 256 / direct), bf16: p = 8, 4681 boxes 0.92 / 0.49 at K = 1,
+  // 1.24 / 1.06 at 6, 1.32 / 1.26 at 8 (3.0e6); 37449 boxes 2.07 / 1.96 at
+  // K = 1 (3.0e6), 2.92 / 3.04 at 2; p = 6 1.49 / 1.40 at 1, 2.03 / 2.00 at 2
+  // (3.7e6), 2.58 / 2.80 at 3.  FP16: p = 8, 4681 boxes 1.12 / 1.06 at K = 4,
+  // 1.24 / 1.36 at 6 (2.3e6); p = 6 0.82 / 0.76 at 6, 0.86 / 0.89 at 8 (1.8e6).
+  // From 9 states on the operands are padded to whole 32-column boxes (see
+  // m2l_operand_states) and the line is lower: bf16 p = 6, 585 boxes
+  // 0.48 / 0.45 at K = 24 (6.9e5), 0.55 / 0.58 at 31.
+  const bool sixteen = sizeof(S) == 4 && P->m2l_mode != HIPFMM_M2L_VALU && P->mfma_ready;
+  const bool bf16 = P->m2l_mode == HIPFMM_M2L_MFMA_BF16X3;
+  const int64_t size = d.nodes * K * d.nc;
+  const bool small = d.nc > 0 && K % 32 != 0 && size <= (K < 9 ? (bf16 ? 3500000 : 1800000) : 700000);
+  const bool mfma = sixteen && !small;
   // The M2L kernels see the plan through `dm`: in harmonic-subspace form the
-  // operands are the compressed multipoles/locals with unit scalings.
+  // operands are the compressed multipoles/locals (the level scalings are in
+  // the transforms).
   DevicePlan dm = d;
   if (d.nc > 0 && d.L >= 2) {
     dm.n = d.nc;
     dm.M = d.Mc;
     dm.Lc = d.Lcc;
-    dm.ms = d.unit_scale;
-    dm.ls = d.unit_scale;
+    dm.state_major = d.compressed_state_major;
     if (!harmonic) hipfmm::launch_m2l_compress<S>(d, K, 2, s);
     if (mfma && P->m2l_mode == HIPFMM_M2L_MFMA_FP16X3)
       hipfmm::launch_m2l_fp16_split(d, K, s);
@@ -1113,6 +1127,10 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][0], s));
   if (mfma)
     hipfmm::launch_m2l_mfma(dm, K, P->m2l_mode, s);
+  else if (sixteen && bf16 && small)
+    hipfmm::launch_m2l_bf16_direct(dm, K, s);
+  else if (d.nc > 0)
+    hipfmm::launch_m2l_full<S>(dm, K, s);
   else
     hipfmm::launch_m2l_valu<S>(dm, K, s);
   mark(kEvM2LKernel1, s);
