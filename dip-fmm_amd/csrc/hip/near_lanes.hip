@@ -20,12 +20,18 @@
 // (the targets past its end are skipped by a uniform branch).  The lanes'
 // sums meet in one butterfly per T targets.
 //
+// A wave's targets come from the list of 16-target tiles, so a leaf of many
+// targets is many waves: with a workgroup per leaf clustered points waited for
+// the fullest leaves (100,000 points in blobs, depth 5, K = 8: 1.16 ms, now
+// .36) and small trees left the chip idle (20,000 points, 512 leaves, K = 1
+// .06, now .034).
+//
 // Measured (near field alone, ms; in brackets the form before it, a workgroup
 // of 32 target slots per pass that staged each neighbour leaf's sources in LDS
 // and formed a pair's geometry once per 1, 4 or 8 states): 2^20 points, 32 per
-// leaf, FP32: K = 1 1.00 (1.77), 2 1.34 (2.70), 4 2.09 (4.61), 8 3.21 (8.01),
-// 16 6.5 (8.3); fields and potentials K = 4 2.28 (4.72); gradients K = 1 1.46
-// (2.05).  256 per leaf: K = 8 19.0 (48.5).  FP64, 2^18 points, 64 per leaf:
+// leaf, FP32: K = 1 .88 (1.77), 2 1.08 (2.70), 4 1.87 (4.61), 8 3.06 (8.01);
+// fields and potentials K = 4 2.08 (4.72); gradients K = 1 1.25 (2.05).
+// 512 per leaf, 2^18 points: K = 8 6.5.  FP64, 2^18 points, 64 per leaf:
 // K = 1 1.09 (1.43), 4 1.87 (4.73).
 #include "common.hpp"
 
@@ -33,7 +39,7 @@ namespace hipfmm {
 
 namespace {
 
-constexpr int kWaves = 4;  // waves per workgroup; each takes every 4th group of T targets of the leaf
+constexpr int kWaves = 4;  // waves per workgroup, each with T targets of a 16-target tile
 
 enum NearOutput { kField = 0, kFieldAndPotential = 1, kGradient = 2 };
 
@@ -128,128 +134,133 @@ struct __attribute__((packed, aligned(sizeof(S)))) States {
   S v[KS];
 };
 
-// Workgroup per target leaf and group of KS <= K states (blockIdx.y; the last
-// group ends at K and may repeat states of the one before, which stores them).
+// A wave has T targets of one leaf and KS <= K states (blockIdx.y; the last
+// group of states ends at K and may repeat some of the one before, which
+// stores them).
 template <class S, int KS, int kWhat>
 __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePlan d, int K) {
   constexpr int T = near_targets<S>(KS, kWhat), C = near_rows(kWhat), V = T * C * KS;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
-  const int leaf = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x));
+  // The tile list's 16 targets in groups of T: a leaf of many targets is as
+  // many waves, whatever the other leaves hold.
+  const int item = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x)) * kWaves + wave;
+  if (item >= d.p2p_tile16_count * (16 / T)) return;
+  const int2 tile = d.p2p_tiles16[item / (16 / T)];
+  const int leaf = tile.x;
   const int2 range = d.leaf_tgt[leaf];
+  const int t0 = range.x + tile.y + item % (16 / T) * T, cnt = min(T, range.y - t0);
+  if (cnt <= 0) return;
   const int k_first = int(blockIdx.y) * KS, k0 = min(k_first, K - KS);
   const int q0 = d.nbr_blk_start[leaf], q1 = d.nbr_blk_start[leaf + 1];
   const S* sm = static_cast<const S*>(d.sm);
   const int group = lane >> 3, e = lane & 7;  // block of the batch, source of the block
-  for (int t0 = range.x + wave * T; t0 < range.y; t0 += kWaves * T) {
-    const int cnt = min(T, range.y - t0);
-    Point<S> tp[T];
-    int self[T];
+  Point<S> tp[T];
+  int self[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int t = i < cnt ? t0 + i : t0;
+    tp[i] = Point<S>::load(d.tgt_pos, d.nt, t);
+    self[i] = __builtin_amdgcn_readfirstlane(d.self[t]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      tp[i].h[c] = uniform(tp[i].h[c]);
+      if constexpr (sizeof(S) == 4) tp[i].l[c] = uniform(tp[i].l[c]);
+    }
+  }
+  S acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = S(0);
+  int2 blk = int2{0, 0};  // first source and count of this lane's block
+  auto block_of = [&](int q) {
+    return q + group < q1 ? d.blk8_src[d.nbr_blk[q + group]] : int2{0, 0};
+  };
+  if (q0 < q1) blk = block_of(q0);
+  for (int q = q0; q < q1; q += 8) {
+    // A lane without a source takes one out of reach with no moment: its
+    // |r|^-1 is tiny and every term of it zero.
+    const bool have = e < blk.y;
+    const int s = have ? blk.x + e : -2;
+    Point<S> sp;
+    S m[3][KS];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      sp.h[c] = Point<S>::far();
+      if constexpr (sizeof(S) == 4) sp.l[c] = S(0);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) m[c][k] = S(0);
+    }
+    if (have) {
+      sp = Point<S>::load(d.src_pos, d.ns, s);
+      const S* ms = sm + int64_t(s) * 3 * K + k0;
+      if (KS == K) {  // one contiguous row
+        const auto row = *reinterpret_cast<const States<S, 3 * KS>*>(ms);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int k = 0; k < KS; ++k) m[c][k] = row.v[c * KS + k];
+      } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const auto row = *reinterpret_cast<const States<S, KS>*>(ms + c * K);
+#pragma unroll
+          for (int k = 0; k < KS; ++k) m[c][k] = row.v[k];
+        }
+      }
+    }
+    if (q + 8 < q1) blk = block_of(q + 8);
 #pragma unroll
     for (int i = 0; i < T; ++i) {
-      const int t = i < cnt ? t0 + i : t0;
-      tp[i] = Point<S>::load(d.tgt_pos, d.nt, t);
-      self[i] = __builtin_amdgcn_readfirstlane(d.self[t]);
+      if (i >= cnt || s == self[i]) continue;
+      const S rx = tp[i].minus(sp, 0), ry = tp[i].minus(sp, 1), rz = tp[i].minus(sp, 2);
+      const S r2 = rx * rx + ry * ry + rz * rz;
+      const S rinv = near_rsqrt(r2);
+      const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
+      S* a = acc + i * C * KS;
+      if constexpr (kWhat == kGradient) {
+        // dH_c/dx_j, 3/(4 pi |r|^4) (delta_cj w + u_c m_j + m_c u_j - 5 u_c u_j w), w = u.m.
+        const S g = S(0.23873241463784300365332564505877154) * rinv * rinv * rinv * rinv;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        tp[i].h[c] = uniform(tp[i].h[c]);
-        if constexpr (sizeof(S) == 4) tp[i].l[c] = uniform(tp[i].l[c]);
-      }
-    }
-    S acc[V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) acc[i] = S(0);
-    int2 blk = int2{0, 0};  // first source and count of this lane's block
-    auto block_of = [&](int q) {
-      return q + group < q1 ? d.blk8_src[d.nbr_blk[q + group]] : int2{0, 0};
-    };
-    if (q0 < q1) blk = block_of(q0);
-    for (int q = q0; q < q1; q += 8) {
-      // A lane without a source takes one out of reach with no moment: its
-      // |r|^-1 is tiny and every term of it zero.
-      const bool have = e < blk.y;
-      const int s = have ? blk.x + e : -2;
-      Point<S> sp;
-      S m[3][KS];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        sp.h[c] = Point<S>::far();
-        if constexpr (sizeof(S) == 4) sp.l[c] = S(0);
-#pragma unroll
-        for (int k = 0; k < KS; ++k) m[c][k] = S(0);
-      }
-      if (have) {
-        sp = Point<S>::load(d.src_pos, d.ns, s);
-        const S* ms = sm + int64_t(s) * 3 * K + k0;
-        if (KS == K) {  // one contiguous row
-          const auto row = *reinterpret_cast<const States<S, 3 * KS>*>(ms);
-#pragma unroll
-          for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int k = 0; k < KS; ++k) m[c][k] = row.v[c * KS + k];
-        } else {
-#pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            const auto row = *reinterpret_cast<const States<S, KS>*>(ms + c * K);
-#pragma unroll
-            for (int k = 0; k < KS; ++k) m[c][k] = row.v[k];
-          }
+        for (int k = 0; k < KS; ++k) {
+          const S mx = m[0][k], my = m[1][k], mz = m[2][k];
+          const S w = ux * mx + uy * my + uz * mz;
+          const S w5 = S(5) * w;
+          a[0 * KS + k] += g * (w + S(2) * ux * mx - w5 * ux * ux);
+          a[1 * KS + k] += g * (ux * my + mx * uy - w5 * ux * uy);
+          a[2 * KS + k] += g * (ux * mz + mx * uz - w5 * ux * uz);
+          a[3 * KS + k] += g * (w + S(2) * uy * my - w5 * uy * uy);
+          a[4 * KS + k] += g * (uy * mz + my * uz - w5 * uy * uz);
+          a[5 * KS + k] += g * (w + S(2) * uz * mz - w5 * uz * uz);
         }
-      }
-      if (q + 8 < q1) blk = block_of(q + 8);
+      } else {
+        // f (3 (u.m) u - m) with f = |r|^-3 / (4 pi) avoids the |r|^-5
+        // overflow of close pairs in FP32.
+        const S f = rinv * rinv * rinv * S(0.079577471545947667884441881686257181);
 #pragma unroll
-      for (int i = 0; i < T; ++i) {
-        if (i >= cnt || s == self[i]) continue;
-        const S rx = tp[i].minus(sp, 0), ry = tp[i].minus(sp, 1), rz = tp[i].minus(sp, 2);
-        const S r2 = rx * rx + ry * ry + rz * rz;
-        const S rinv = near_rsqrt(r2);
-        const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
-        S* a = acc + i * C * KS;
-        if constexpr (kWhat == kGradient) {
-          // dH_c/dx_j, 3/(4 pi |r|^4) (delta_cj w + u_c m_j + m_c u_j - 5 u_c u_j w), w = u.m.
-          const S g = S(0.23873241463784300365332564505877154) * rinv * rinv * rinv * rinv;
-#pragma unroll
-          for (int k = 0; k < KS; ++k) {
-            const S mx = m[0][k], my = m[1][k], mz = m[2][k];
-            const S w = ux * mx + uy * my + uz * mz;
-            const S w5 = S(5) * w;
-            a[0 * KS + k] += g * (w + S(2) * ux * mx - w5 * ux * ux);
-            a[1 * KS + k] += g * (ux * my + mx * uy - w5 * ux * uy);
-            a[2 * KS + k] += g * (ux * mz + mx * uz - w5 * ux * uz);
-            a[3 * KS + k] += g * (w + S(2) * uy * my - w5 * uy * uy);
-            a[4 * KS + k] += g * (uy * mz + my * uz - w5 * uy * uz);
-            a[5 * KS + k] += g * (w + S(2) * uz * mz - w5 * uz * uz);
-          }
-        } else {
-          // f (3 (u.m) u - m) with f = |r|^-3 / (4 pi) avoids the |r|^-5
-          // overflow of close pairs in FP32.
-          const S f = rinv * rinv * rinv * S(0.079577471545947667884441881686257181);
-#pragma unroll
-          for (int k = 0; k < KS; ++k) {
-            const S mx = m[0][k], my = m[1][k], mz = m[2][k];
-            const S w = ux * mx + uy * my + uz * mz, w3 = S(3) * w;
-            a[0 * KS + k] += f * (w3 * ux - mx);
-            a[1 * KS + k] += f * (w3 * uy - my);
-            a[2 * KS + k] += f * (w3 * uz - mz);
-            if constexpr (kWhat == kFieldAndPotential)
-              a[3 * KS + k] += f * (rx * mx + ry * my + rz * mz);
-          }
+        for (int k = 0; k < KS; ++k) {
+          const S mx = m[0][k], my = m[1][k], mz = m[2][k];
+          const S w = ux * mx + uy * my + uz * mz, w3 = S(3) * w;
+          a[0 * KS + k] += f * (w3 * ux - mx);
+          a[1 * KS + k] += f * (w3 * uy - my);
+          a[2 * KS + k] += f * (w3 * uz - mz);
+          if constexpr (kWhat == kFieldAndPotential)
+            a[3 * KS + k] += f * (rx * mx + ry * my + rz * mz);
         }
       }
     }
-    int first = 0;
-    wave_totals<V, 32>(acc, lane, first);
+  }
+  int first = 0;
+  wave_totals<V, 32>(acc, lane, first);
 #pragma unroll
-    for (int v = 0; v < totals_left(V); ++v) {
-      const int at = first + v, i = at / (C * KS), c = at / KS % C, k = k0 + at % KS;
-      if (i >= cnt || k < k_first) continue;
-      const int64_t t = t0 + i;
-      if constexpr (kWhat == kGradient)
-        static_cast<S*>(d.Gn)[(t * 6 + c) * K + k] = acc[v];
-      else if (c < 3)
-        static_cast<S*>(d.Hn)[(t * 3 + c) * K + k] = acc[v];
-      else
-        static_cast<S*>(d.Pn)[t * K + k] = acc[v];
-    }
+  for (int v = 0; v < totals_left(V); ++v) {
+    const int at = first + v, i = at / (C * KS), c = at / KS % C, k = k0 + at % KS;
+    if (i >= cnt || k < k_first) continue;
+    const int64_t t = t0 + i;
+    if constexpr (kWhat == kGradient)
+      static_cast<S*>(d.Gn)[(t * 6 + c) * K + k] = acc[v];
+    else if (c < 3)
+      static_cast<S*>(d.Hn)[(t * 3 + c) * K + k] = acc[v];
+    else
+      static_cast<S*>(d.Pn)[t * K + k] = acc[v];
   }
 }
 
@@ -261,8 +272,11 @@ void launch_near(const DevicePlan& d, int K, hipStream_t s) {
   const int parts = (K + most - 1) / most, ks = (K + parts - 1) / parts;
   auto go = [&](auto count) {
     constexpr int KS = decltype(count)::value;
-    if constexpr (KS <= most)
-      near_lanes_kernel<S, KS, kWhat><<<dim3(unsigned(d.leaves), unsigned(parts)), 64 * kWaves, 0, s>>>(d, K);
+    if constexpr (KS <= most) {
+      const int64_t items = int64_t(d.p2p_tile16_count) * (16 / near_targets<S>(KS, kWhat));
+      const dim3 grid(unsigned((items + kWaves - 1) / kWaves), unsigned(parts));
+      if (items > 0) near_lanes_kernel<S, KS, kWhat><<<grid, 64 * kWaves, 0, s>>>(d, K);
+    }
   };
   switch (ks) {
     case 1: go(std::integral_constant<int, 1>{}); break;
