@@ -15,6 +15,8 @@
 #include "common.hpp"
 #include "bf16_split.hpp"
 
+#include <type_traits>
+
 namespace hipfmm {
 
 namespace {
@@ -389,21 +391,22 @@ __global__ void __launch_bounds__(64 * kP2PWaves) p2p_mfma16_kernel(const Device
 // The sorted moments as B operands of p2p_bf16_kernel: per block of 8
 // sources of one leaf and tile of 32 states,
 // smb[block][state tile][c'][piece][32][8] (pieces hi, mid, lo of
-// m[s][c'][k]), zero past the leaf's last source; a wave's 18 operand loads
-// of one block then sit at fixed offsets from one address.  Thread = (block,
-// state); reads are coalesced over the states, writes are 16-byte rows.
-__global__ void __launch_bounds__(256) split_moments_kernel(const DevicePlan d, int K) {
+// m[s][c'][k]), zero past the leaf's last source and past the last state; a
+// wave's 18 operand loads of one block then sit at fixed offsets from one
+// address.  Thread = (block, state of the KP = 32-padded tiles); reads are
+// coalesced over the states, writes are 16-byte rows.
+__global__ void __launch_bounds__(256) split_moments_kernel(const DevicePlan d, int K, int KP) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= int64_t(d.blk8_count) * K) return;
-  const int b = int(i / K), k = int(i % K);
+  if (i >= int64_t(d.blk8_count) * KP) return;
+  const int b = int(i / KP), k = int(i % KP);
   const int2 bs = d.blk8_src[b];
   const float* sm = static_cast<const float*>(d.sm);
-  uint4* out = static_cast<uint4*>(d.smb) + ((int64_t(b) * (K / 32) + k / 32) * 9) * 32 + k % 32;
+  uint4* out = static_cast<uint4*>(d.smb) + ((int64_t(b) * (KP / 32) + k / 32) * 9) * 32 + k % 32;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = e < bs.y ? sm[(int64_t(bs.x + e) * 3 + c) * K + k] : 0.0f;
+    for (int e = 0; e < 8; ++e) x[e] = e < bs.y && k < K ? sm[(int64_t(bs.x + e) * 3 + c) * K + k] : 0.0f;
     uint4 h, m, l;
     split3_bf16(x, h, m, l);
     out[(3 * c) * 32] = h;
@@ -412,24 +415,92 @@ __global__ void __launch_bounds__(256) split_moments_kernel(const DevicePlan d, 
   }
 }
 
-// part[h] += D_ab m_b for both 16-state halves from the pieces of D_ab (A
+// part[h] += D_ab m_b for the kH 16-state halves from the pieces of D_ab (A
 // operands) and of m_b (B operands): the six products of pieces whose orders
-// sum to at most 2, smallest first.
-__device__ __forceinline__ void p2p_bf16_products(f32x4 (&part)[2], const uint4& ah, const uint4& am, const uint4& al,
-                                                  const uint4 (&b)[3][2]) {
-  // The two halves' chains alternate, so consecutive products are independent.
+// sum to at most 2, smallest first.  The halves' chains alternate, so that
+// consecutive products are independent.
+template <int kH>
+__device__ __forceinline__ void p2p_bf16_products(f32x4 (&part)[kH], const uint4& ah, const uint4& am, const uint4& al,
+                                                  const uint4 (&b)[3][kH]) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(am, b[1][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(am, b[1][h], part[h]);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(al, b[0][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(al, b[0][h], part[h]);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(ah, b[2][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(ah, b[2][h], part[h]);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(am, b[0][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(am, b[0][h], part[h]);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(ah, b[1][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(ah, b[1][h], part[h]);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) part[h] = mfma_bf16(ah, b[0][h], part[h]);
+  for (int h = 0; h < kH; ++h) part[h] = mfma_bf16(ah, b[0][h], part[h]);
+}
+
+// A tile's sums in batches that are no multiple of 32 states, where one of
+// them is not finite (rare): those of that lane's target and state again, one
+// pair at a time.  In the products a source that is left out (a target's own,
+// a padding slot) has weight zero, and zero times a moment that is not finite
+// is NaN; here it is left out.  kRows: 3 the field, 4 with the potential, 6 the
+// gradient; acc[c][h][i] is row c of state k0 + 16 h, target t0 + i.
+template <int kRows, int kH>
+__device__ __forceinline__ void p2p_repair(const DevicePlan& d, f32x4 (&acc)[kRows][kH], int leaf, int t0, int cnt,
+                                           int k0, int K) {
+  bool bad = false;
+#pragma unroll
+  for (int c = 0; c < kRows; ++c)
+#pragma unroll
+    for (int h = 0; h < kH; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bad |= !__builtin_isfinite(acc[c][h][i]);
+  if (__any(bad) == 0) return;
+  const int q0 = d.nbr_blk_start[leaf], q1 = d.nbr_blk_start[leaf + 1];
+  const float* sm = static_cast<const float*>(d.sm);
+#pragma unroll 1
+  for (int j = 0; j < 4 * kH; ++j) {
+    const int h = j >> 2, i = j & 3, k = k0 + 16 * h;
+    if (i >= cnt || k >= K) continue;
+    const int t = t0 + i, self = d.self[t];
+    const PairPos<float> tp = PairPos<float>::load(d.tgt_pos, d.nt, t);
+    float sum[kRows];
+#pragma unroll
+    for (int c = 0; c < kRows; ++c) sum[c] = 0.0f;
+#pragma unroll 1
+    for (int q = q0; q < q1; ++q) {
+      const int2 bs = d.blk8_src[d.nbr_blk[q]];
+#pragma unroll 1
+      for (int s = bs.x; s < bs.x + bs.y; ++s) {
+        if (s == self) continue;
+        float rx, ry, rz;
+        tp.diff(PairPos<float>::load(d.src_pos, d.ns, s), rx, ry, rz);
+        const float rinv = __builtin_amdgcn_rsqf(rx * rx + ry * ry + rz * rz);
+        const float ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
+        const float* ms = sm + int64_t(s) * 3 * K + k;
+        const float mx = ms[0], my = ms[K], mz = ms[2 * K], w = ux * mx + uy * my + uz * mz;
+        if constexpr (kRows == 6) {
+          const float g = 0.23873241463784300365332564505877154f * rinv * rinv * rinv * rinv, w5 = 5.0f * w;
+          sum[0] += g * (w + 2.0f * ux * mx - w5 * ux * ux);
+          sum[1] += g * (ux * my + mx * uy - w5 * ux * uy);
+          sum[2] += g * (ux * mz + mx * uz - w5 * ux * uz);
+          sum[3] += g * (w + 2.0f * uy * my - w5 * uy * uy);
+          sum[4] += g * (uy * mz + my * uz - w5 * uy * uz);
+          sum[5] += g * (w + 2.0f * uz * mz - w5 * uz * uz);
+        } else {
+          const float f = rinv * rinv * rinv * 0.079577471545947667884441881686257181f;
+          sum[0] += f * (3.0f * w * ux - mx);
+          sum[1] += f * (3.0f * w * uy - my);
+          sum[2] += f * (3.0f * w * uz - mz);
+          if constexpr (kRows == 4) sum[3] += f * (rx * mx + ry * my + rz * mz);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kRows; ++c)
+#pragma unroll
+      for (int hh = 0; hh < kH; ++hh)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii)
+          if (4 * hh + ii == j && !__builtin_isfinite(acc[c][hh][ii])) acc[c][hh][ii] = sum[c];
+  }
 }
 
 // List-1 P2P on the matrix cores with bf16 operands
@@ -459,10 +530,13 @@ __device__ __forceinline__ void p2p_bf16_products(f32x4 (&part)[2], const uint4&
 //
 // Fields are capped at 168 registers, three waves per SIMD (4.7 ms at 1M
 // points, p = 8, depth 5, K = 32, against 7.4 ms for the FP32 kernel); the
-// potential form runs at two, where the cap would spill.
-template <bool kPot>
-__global__ void __launch_bounds__(64 * kP2PWaves) __attribute__((amdgpu_waves_per_eu(kPot ? 2 : 3)))
-p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_count, int K) {
+// potential form runs at two, where the cap would spill; with one half of
+// states (kH = 1) each has one more.
+// kH: 16-state halves of a state tile (one where at most 16 states are left);
+// tile0: its first state tile; kRagged: K is no multiple of 32.
+template <bool kPot, int kH, bool kRagged>
+__global__ void __launch_bounds__(64 * kP2PWaves) __attribute__((amdgpu_waves_per_eu(kPot ? (kH == 1 ? 3 : 2) : (kH == 1 ? 4 : 3))))
+p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_count, int K, int tile0) {
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int item = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x)) * kP2PWaves + wave;
   if (item >= tile_count) return;
@@ -474,14 +548,14 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
   const int t = row_ok ? trange.x + tile.y + col : trange.x;
   const PairPos<float> tp = PairPos<float>::load(d.tgt_pos, d.nt, t);
   const int self = row_ok ? d.self[t] : -2;
-  const int kc0 = int(blockIdx.y) * 32;
+  const int kc0 = (tile0 + int(blockIdx.y)) * 32, KT = (K + 31) / 32;
   const uint4* mb = static_cast<const uint4*>(d.smb);
   constexpr int kRows = kPot ? 4 : 3;  // field components, then the potential
-  f32x4 acc[kRows][2];
+  f32x4 acc[kRows][kH];
 #pragma unroll
   for (int c = 0; c < kRows; ++c)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) acc[c][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int h = 0; h < kH; ++h) acc[c][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   // The neighbourhood's 8-source blocks in one list, four per product (one
   // per lane group): a leaf pads to 8 sources rather than to 32.
   const int q0 = d.nbr_blk_start[leaf], q1 = d.nbr_blk_start[leaf + 1];
@@ -492,14 +566,14 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
     const int blk = d.nbr_blk[grp_ok ? q + g : q];
     const int2 bs = d.blk8_src[blk];
     const int cnt = grp_ok ? bs.y : 0;
-    const uint4* bp = mb + ((int64_t(blk) * (K / 32) + (kc0 >> 5)) * 9) * 32 + col;
-    uint4 b[3][3][2];  // [component][piece][state half]
+    const uint4* bp = mb + ((int64_t(blk) * KT + (kc0 >> 5)) * 9) * 32 + col;
+    uint4 b[3][3][kH];  // [component][piece][state half]
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int pc = 0; pc < 3; ++pc)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) b[c][pc][h] = bp[(3 * c + pc) * 32 + 16 * h];
+        for (int h = 0; h < kH; ++h) b[c][pc][h] = bp[(3 * c + pc) * 32 + 16 * h];
     float r[3][8], f[8], gf[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -513,11 +587,11 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
       f[e] = ri2 * rinv * 0.079577471545947667884441881686257181f;
       gf[e] = 3.0f * f[e] * ri2;
     }
-    f32x4 part[kRows][2];
+    f32x4 part[kRows][kH];
 #pragma unroll
     for (int c = 0; c < kRows; ++c)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) part[c][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int h = 0; h < kH; ++h) part[c][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -527,10 +601,18 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
         for (int e = 0; e < 8; ++e) v[e] = gf[e] * r[a][e] * r[bc][e] - (a == bc ? f[e] : 0.0f);
         uint4 ph, pm, pl;
         split3_bf16(v, ph, pm, pl);
-        const uint4 bb[3][2] = {{b[bc][0][0], b[bc][0][1]}, {b[bc][1][0], b[bc][1][1]}, {b[bc][2][0], b[bc][2][1]}};
+        uint4 bb[3][kH];
+#pragma unroll
+        for (int pc = 0; pc < 3; ++pc)
+#pragma unroll
+          for (int h = 0; h < kH; ++h) bb[pc][h] = b[bc][pc][h];
         p2p_bf16_products(part[a], ph, pm, pl, bb);
         if (a != bc) {
-          const uint4 ba[3][2] = {{b[a][0][0], b[a][0][1]}, {b[a][1][0], b[a][1][1]}, {b[a][2][0], b[a][2][1]}};
+          uint4 ba[3][kH];
+#pragma unroll
+          for (int pc = 0; pc < 3; ++pc)
+#pragma unroll
+            for (int h = 0; h < kH; ++h) ba[pc][h] = b[a][pc][h];
           p2p_bf16_products(part[bc], ph, pm, pl, ba);
         }
       }
@@ -543,24 +625,33 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
         for (int e = 0; e < 8; ++e) v[e] = f[e] * r[cp][e];
         uint4 ph, pm, pl;
         split3_bf16(v, ph, pm, pl);
-        const uint4 bb[3][2] = {{b[cp][0][0], b[cp][0][1]}, {b[cp][1][0], b[cp][1][1]}, {b[cp][2][0], b[cp][2][1]}};
+        uint4 bb[3][kH];
+#pragma unroll
+        for (int pc = 0; pc < 3; ++pc)
+#pragma unroll
+          for (int h = 0; h < kH; ++h) bb[pc][h] = b[cp][pc][h];
         p2p_bf16_products(part[3], ph, pm, pl, bb);
       }
     }
 #pragma unroll
     for (int c = 0; c < kRows; ++c)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) acc[c][h] += part[c][h];
+      for (int h = 0; h < kH; ++h) acc[c][h] += part[c][h];
   }
   // acc[c][h][i]: target tile.y + 4g + i, state kc0 + 16h + col.
+  if constexpr (kRagged) {
+    const int t0 = trange.x + tile.y + 4 * g;
+    p2p_repair<kRows, kH>(d, acc, leaf, t0, trange.y - t0, kc0 + col, K);
+  }
   float* Hn = static_cast<float*>(d.Hn);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int64_t ot = int64_t(trange.x) + tile.y + 4 * g + i;
     if (ot >= trange.y) continue;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kH; ++h) {
       const int k = kc0 + 16 * h + col;
+      if (kRagged && k >= K) continue;
 #pragma unroll
       for (int c = 0; c < 3; ++c) Hn[(ot * 3 + c) * K + k] = acc[c][h][i];
       if constexpr (kPot) static_cast<float*>(d.Pn)[ot * K + k] = acc[3][h][i];
@@ -568,13 +659,38 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
   }
 }
 
+// Batches that are no multiple of 32 take the bf16 kernels from the state count
+// at which a whole 32-state (or 16-state) tile costs less than the vector ALUs'
+// pass per group of states (the near-field variants choose among the kernels of
+// the multiples of 32).  Near field alone, ms, vector ALUs / bf16 tiles:
+//   fields, 2^20 points, 32 per leaf: K = 8 3.06 / 3.39, 9 4.45 / 3.38,
+//     16 6.44 / 3.58, 31 13.7 / 5.1; 512 per leaf, 2^18 points: K = 8 6.5 / 7.5,
+//     9 10.4 / 7.6; 20,000 points: K = 8 .074 / .123, 9 .097 / .124;
+//   fields and potentials, 2^20 points: K = 8 4.07 / 4.12, 9 5.24 / 4.1;
+//   gradients, 2^20 points: K = 6 5.6 / 5.2, 7 6.85 / 5.3; 20,000 points:
+//     K = 6 .114 / .17, 8 .139 / .17.
+static bool near_on_matrix_cores(int K, bool gradient) {
+  return K >= (gradient ? kNearGradBf16States : kNearBf16States);
+}
+
 // The moments' bf16 pieces for the near-field kernels on bf16 operands.
 void launch_split_moments(const DevicePlan& d, int K, hipStream_t s) {
   if (d.smb == nullptr || d.smb_blocks < d.blk8_count)
     throw invalid_argument("bf16 near-field moment buffer is not allocated");
   if (d.blk8_count == 0) return;  // without sources the near-field kernels write zeros
-  const int64_t threads = int64_t(d.blk8_count) * K;
-  split_moments_kernel<<<unsigned((threads + 255) / 256), 256, 0, s>>>(d, K);
+  const int KP = (K + 31) / 32 * 32;
+  const int64_t threads = int64_t(d.blk8_count) * KP;
+  split_moments_kernel<<<unsigned((threads + 255) / 256), 256, 0, s>>>(d, K, KP);
+  HIPFMM_CHECK(hipGetLastError());
+}
+
+// State tiles of 32, and a last one of 16 where at most 16 states are left:
+// launch(halves, first tile, tiles).
+template <class F>
+void for_state_tiles(int K, F&& launch) {
+  const int rest = K % 32, whole = K / 32 + (rest > 16 ? 1 : 0);
+  if (whole > 0) launch(std::integral_constant<int, 2>{}, 0, whole);
+  if (rest > 0 && rest <= 16) launch(std::integral_constant<int, 1>{}, K / 32, 1);
   HIPFMM_CHECK(hipGetLastError());
 }
 
@@ -582,12 +698,21 @@ void launch_p2p_bf16(const DevicePlan& d, int K, bool potential, hipStream_t s) 
   const int count = d.p2p_tile16_count;
   if (count == 0) return;
   launch_split_moments(d, K, s);
-  const dim3 grid(unsigned((count + kP2PWaves - 1) / kP2PWaves), unsigned(K / 32));
-  if (potential)
-    p2p_bf16_kernel<true><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K);
-  else
-    p2p_bf16_kernel<false><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K);
-  HIPFMM_CHECK(hipGetLastError());
+  const bool ragged = K % 32 != 0;
+  for_state_tiles(K, [&](auto halves, int tile0, int tiles) {
+    constexpr int H = decltype(halves)::value;
+    const dim3 grid(unsigned((count + kP2PWaves - 1) / kP2PWaves), unsigned(tiles));
+    if (potential && ragged)
+      p2p_bf16_kernel<true, H, true><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+    else if (ragged)
+      p2p_bf16_kernel<false, H, true><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+    else if constexpr (H == 2) {
+      if (potential)
+        p2p_bf16_kernel<true, 2, false><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+      else
+        p2p_bf16_kernel<false, 2, false><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+    }
+  });
 }
 
 template <class S>
@@ -595,7 +720,7 @@ void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s) {
   if (d.leaves == 0 || d.nt == 0) return;
   if (potential && d.Pn == nullptr) throw invalid_argument("near-field potential buffer is not allocated");
   if constexpr (sizeof(S) == 4) {
-    if (K % 32 == 0 && (d.p2p_variant == 4 || d.p2p_variant == 0)) {
+    if (K % 32 == 0 ? d.p2p_variant == 4 || d.p2p_variant == 0 : near_on_matrix_cores(K, false)) {
       launch_p2p_bf16(d, K, potential, s);
       return;
     }
@@ -629,11 +754,10 @@ template void launch_p2p<double>(const DevicePlan&, int, bool, hipStream_t);
 
 // acc[E] += W m_D over both state halves, for one entry of W (its pieces)
 // and the moments' component D.
-template <int E, int D>
-__device__ __forceinline__ void grad_bf16_products(f32x4 (&acc)[6][2], const uint4& ph, const uint4& pm,
-                                                   const uint4& pl, const uint4 (&b)[3][3][2]) {
-  const uint4 bb[3][2] = {{b[D][0][0], b[D][0][1]}, {b[D][1][0], b[D][1][1]}, {b[D][2][0], b[D][2][1]}};
-  p2p_bf16_products(acc[E], ph, pm, pl, bb);
+template <int E, int D, int kH>
+__device__ __forceinline__ void grad_bf16_products(f32x4 (&acc)[6][kH], const uint4& ph, const uint4& pm,
+                                                   const uint4& pl, const uint4 (&b)[3][3][kH]) {
+  p2p_bf16_products(acc[E], ph, pm, pl, b[D]);
 }
 
 // Near-field gradient on bf16 three-piece operands (FP32 plans, K a multiple
@@ -646,8 +770,9 @@ __device__ __forceinline__ void grad_bf16_products(f32x4 (&acc)[6][2], const uin
 // accumulation straight into the totals, as in the FP32 gradient kernel.
 // Padding pairs and the identity pair have |r|^-1 = 0; coincident pairs give
 // NaN.  Writes Gn[t][6][K] (xx xy xz yy yz zz).
+template <int kH, bool kRagged>
 __global__ void __launch_bounds__(64 * kP2PWaves) __attribute__((amdgpu_waves_per_eu(2)))
-p2p_grad_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_count, int K) {
+p2p_grad_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_count, int K, int tile0) {
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int item = xcd_contiguous_block(int(blockIdx.x), int(gridDim.x)) * kP2PWaves + wave;
   if (item >= tile_count) return;
@@ -659,11 +784,13 @@ p2p_grad_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int til
   const int t = row_ok ? trange.x + tile.y + col : trange.x;
   const PairPos<float> tp = PairPos<float>::load(d.tgt_pos, d.nt, t);
   const int self = row_ok ? d.self[t] : -2;
-  const int kc0 = int(blockIdx.y) * 32;
+  const int kc0 = (tile0 + int(blockIdx.y)) * 32, KT = (K + 31) / 32;
   const uint4* mb = static_cast<const uint4*>(d.smb);
-  f32x4 acc[6][2];
+  f32x4 acc[6][kH];
 #pragma unroll
-  for (int e = 0; e < 6; ++e) acc[e][0] = acc[e][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int e = 0; e < 6; ++e)
+#pragma unroll
+    for (int h = 0; h < kH; ++h) acc[e][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const float c34pi = 0.23873241463784300365332564505877154f;  // 3/(4 pi)
   const int q0 = d.nbr_blk_start[leaf], q1 = d.nbr_blk_start[leaf + 1];
   const float4* shi = static_cast<const float4*>(d.src_pos);
@@ -673,14 +800,14 @@ p2p_grad_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int til
     const int blk = d.nbr_blk[grp_ok ? q + g : q];
     const int2 bs = d.blk8_src[blk];
     const int cnt = grp_ok ? bs.y : 0;
-    const uint4* bp = mb + ((int64_t(blk) * (K / 32) + (kc0 >> 5)) * 9) * 32 + col;
-    uint4 b[3][3][2];  // [component][piece][state half]
+    const uint4* bp = mb + ((int64_t(blk) * KT + (kc0 >> 5)) * 9) * 32 + col;
+    uint4 b[3][3][kH];  // [component][piece][state half]
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int pc = 0; pc < 3; ++pc)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) b[c][pc][h] = bp[(3 * c + pc) * 32 + 16 * h];
+        for (int h = 0; h < kH; ++h) b[c][pc][h] = bp[(3 * c + pc) * 32 + 16 * h];
     float ux[8], uy[8], uz[8], gg[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -750,15 +877,22 @@ p2p_grad_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int til
     grad_bf16_products<5, 2>(acc, ph, pm, pl, b);
   }
   // acc[e][h][i]: target tile.y + 4g + i, state kc0 + 16h + col.
+  if constexpr (kRagged) {
+    const int t0 = trange.x + tile.y + 4 * g;
+    p2p_repair<6, kH>(d, acc, leaf, t0, trange.y - t0, kc0 + col, K);
+  }
   float* Gn = static_cast<float*>(d.Gn);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int64_t ot = int64_t(trange.x) + tile.y + 4 * g + i;
     if (ot >= trange.y) continue;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < kH; ++h) {
+      const int k = kc0 + 16 * h + col;
+      if (kRagged && k >= K) continue;
 #pragma unroll
-      for (int e = 0; e < 6; ++e) Gn[(ot * 6 + e) * K + kc0 + 16 * h + col] = acc[e][h][i];
+      for (int e = 0; e < 6; ++e) Gn[(ot * 6 + e) * K + k] = acc[e][h][i];
+    }
   }
 }
 
@@ -858,14 +992,22 @@ void launch_p2p_grad(const DevicePlan& d, int K, hipStream_t s) {
   if (d.leaves == 0 || d.nt == 0) return;
   if (d.Gn == nullptr) throw invalid_argument("near-field gradient buffer is not allocated");
   if constexpr (sizeof(S) == 4) {
-    if (K % 32 == 0 && d.p2p_tile16_count > 0) {
-      const dim3 grid(unsigned((d.p2p_tile16_count + kP2PWaves - 1) / kP2PWaves), unsigned(K / 32));
-      if (d.p2p_variant == 0 || d.p2p_variant == 4) {
-        launch_split_moments(d, K, s);
-        p2p_grad_bf16_kernel<<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, d.p2p_tile16_count, K);
-      } else {
-        p2p_grad_mfma16_kernel<<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, d.p2p_tile16_count, K);
-      }
+    const int count = d.p2p_tile16_count;
+    const unsigned blocks = unsigned((count + kP2PWaves - 1) / kP2PWaves);
+    if (count > 0 && (K % 32 == 0 ? d.p2p_variant == 0 || d.p2p_variant == 4 : near_on_matrix_cores(K, true))) {
+      launch_split_moments(d, K, s);
+      for_state_tiles(K, [&](auto halves, int tile0, int tiles) {
+        constexpr int H = decltype(halves)::value;
+        const dim3 grid(blocks, unsigned(tiles));
+        if (K % 32 != 0)
+          p2p_grad_bf16_kernel<H, true><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+        else if constexpr (H == 2)
+          p2p_grad_bf16_kernel<2, false><<<grid, 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K, tile0);
+      });
+      return;
+    }
+    if (count > 0 && K % 32 == 0) {
+      p2p_grad_mfma16_kernel<<<dim3(blocks, unsigned(K / 32)), 64 * kP2PWaves, 0, s>>>(d, d.p2p_tiles16, count, K);
       HIPFMM_CHECK(hipGetLastError());
       return;
     }

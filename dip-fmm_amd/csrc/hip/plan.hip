@@ -821,9 +821,9 @@ void ensure_capacity(hipfmm_plan* P, int K, bool potential, bool gradient = fals
   d.Hn = alloc(points * 3 * cap, sizeof(S));
   d.smb = nullptr;
   d.smb_blocks = 0;
-  if (sizeof(S) == 4 && cap >= 32) {  // bf16 moments for K a multiple of 32 up to cap
+  if (sizeof(S) == 4 && cap >= hipfmm::kNearGradBf16States) {  // bf16 moments in tiles of 32 states
     d.smb_blocks = std::max({d.blk8_count, P->adj_blk8_count, 1});
-    d.smb = alloc(size_t(d.smb_blocks) * 9 * 8 * (cap / 32 * 32), 2);
+    d.smb = alloc(size_t(d.smb_blocks) * 9 * 8 * ((cap + 31) / 32 * 32), 2);
   }
   d.Pn = nullptr;
   d.potentials_out = nullptr;
