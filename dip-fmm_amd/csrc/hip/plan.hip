@@ -55,13 +55,10 @@ enum Ev {
   kEvM2L,
   kEvL2L,
   kEvL2P,
-  kEvNear0,
+  kEvCaptured,
   kEvNear1,
   kEvD2H0,
   kEvD2H1,
-  kEvUser,
-  kEvM2LKernel0,
-  kEvM2LKernel1,
   kEvCount
 };
 
@@ -72,7 +69,10 @@ struct hipfmm_plan {
   int device = 0;
   std::vector<void*> persistent;
   std::vector<void*> state;
-  hipStream_t s_far = nullptr, s_near = nullptr;
+  hipStream_t s_far = nullptr, s_near = nullptr;  // s_far: see far_stream
+  bool done_recorded = false;         // ev[kEvL2P] marks the end of the last evaluate outside a capture
+  int last_done = 0;                  // event at the end of the last evaluate
+  unsigned long long capture_id = 0;  // of the last captured evaluate, which ends at ev[kEvCaptured]
   hipEvent_t ev[kEvCount] = {};
   void* pinned_in = nullptr;
   void* pinned_out = nullptr;
@@ -110,6 +110,8 @@ struct hipfmm_plan {
   static constexpr int kRing = 64;
   hipEvent_t m2l_ring[kRing][2] = {};
   bool m2l_ring_pending[kRing] = {};
+  int last_ring_slot = 0;         // of the last evaluate
+  bool last_m2l_expands = false;  // its M2L ends at kEvM2L, after its kernel
   uint64_t m2l_launch_count = 0;
   double m2l_total_seconds = 0.0;
   uint64_t m2l_total_launches = 0;
@@ -381,7 +383,7 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   // (lists.hip), on the far stream; each builder returns once its arrays
   // are complete.
   const auto index_t0 = std::chrono::steady_clock::now();
-  const hipStream_t sb = P->s_far;
+  const hipStream_t sb = P->s_near;
   const hipfmm::DeviceAllocator persistent = [P](size_t bytes) {
     return device_alloc(P, bytes, P->persistent, P->persistent_bytes);
   };
@@ -792,20 +794,32 @@ void free_state(hipfmm_plan* P) {
   P->d.kcap = 0;
 }
 
+// Earlier evaluates may still be running on the callers' and the plan's streams.
+void wait_for_evaluates(hipfmm_plan* P) {
+  if (P->done_recorded) HIPFMM_CHECK(hipEventSynchronize(P->ev[kEvL2P]));
+  if (P->s_far) HIPFMM_CHECK(hipStreamSynchronize(P->s_far));
+  HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
+}
+
+// The plan's own stream of the far field, for evaluates without a stream of
+// the caller's: created with the first of them, since streams share the
+// process's few hardware queues.
+hipStream_t far_stream(hipfmm_plan* P) {
+  if (!P->s_far) HIPFMM_CHECK(hipStreamCreateWithFlags(&P->s_far, hipStreamNonBlocking));
+  return P->s_far;
+}
+
 template <class S>
 void ensure_capacity(hipfmm_plan* P, int K, bool potential, bool gradient = false) {
   DevicePlan& d = P->d;
   if ((potential && !P->potential_used) || (gradient && !P->gradient_used)) {
     P->potential_used = P->potential_used || potential;
     P->gradient_used = P->gradient_used || gradient;
-    HIPFMM_CHECK(hipStreamSynchronize(P->s_far));
-    HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
+    wait_for_evaluates(P);
     free_state(P);  // reallocated below with the extra buffers
   }
   if (K <= d.kcap) return;
-  // Earlier evaluates may still be running on the plan's streams.
-  HIPFMM_CHECK(hipStreamSynchronize(P->s_far));
-  HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
+  wait_for_evaluates(P);
   free_state(P);
   const int cap = std::min(hipfmm::kMaxBatch, std::max(K, 1));
   const size_t cs = size_t(d.nodes) * d.n * cap;
@@ -886,17 +900,24 @@ void finalize_timings(hipfmm_plan* P) {
   if (P->last_host) HIPFMM_CHECK(hipEventSynchronize(P->ev[kEvD2H1]));
   hipfmm_timings& t = P->timings;
   hipEvent_t* e = P->ev;
-  t.h2d_seconds = 1e-3 * elapsed(e[kEvH2D0], e[kEvH2D1]);
-  t.p2m_seconds = 1e-3 * elapsed(e[kEvH2D1], e[kEvP2M]);
+  // A record between two kernels costs about 6 us, so no point of the stream
+  // has two: without a copy the kernels start where the call does, the near
+  // field starts at the gather's end, and the M2L ends with its kernel unless
+  // an expansion follows.
+  const hipEvent_t kernels0 = P->last_host ? e[kEvH2D1] : e[kEvH2D0];
+  const hipEvent_t* m2l_kernel = P->m2l_ring[P->last_ring_slot];
+  const hipEvent_t m2l_end = P->last_m2l_expands ? e[kEvM2L] : m2l_kernel[1];
+  t.h2d_seconds = P->last_host ? 1e-3 * elapsed(e[kEvH2D0], e[kEvH2D1]) : 0.0;
+  t.p2m_seconds = 1e-3 * elapsed(kernels0, e[kEvP2M]);
   t.m2m_seconds = 1e-3 * elapsed(e[kEvP2M], e[kEvM2M]);
-  t.m2l_seconds = 1e-3 * elapsed(e[kEvM2M], e[kEvM2L]);
-  t.l2l_seconds = 1e-3 * elapsed(e[kEvM2L], e[kEvL2L]);
+  t.m2l_seconds = 1e-3 * elapsed(e[kEvM2M], m2l_end);
+  t.l2l_seconds = 1e-3 * elapsed(m2l_end, e[kEvL2L]);
   t.l2p_seconds = 1e-3 * elapsed(e[kEvL2L], e[kEvL2P]);
-  t.p2p_seconds = 1e-3 * elapsed(e[kEvNear0], e[kEvNear1]);
-  t.kernel_seconds = 1e-3 * elapsed(e[kEvH2D1], e[kEvL2P]);
+  t.p2p_seconds = 1e-3 * elapsed(e[kEvGather], e[kEvNear1]);
+  t.kernel_seconds = 1e-3 * elapsed(kernels0, e[kEvL2P]);
   t.d2h_seconds = P->last_host ? 1e-3 * elapsed(e[kEvD2H0], e[kEvD2H1]) : 0.0;
   t.total_seconds = 1e-3 * elapsed(e[kEvH2D0], P->last_host ? e[kEvD2H1] : e[kEvL2P]);
-  t.m2l_kernel_seconds = P->d.L >= 2 ? 1e-3 * elapsed(e[kEvM2LKernel0], e[kEvM2LKernel1]) : 0.0;
+  t.m2l_kernel_seconds = P->d.L >= 2 ? 1e-3 * elapsed(m2l_kernel[0], m2l_kernel[1]) : 0.0;
   P->timings_pending = false;
 }
 
@@ -940,14 +961,18 @@ void install_identity(hipfmm_plan* P, const int* self) {
   }
 }
 
-// One evaluate enqueued on the plan's streams.  `fork`: when set, the
-// plan's streams start after this event (recorded by the caller on `user`)
-// instead of an event of their own; `join` = false leaves the wait of `user`
-// on the plan's last stage to the caller.
+// One evaluate.  The near field runs on a stream of the plan's.  The rest of a
+// device-resident evaluate runs on the caller's stream `user`, which then needs
+// no fork and no join (1,000 points, p = 4, depth 2: 97 us per evaluate, with
+// both 117).
+// `fork`: when set, the far field runs on the plan's own stream after this
+// event (recorded by the caller on `user`), and the wait of `user` on the
+// plan's last stage is left to the caller.  Evaluates of one plan run in the
+// order of their calls, whatever their streams.
 template <class S>
 void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* potentials, int K, const int* self,
                    int memspace, hipStream_t user, bool adjoint, void* field_gradients = nullptr,
-                   hipEvent_t fork = nullptr, bool join = true) {
+                   hipEvent_t fork = nullptr) {
   const bool want_pot = potentials != nullptr;
   const bool want_grad = field_gradients != nullptr;
   {
@@ -971,8 +996,19 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   ensure_capacity<S>(P, K, want_pot, want_grad);
   DevicePlan d = adjoint ? role_exchanged(P) : P->d;
   d.compressed_state_major = d.nc > 0 && (sizeof(S) == 8 || K % 32 != 0);
-  hipStream_t s = P->s_far;
+  const bool host = memspace == HIPFMM_HOST;
+  const hipStream_t s = host || fork != nullptr ? far_stream(P) : user;
   hipEvent_t* e = P->ev;
+  // The plan's buffers are free once its last evaluate is done.  An event
+  // recorded inside a capture marks nothing outside it, so a captured evaluate
+  // has one of its own, and follows only those of the same capture (a graph's
+  // replays are the caller's to order).
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  unsigned long long capture_id = 0;
+  HIPFMM_CHECK(hipStreamGetCaptureInfo(host ? s : user, &capture, &capture_id));
+  const bool captured = capture != hipStreamCaptureStatusNone;
+  if (captured ? P->capture_id == capture_id : P->done_recorded)
+    HIPFMM_CHECK(hipStreamWaitEvent(s, e[captured ? kEvCaptured : kEvL2P], 0));
   auto mark = [&](int ev, hipStream_t on) {
     HIPFMM_CHECK(hipEventRecord(e[ev], on));
   };
@@ -985,7 +1021,6 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const size_t out_bytes = fields != nullptr ? size_t(K) * d.nt * 3 * sizeof(S) : 0;
   const size_t pot_bytes = want_pot ? size_t(K) * d.nt * sizeof(S) : 0;
   const size_t grad_bytes = want_grad ? size_t(K) * d.nt * 6 * sizeof(S) : 0;
-  const bool host = memspace == HIPFMM_HOST;
   if (host) {
     if (P->pinned_grad_bytes < grad_bytes) {
       if (P->pinned_grad) (void)hipHostFree(P->pinned_grad);
@@ -1024,13 +1059,8 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     P->stats.evaluation_h2d_calls += 1;
     P->stats.evaluation_d2h_calls += 1;
   } else {
-    if (fork == nullptr) {
-      HIPFMM_CHECK(hipEventRecord(e[kEvUser], user));
-      fork = e[kEvUser];
-    }
-    HIPFMM_CHECK(hipStreamWaitEvent(s, fork, 0));
+    if (fork != nullptr) HIPFMM_CHECK(hipStreamWaitEvent(s, fork, 0));
     mark(kEvH2D0, s);
-    mark(kEvH2D1, s);
     mu = static_cast<const S*>(moments);
     out = static_cast<S*>(fields);
     pot = static_cast<S*>(potentials);
@@ -1042,7 +1072,6 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   hipfmm::launch_gather<S>(d, mu, scale, K, s);
   HIPFMM_CHECK(hipEventRecord(e[kEvGather], s));
   HIPFMM_CHECK(hipStreamWaitEvent(P->s_near, e[kEvGather], 0));
-  mark(kEvNear0, P->s_near);
   if (want_grad)
     hipfmm::launch_p2p_grad<S>(d, K, P->s_near);
   else
@@ -1068,10 +1097,10 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   } else {
     for (int level = d.L - 1; level >= 2; --level) hipfmm::launch_m2m<S>(d, level, K, s);
   }
-  // Levels 0 and 1 hold no list-2 work; keep their coefficients zero.
-  const size_t top = size_t(std::min<int64_t>(d.nodes, 9)) * d.n * K;
-  hipfmm::launch_zero<S>(static_cast<S*>(d.M), top, s);
-  hipfmm::launch_zero<S>(static_cast<S*>(d.Lc), d.L >= 2 ? top : size_t(d.nodes) * d.n * K, s);
+  // Levels 0 and 1 hold no list-2 work: their coefficients are zero
+  // (hipfmm_plan_coefficients), and only a tree without deeper levels reads
+  // them here.
+  if (d.L < 2) hipfmm::launch_zero<S>(static_cast<S*>(d.Lc), size_t(d.nodes) * d.n * K, s);
   mark(kEvM2M, s);
   // The 16-bit modes split the multipoles in a pass of their own and run in
   // workgroups of 256 columns whose chain of up to 189 offsets takes 0.23-0.6
@@ -1120,8 +1149,8 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   // p = 6, one state: M2L 2.04 ms beside the near field's tail, 1.24 ms after
   // it).  A smaller matrix-core batch has too few workgroups to fill the chip
   // and keeps running beside the near field.
-  if (!mfma || K >= 32) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
-  mark(kEvM2LKernel0, s);
+  const bool after_near = !mfma || K >= 32;
+  if (after_near) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
   const int ring_slot = int(P->m2l_launch_count % hipfmm_plan::kRing);
   drain_m2l_slot(P, ring_slot);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][0], s));
@@ -1133,12 +1162,15 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     hipfmm::launch_m2l_full<S>(dm, K, s);
   else
     hipfmm::launch_m2l_valu<S>(dm, K, s);
-  mark(kEvM2LKernel1, s);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][1], s));
   P->m2l_ring_pending[ring_slot] = true;
+  P->last_ring_slot = ring_slot;
   ++P->m2l_launch_count;
-  if (d.nc > 0 && d.L >= 2 && !harmonic) hipfmm::launch_m2l_expand<S>(d, K, 2, s);
-  mark(kEvM2L, s);
+  P->last_m2l_expands = d.nc > 0 && d.L >= 2 && !harmonic;
+  if (P->last_m2l_expands) {
+    hipfmm::launch_m2l_expand<S>(d, K, 2, s);
+    mark(kEvM2L, s);
+  }
   if (harmonic) {
     for (int level = 3; level <= d.L; ++level) hipfmm::launch_l2l<S>(dc, level, K, s);
     hipfmm::launch_m2l_expand<S>(d, K, d.L, s);
@@ -1146,12 +1178,17 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     for (int level = 3; level <= d.L; ++level) hipfmm::launch_l2l<S>(d, level, K, s);
   }
   mark(kEvL2L, s);
-  HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
+  if (!after_near) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
   if (want_grad)
     hipfmm::launch_l2p_grad_unsort<S>(d, grad, K, s);
   else
     hipfmm::launch_l2p_unsort<S>(d, out, pot, K, s);
-  HIPFMM_CHECK(hipEventRecord(e[kEvL2P], s));
+  P->last_done = captured ? kEvCaptured : kEvL2P;
+  HIPFMM_CHECK(hipEventRecord(e[P->last_done], s));
+  if (captured)
+    P->capture_id = capture_id;
+  else
+    P->done_recorded = true;
   P->last_K = K;
   P->last_host = host;
   P->timings_pending = true;
@@ -1167,8 +1204,6 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     if (pot_bytes) std::memcpy(potentials, P->pinned_pot, pot_bytes);
     if (grad_bytes) std::memcpy(field_gradients, P->pinned_grad, grad_bytes);
     finalize_timings(P);
-  } else if (join) {
-    HIPFMM_CHECK(hipStreamWaitEvent(user, e[kEvL2P], 0));
   }
 }
 
@@ -1281,7 +1316,6 @@ int hipfmm_plan_create(const hipfmm_plan_desc* desc, hipfmm_plan** plan) {
     }
     auto P = std::make_unique<hipfmm_plan>();
     HIPFMM_CHECK(hipGetDevice(&P->device));
-    HIPFMM_CHECK(hipStreamCreateWithFlags(&P->s_far, hipStreamNonBlocking));
     HIPFMM_CHECK(hipStreamCreateWithFlags(&P->s_near, hipStreamNonBlocking));
     for (auto& ev : P->ev) HIPFMM_CHECK(hipEventCreate(&ev));
     for (auto& pair : P->m2l_ring)
@@ -1493,9 +1527,13 @@ int hipfmm_plan_coefficients(hipfmm_plan* plan, int which, int node, int state, 
     require(d.m2m_dense_c == nullptr || node >= hipfmm::level_offset(d.L),
             "this plan forms the expansions above the leaf level in harmonic-subspace form only");
     DeviceGuard guard(plan->device);
-    HIPFMM_CHECK(hipStreamSynchronize(plan->s_far));
+    wait_for_evaluates(plan);
     const int K = plan->last_K;
     const size_t elem = d.precision == 32 ? 4 : 8;
+    if (node < 9) {  // levels 0 and 1
+      std::fill(out, out + d.n, 0.0);
+      return;
+    }
     std::vector<unsigned char> buf(size_t(d.n) * K * elem);
     const void* base = which == 0 ? d.M : d.Lc;
     HIPFMM_CHECK(hipMemcpy(buf.data(), static_cast<const unsigned char*>(base) + size_t(node) * d.n * K * elem,
@@ -1513,6 +1551,7 @@ void hipfmm_plan_destroy(hipfmm_plan* plan) {
   int prev = -1;
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(plan->device);
+  if (plan->done_recorded) (void)hipEventSynchronize(plan->ev[kEvL2P]);
   if (plan->s_far) (void)hipStreamSynchronize(plan->s_far);
   if (plan->s_near) (void)hipStreamSynchronize(plan->s_near);
   free_state(plan);
@@ -1652,6 +1691,7 @@ int hipfmm_group_create(hipfmm_plan* const* plans, int count, const void* const*
       hipfmm_plan* P = plans[i];
       if (sorted_self_indices != nullptr) install_identity(P, sorted_self_indices[i]);
       if (P->timings_pending) finalize_timings(P);
+      far_stream(P);
       if (P->d.precision == 32)
         ensure_capacity<float>(P, batches[i], false);
       else
@@ -1674,12 +1714,12 @@ int hipfmm_group_launch(hipfmm_group* group, void* stream) {
       hipfmm_plan* P = group->plans[i];
       if (P->d.precision == 32)
         evaluate_impl<float>(P, group->moments[i], group->fields[i], nullptr, group->batches[i], nullptr,
-                             HIPFMM_DEVICE, user, false, nullptr, group->fork, false);
+                             HIPFMM_DEVICE, user, false, nullptr, group->fork);
       else
         evaluate_impl<double>(P, group->moments[i], group->fields[i], nullptr, group->batches[i], nullptr,
-                              HIPFMM_DEVICE, user, false, nullptr, group->fork, false);
+                              HIPFMM_DEVICE, user, false, nullptr, group->fork);
     }
-    for (hipfmm_plan* P : group->plans) HIPFMM_CHECK(hipStreamWaitEvent(user, P->ev[kEvL2P], 0));
+    for (hipfmm_plan* P : group->plans) HIPFMM_CHECK(hipStreamWaitEvent(user, P->ev[P->last_done], 0));
   });
 }
 

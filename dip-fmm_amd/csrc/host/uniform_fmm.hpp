@@ -259,10 +259,11 @@ class UniformFmm {
   std::span<const int> resolve_self_indices(std::span<const int> ids) const;
   void validate_identities(std::span<const int> ids, std::size_t moment_count) const;
   std::vector<int> sorted_self_indices(std::span<const int> ids) const;
+  const int* plan_self_indices(std::span<const int> ids, std::vector<int>& map) const;
   void record_timings();
   template <class S>
   void run_outputs(const S* moments, std::vector<S>& fields, std::vector<S>& potentials, OutputFlags output,
-                   const std::vector<int>& self);
+                   const int* self);
 
   UniformTree tree_;
   Basis basis_;
