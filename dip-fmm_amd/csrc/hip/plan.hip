@@ -1317,9 +1317,15 @@ int hipfmm_plan_create(const hipfmm_plan_desc* desc, hipfmm_plan** plan) {
     auto P = std::make_unique<hipfmm_plan>();
     HIPFMM_CHECK(hipGetDevice(&P->device));
     HIPFMM_CHECK(hipStreamCreateWithFlags(&P->s_near, hipStreamNonBlocking));
-    for (auto& ev : P->ev) HIPFMM_CHECK(hipEventCreate(&ev));
+    // The events between stages order kernels of this device and are read for
+    // their times, so they release at device scope; the default's release to
+    // the system took 3-4 us at each (1,000 points, p = 4: 95 us per evaluate,
+    // now 74).  The ends of an evaluate keep it.
+    for (int i = 0; i < kEvCount; ++i)
+      HIPFMM_CHECK(hipEventCreateWithFlags(
+          &P->ev[i], i == kEvL2P || i == kEvCaptured || i == kEvD2H1 ? hipEventDefault : hipEventDisableSystemFence));
     for (auto& pair : P->m2l_ring)
-      for (auto& ev : pair) HIPFMM_CHECK(hipEventCreate(&ev));
+      for (auto& ev : pair) HIPFMM_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableSystemFence));
     P->device_moment_scale = desc->device_moment_scale;
     P->m2l_mode = desc->m2l_mode;
     try {
