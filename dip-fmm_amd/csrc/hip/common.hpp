@@ -34,6 +34,7 @@ __host__ __device__ inline int64_t box_x3_elems(int R, int D) {
 }
 // Tiles per workgroup of the matrix-core M2L shapes (4 waves x 1..5 tiles).
 constexpr int kM2LGroupTiles[5] = {4, 8, 12, 16, 20};
+constexpr int kM2LSparseTiles = 8;
 constexpr int kMaxOrder = 10;
 constexpr int kOffsetSlots = 343;  // (dx,dy,dz) in [-3,3]^3
 
@@ -122,6 +123,8 @@ struct ShiftCsr {
   void* values = nullptr;      // (L+1) x 8 x nnz scalars (levels 1..L used)
 };
 
+__host__ __device__ inline bool bit_of(const uint32_t* bits, int64_t node) { return (bits[node >> 5] >> (node & 31)) & 1u; }
+
 // Everything the kernels read, with device pointers.
 struct DevicePlan {
   int precision = 32;
@@ -179,6 +182,18 @@ struct DevicePlan {
   int* m2l_order = nullptr;
   int m2l_order_base[5][kMaxLevels] = {};
   int m2l_order_len[5][kMaxLevels] = {};
+  // Where many boxes hold no points (null otherwise; plan.hip gives the line):
+  // a bit per node that holds sources and one per node that holds targets, and
+  // the tile order of kM2LSparseTiles tiles per workgroup over the boxes that
+  // hold targets: the parent of tile i of a parity is sparse_order[
+  // sparse_base[level] + parity * sparse_len[level] + i].  The M2L leaves out
+  // sources without moments (zeros), and the locals of boxes without targets,
+  // which no target reads.
+  const uint32_t* source_bits = nullptr;
+  const uint32_t* target_bits = nullptr;
+  const int* sparse_order = nullptr;
+  int sparse_base[kMaxLevels] = {};
+  int sparse_len[kMaxLevels] = {};
   void* ms = nullptr;        // (L+1) x n
   void* ls = nullptr;
   ShiftCsr m2m, l2l;

@@ -23,6 +23,8 @@
 //     the last depth value is left out, and where n = 16 r + 1 (p = 6 and 8)
 //     the last row is summed on the vector ALUs from the fragments at hand, an
 //     eighth of what a row tile for it would cost.
+//   * Sources and targets in boxes without points are left out where the plan
+//     has the bits for it (DevicePlan::source_bits).
 //   * A source's Morton index is formed in dilated coordinates: three
 //     subtractions under masks; an index outside the grid carries into higher
 //     bits, so one compare tells.
@@ -114,18 +116,21 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_full_kernel(const DevicePl
   const int64_t cols = (int64_t(1) << (3 * (level - 1))) * K;
   const uint32_t boxes = uint32_t(1) << (3 * level);
   const int64_t box_size = int64_t(N) * K;
-  const S* Mc = static_cast<const S*>(d.M) + level_offset(level) * box_size;
+  const int64_t lvl0 = level_offset(level);
+  const S* Mc = static_cast<const S*>(d.M) + lvl0 * box_size;
   // Targets: dilated coordinates, state, and the index limit of a source in
   // the grid (0 for a column past the end: no source passes).
   uint32_t tx[CT], ty[CT], tz[CT], limit[CT];
   int state[CT];
+  bool alive = false;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     const int64_t col = (int64_t(lb >> 3) * CT + c) * 16 + i;
     const uint32_t parent = uint32_t((col < cols ? col : 0) / K), m = parent * 8 + uint32_t(parity);
     state[c] = int(col < cols ? col - int64_t(parent) * K : 0);
     tx[c] = m & kX, ty[c] = m & kY, tz[c] = m & kZ;
-    limit[c] = col < cols ? boxes : 0u;
+    limit[c] = col < cols && (d.target_bits == nullptr || bit_of(d.target_bits, lvl0 + m)) ? boxes : 0u;
+    alive |= limit[c] != 0;
   }
   typename M::Acc acc[RT][CT];
   S xs[CT];
@@ -135,7 +140,7 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_full_kernel(const DevicePl
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][c] = typename M::Acc{};
   }
-  const int o_end = (wave + 1) * kOffsets / waves;
+  const int o_end = __any(alive) ? (wave + 1) * kOffsets / waves : 0;  // nothing for columns without targets
   const int4* step = steps + parity * kOffsets;
   // The next offset from `o` on with a source for some column: its operands.
   const S* src[CT];
@@ -148,7 +153,8 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_full_kernel(const DevicePl
       for (int c = 0; c < CT; ++c) {
         const uint32_t s = ((tx[c] - uint32_t(st.x)) & kX) | ((ty[c] - uint32_t(st.y)) & kY) |
                            ((tz[c] - uint32_t(st.z)) & kZ);
-        const bool ok = s < limit[c];
+        bool ok = s < limit[c];
+        if (d.source_bits != nullptr) ok = ok && bit_of(d.source_bits, lvl0 + s);
         any |= ok;
         src[c] = (ok ? Mc + int64_t(s) * box_size : zeros) + state[c] * (kRuns ? N : 1);
       }
@@ -260,7 +266,7 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_full_kernel(const DevicePl
     __syncthreads();
   }
   if (wave != 0) return;
-  S* Lc = static_cast<S*>(d.Lc) + level_offset(level) * box_size;
+  S* Lc = static_cast<S*>(d.Lc) + lvl0 * box_size;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     if (limit[c] == 0) continue;
@@ -301,23 +307,26 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_bf16_direct_kernel(const D
   const int64_t cols = (int64_t(1) << (3 * (level - 1))) * K;
   const uint32_t boxes = uint32_t(1) << (3 * level);
   const int64_t box_size = int64_t(N) * K;
-  const float* Mc = static_cast<const float*>(d.M) + level_offset(level) * box_size;
+  const int64_t lvl0 = level_offset(level);
+  const float* Mc = static_cast<const float*>(d.M) + lvl0 * box_size;
   uint32_t tx[CT], ty[CT], tz[CT], limit[CT];
   int state[CT];
+  bool alive = false;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     const int64_t col = (int64_t(lb >> 3) * CT + c) * 32 + i;
     const uint32_t parent = uint32_t((col < cols ? col : 0) / K), m = parent * 8 + uint32_t(parity);
     state[c] = int(col < cols ? col - int64_t(parent) * K : 0);
     tx[c] = m & kX, ty[c] = m & kY, tz[c] = m & kZ;
-    limit[c] = col < cols ? boxes : 0u;
+    limit[c] = col < cols && (d.target_bits == nullptr || bit_of(d.target_bits, lvl0 + m)) ? boxes : 0u;
+    alive |= limit[c] != 0;
   }
   f32x16 acc[MT][CT];
 #pragma unroll
   for (int r = 0; r < MT; ++r)
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[r][c] = f32x16{};
-  const int o_end = (wave + 1) * kOffsets / waves;
+  const int o_end = __any(alive) ? (wave + 1) * kOffsets / waves : 0;  // nothing for columns without targets
   const int4* step = steps + parity * kOffsets;
   const float* src[CT];
   const uint4 *hi = nullptr, *lo = nullptr;
@@ -329,7 +338,8 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_bf16_direct_kernel(const D
       for (int c = 0; c < CT; ++c) {
         const uint32_t s = ((tx[c] - uint32_t(st.x)) & kX) | ((ty[c] - uint32_t(st.y)) & kY) |
                            ((tz[c] - uint32_t(st.z)) & kZ);
-        const bool ok = s < limit[c];
+        bool ok = s < limit[c];
+        if (d.source_bits != nullptr) ok = ok && bit_of(d.source_bits, lvl0 + s);
         any |= ok;
         src[c] = (ok ? Mc + int64_t(s) * box_size : zeros) + state[c] * N;
       }
@@ -430,7 +440,7 @@ __global__ void __launch_bounds__(64 * kWavesMax) m2l_bf16_direct_kernel(const D
     __syncthreads();
   }
   if (wave != 0) return;
-  float* Lc = static_cast<float*>(d.Lc) + level_offset(level) * box_size;
+  float* Lc = static_cast<float*>(d.Lc) + lvl0 * box_size;
 #pragma unroll
   for (int c = 0; c < CT; ++c) {
     if (limit[c] == 0) continue;

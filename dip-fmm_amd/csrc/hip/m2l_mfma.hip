@@ -169,11 +169,17 @@ struct LevelTable {
   // (-1: padding); null when tiles follow the Morton order of the parents.
   const int* order;
   int order_base[12];
+  int order_stride[12];  // from one parity's order to the next (0: they share one)
 };
 
 // Morton index of the parent of tile group bg (-1 for a padding tile).
-__device__ __forceinline__ int64_t tile_parent(const LevelTable& lt, int li, int bg) {
-  return lt.order ? int64_t(lt.order[lt.order_base[li] + bg]) : int64_t(bg);
+__device__ __forceinline__ int64_t tile_parent(const LevelTable& lt, int li, int parity, int bg) {
+  return lt.order ? int64_t(lt.order[lt.order_base[li] + parity * lt.order_stride[li] + bg]) : int64_t(bg);
+}
+
+// False for a source box known to hold no sources: its operands are zeros.
+__device__ __forceinline__ bool holds_sources(const DevicePlan& d, int64_t node) {
+  return d.source_bits == nullptr || bit_of(d.source_bits, node);
 }
 
 // Per-lane view of the columns of the NB tiles one wave owns.  With
@@ -362,7 +368,7 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
     const int bg = tile / kchunks, kc = tile % kchunks;
     int64_t q;
     if constexpr (kUniformBox) {
-      q = tile < tiles ? tile_parent(lt, li, bg) : -1;  // one box per tile
+      q = tile < tiles ? tile_parent(lt, li, parity, bg) : -1;  // one box per tile
       c.kk[nb] = kc * 32;
       c.valid[nb] = q >= 0 && q < parents;
     } else {
@@ -378,8 +384,8 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
   }
   for (int i = threadIdx.x; i < kParityOffsets; i += W * 64) offs_all[i] = d.parity_offsets[parity * kParityOffsets + i];
   __syncthreads();
-  // Offsets no column of this workgroup can use (source outside the grid for
-  // all of them) are dropped from the step sequence.
+  // Offsets no column of this workgroup can use (source outside the grid, or
+  // without points, for all of them) are dropped from the step sequence.
   if constexpr (kUniformBox) {
     // Every tile is one box: thread i decides offset i for all W*NB tiles.
     for (int i = threadIdx.x; i < kParityOffsets; i += W * 64) {
@@ -388,12 +394,13 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
       for (int t = 0; t < W * NB; ++t) {
         const int tile = wgp * W * NB + t;
         if (tile >= tiles) continue;
-        const int64_t q = tile_parent(lt, li, tile / kchunks);
+        const int64_t q = tile_parent(lt, li, parity, tile / kchunks);
         if (q < 0 || q >= parents) continue;
         int x, y, z;
         demorton3(uint32_t(q), level - 1, x, y, z);
         const int sx = 2 * x + px - o.x, sy = 2 * y + py - o.y, sz = 2 * z + pz - o.z;
-        any |= sx >= 0 && sy >= 0 && sz >= 0 && sx < sg.nbox && sy < sg.nbox && sz < sg.nbox;
+        any |= sx >= 0 && sy >= 0 && sz >= 0 && sx < sg.nbox && sy < sg.nbox && sz < sg.nbox &&
+               holds_sources(d, sg.lvl0 + morton3(uint32_t(sx), uint32_t(sy), uint32_t(sz), level));
       }
       used[0][i] = any ? 1 : 0;
     }
@@ -439,7 +446,7 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
       }
       const int tile = wgp * W * NB + t;
       const int kc = tile % kchunks;
-      const int64_t q = tile < tiles ? tile_parent(lt, li, tile / kchunks) : -1;
+      const int64_t q = tile < tiles ? tile_parent(lt, li, parity, tile / kchunks) : -1;
       uint32_t off = kOutside;
       if (q >= 0 && q < parents) {
         int x, y, z;
@@ -447,7 +454,8 @@ __global__ void __launch_bounds__(W * 64, 1) m2l_mfma_kernel(const DevicePlan d,
         const int sx = 2 * x + px - o.x, sy = 2 * y + py - o.y, sz = 2 * z + pz - o.z;
         if (sx >= 0 && sy >= 0 && sz >= 0 && sx < sg.nbox && sy < sg.nbox && sz < sg.nbox) {
           const uint64_t snode = uint64_t(sg.lvl0 + morton3(uint32_t(sx), uint32_t(sy), uint32_t(sz), level));
-          off = uint32_t((snode * uint64_t(sg.KS) * uint64_t(K) + uint64_t(kc) * 32u) * 32u);
+          if (holds_sources(d, int64_t(snode)))
+            off = uint32_t((snode * uint64_t(sg.KS) * uint64_t(K) + uint64_t(kc) * 32u) * 32u);
         }
       }
       tab.b[a][t] = off;
@@ -542,18 +550,22 @@ LevelTable level_table(const DevicePlan& d, int states, int K, int nb) {
   for (int i = 0; i < 5; ++i)
     if (kM2LGroupTiles[i] == kWaves * nb) g = i;
   const bool ordered = uniform_box(d, K) && d.m2l_order != nullptr && g >= 0;
-  lt.order = ordered ? d.m2l_order : nullptr;
+  const bool sparse = ordered && d.sparse_order != nullptr && kWaves * nb == kM2LSparseTiles;
+  lt.order = sparse ? d.sparse_order : ordered ? d.m2l_order : nullptr;
   int begin = 0;
   for (int i = 0; i < lt.count; ++i) {
-    const int level = 2 + i;
+    const int level = sparse ? d.L - i : 2 + i;  // the last level first (see inner_class_first)
     lt.level[i] = level;
     int cpb = 1;
     while (cpb < K && cpb < 32) cpb *= 2;
     const int kchunks = (K + cpb - 1) / cpb;
     const int64_t parents = int64_t(1) << (3 * (level - 1));
     const int boxes_per_tile = 32 / cpb;
-    const int groups = ordered ? d.m2l_order_len[g][level] : int((parents + boxes_per_tile - 1) / boxes_per_tile);
-    lt.order_base[i] = ordered ? d.m2l_order_base[g][level] : 0;
+    const int groups = sparse    ? d.sparse_len[level]
+                       : ordered ? d.m2l_order_len[g][level]
+                                 : int((parents + boxes_per_tile - 1) / boxes_per_tile);
+    lt.order_base[i] = sparse ? d.sparse_base[level] : ordered ? d.m2l_order_base[g][level] : 0;
+    lt.order_stride[i] = sparse ? d.sparse_len[level] : 0;
     const int tiles = groups * kchunks;
     const int bpp = (tiles + kWaves * nb - 1) / (kWaves * nb);
     lt.block_begin[i] = begin;
@@ -579,7 +591,8 @@ LevelTable level_table(const DevicePlan& d, int states, int K, int nb) {
 // 13.7 GB.)
 bool inner_class_first(const LevelTable& lt, int L, int G, LevelTable& out) {
   const int last = lt.count - 1;
-  if (lt.order == nullptr || L < 4 || last < 0 || lt.level[last] != L || lt.count + 2 > 12) return false;
+  if (lt.order == nullptr || L < 4 || last < 0 || lt.level[last] != L || lt.order_stride[last] != 0 || lt.count + 2 > 12)
+    return false;
   const int64_t np = int64_t(1) << (L - 1);
   const int inner_groups = int(((np - 2) * (np - 2) * (np - 2) + G - 1) / G * G);
   const int kchunks = lt.kchunks[last], inner_tiles = inner_groups * kchunks;
@@ -609,6 +622,7 @@ template <int MT, int NB, int kStages, bool kF16>
 void launch_uniform(const DevicePlan& v, const LevelTable& lt, int K, hipStream_t s) {
   LevelTable t;
   const LevelTable& use = inner_class_first(lt, v.L, kWaves * NB, t) ? t : lt;
+  if (use.block_begin[use.count] == 0) return;  // no box holds targets
   m2l_mfma_kernel<MT, NB, kWaves, kStages, true, kF16>
       <<<unsigned(use.block_begin[use.count]), kWaves * 64, 0, s>>>(v, use, K);
 }

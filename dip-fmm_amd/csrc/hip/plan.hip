@@ -64,6 +64,17 @@ enum Ev {
 
 }  // namespace
 
+// The M2L kernels: in the type's own precision on the vector ALUs or the matrix
+// cores, in bf16 without split operands, and in tiles of split operands.
+enum M2lPath { kVectorM2l, kFullM2l, kDirectM2l, kTileM2l };
+
+// Tile order of the M2L over the boxes that hold points (DevicePlan::sparse_order).
+struct SparseBoxes {
+  std::vector<int> order;
+  int base[hipfmm::kMaxLevels] = {};
+  int len[hipfmm::kMaxLevels] = {};
+};
+
 struct hipfmm_plan {
   DevicePlan d;
   int device = 0;
@@ -91,6 +102,8 @@ struct hipfmm_plan {
   int* adj_nbr_blk_start = nullptr;
   int* adj_nbr_blk = nullptr;
   int* adj_self = nullptr;
+  SparseBoxes adj_sparse;  // bases and lengths; the order itself is adj_sparse_order
+  const int* adj_sparse_order = nullptr;
   bool adj_self_valid = true;  // false when two targets share one source
   bool potential_used = false;  // keep the near-field potential buffers in the state
   bool gradient_used = false;   // keep the field-gradient buffers in the state
@@ -111,6 +124,9 @@ struct hipfmm_plan {
   hipEvent_t m2l_ring[kRing][2] = {};
   bool m2l_ring_pending[kRing] = {};
   int last_ring_slot = 0;         // of the last evaluate
+  M2lPath last_path = kFullM2l;   // what it ran, for complete_locals
+  int last_mode = 0;
+  bool last_adjoint = false;
   bool last_m2l_expands = false;  // its M2L ends at kEvM2L, after its kernel
   uint64_t m2l_launch_count = 0;
   double m2l_total_seconds = 0.0;
@@ -322,6 +338,103 @@ void refresh_adjoint_self(hipfmm_plan* P) {
     inv[s] = t;
   }
   if (P->adj_self && d.ns) HIPFMM_CHECK(hipMemcpy(P->adj_self, inv.data(), size_t(d.ns) * sizeof(int), hipMemcpyHostToDevice));
+}
+
+// List-2 pairs of the levels 2..L: of the grid, and with points on both sides
+// (of all levels and of the last).
+template <class F>
+void count_m2l_pairs(int L, F&& occupied, uint64_t& grid, uint64_t& pairs, uint64_t& leaf_pairs) {
+  for (int level = 2; level <= L; ++level) {
+    const int nb = 1 << level;
+    for (int64_t m = 0; m < (int64_t(1) << (3 * level)); ++m) {
+      int x, y, z;
+      hipfmm::demorton3(uint32_t(m), level, x, y, z);
+      auto inside = [&](int c, int reach) {  // sources within reach boxes of the target's parent, or of the target
+        const int lo = reach == 1 ? c - 1 : (c & ~1) - 2, hi = reach == 1 ? c + 1 : (c & ~1) + 3;
+        return uint64_t(std::min(hi, nb - 1) - std::max(lo, 0) + 1);
+      };
+      grid += inside(x, 2) * inside(y, 2) * inside(z, 2) - inside(x, 1) * inside(y, 1) * inside(z, 1);
+      if (!occupied(level, m, false)) continue;
+      for (int ox = (x & 1) - 3; ox <= (x & 1) + 2; ++ox)
+        for (int oy = (y & 1) - 3; oy <= (y & 1) + 2; ++oy)
+          for (int oz = (z & 1) - 3; oz <= (z & 1) + 2; ++oz) {
+            if (std::max({std::abs(ox), std::abs(oy), std::abs(oz)}) <= 1) continue;
+            const int sx = x - ox, sy = y - oy, sz = z - oz;
+            if (sx < 0 || sy < 0 || sz < 0 || sx >= nb || sy >= nb || sz >= nb) continue;
+            if (occupied(level, int64_t(hipfmm::morton3(sx, sy, sz, level)), true)) {
+              ++pairs;
+              if (level == L) ++leaf_pairs;
+            }
+          }
+    }
+  }
+}
+
+// The parents of a level's boxes in the order of the M2L's tiles, a list per
+// boundary class (one in Morton order below level 4).
+std::vector<std::vector<int>> boundary_classes(int level) {
+  const int bits = level - 1, np = 1 << bits;
+  const int64_t parents = int64_t(1) << (3 * bits);
+  if (level < 4) {
+    std::vector<int> all(static_cast<size_t>(parents));
+    for (int64_t q = 0; q < parents; ++q) all[size_t(q)] = int(q);
+    return {all};
+  }
+  // Within a class the parents follow the Morton order of their coordinates
+  // relative to the class's own region (inner axes from 1, boundary axes
+  // fixed), so a workgroup's parents are whole aligned octants of the inner
+  // region (14 = 2 x 7 per axis at level 5) or compact patches of a face.
+  std::vector<std::vector<std::pair<uint32_t, int>>> cls(27);
+  auto axis_class = [&](int c) { return c == 0 ? 0 : (c == np - 1 ? 2 : 1); };
+  auto rel = [&](int c) { return uint32_t(axis_class(c) == 1 ? c - 1 : 0); };
+  for (int64_t q = 0; q < parents; ++q) {
+    int x, y, z;
+    hipfmm::demorton3(uint32_t(q), bits, x, y, z);
+    cls[(axis_class(x) * 3 + axis_class(y)) * 3 + axis_class(z)].push_back(
+        {hipfmm::morton3(rel(x), rel(y), rel(z), bits), int(q)});
+  }
+  // Classes in the order inner, faces, edges, corners: the inner class (most
+  // of the work, every offset active) first, so that its equal-length
+  // workgroups start together and walk the offsets in step, reading one
+  // shifted region of sources that L2 holds; the shorter boundary workgroups
+  // follow and fill the tail.
+  auto boundary_axes = [](int k) { return int(k / 9 != 1) + int(k / 3 % 3 != 1) + int(k % 3 != 1); };
+  std::vector<int> class_order(27);
+  for (int k = 0; k < 27; ++k) class_order[k] = k;
+  std::stable_sort(class_order.begin(), class_order.end(),
+                   [&](int a, int b) { return boundary_axes(a) < boundary_axes(b); });
+  std::vector<std::vector<int>> out;
+  for (const int k : class_order) {
+    auto& c = cls[k];
+    std::stable_sort(c.begin(), c.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+    out.emplace_back();
+    for (const auto& e : c) out.back().push_back(e.second);
+  }
+  return out;
+}
+
+// The tile order of the M2L over the boxes of a level that `holds` names: per
+// parity the parents of its boxes, each class padded to whole workgroups and
+// the parities to one length.
+template <class F>
+void add_sparse_level(SparseBoxes& b, int level, const std::vector<std::vector<int>>& classes, F&& holds) {
+  std::vector<int> lists[8];
+  size_t most = 0;
+  for (int parity = 0; parity < 8; ++parity) {
+    auto& l = lists[parity];
+    for (const auto& c : classes) {
+      for (const int q : c)
+        if (holds(int64_t(q) * 8 + parity)) l.push_back(q);
+      l.resize((l.size() + hipfmm::kM2LSparseTiles - 1) / hipfmm::kM2LSparseTiles * hipfmm::kM2LSparseTiles, -1);
+    }
+    most = std::max(most, l.size());
+  }
+  b.base[level] = int(b.order.size());
+  b.len[level] = int(most);
+  for (auto& l : lists) {
+    l.resize(most, -1);
+    b.order.insert(b.order.end(), l.begin(), l.end());
+  }
 }
 
 template <class S>
@@ -651,52 +764,59 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   // workgroups: at 1M points, depth 5, the products beyond the list-2 pairs
   // fall from 17% to 3%.  Levels 2 and 3 keep the Morton order, which pads
   // less there.
+  // Where a tenth or more of the list-2 pairs have a box without points, the
+  // M2L takes boxes with targets only, and sources with points only: 2^20
+  // points in blobs, depth 6, 32 states, M2L 52.6 -> 35.9 ms; 262,144 points of a slab
+  // seen from a plane, depth 5, one state, 296 -> 46 us.  Below that line the empty
+  // boxes are scattered singly, and the lists and bits would save less than
+  // their lookups cost.
+  const auto occupied = [&](int level, int64_t m, bool sources) {
+    const int64_t* r = ranges + 4 * (hipfmm::level_offset(level) + m) + (sources ? 0 : 2);
+    return r[1] > r[0];
+  };
+  uint64_t grid_pairs = 0, m2l_pairs = 0, leaf_pairs = 0;
+  count_m2l_pairs(L, occupied, grid_pairs, m2l_pairs, leaf_pairs);
+  const bool sparse = 10 * m2l_pairs <= 9 * grid_pairs && grid_pairs > 0;
   if (L >= 2 && L < hipfmm::kMaxLevels) {
     std::vector<int> order;
-    for (int g = 0; g < 5; ++g) {
-      const int G = hipfmm::kM2LGroupTiles[g];
-      for (int level = 2; level <= L; ++level) {
-        const int bits = level - 1, np = 1 << bits;
-        const int64_t parents = int64_t(1) << (3 * bits);
+    SparseBoxes boxes[2];  // of targets, and of sources (the adjoint's targets)
+    for (int level = 2; level <= L; ++level) {
+      const auto classes = boundary_classes(level);
+      for (int g = 0; g < 5; ++g) {
+        const int G = hipfmm::kM2LGroupTiles[g];
         d.m2l_order_base[g][level] = int(order.size());
-        if (level < 4) {
-          for (int64_t q = 0; q < parents; ++q) order.push_back(int(q));
-        } else {
-          // Within a class the parents follow the Morton order of their
-          // coordinates relative to the class's own region (inner axes from
-          // 1, boundary axes fixed), so a workgroup's parents are whole
-          // aligned octants of the inner region (14 = 2 x 7 per axis at
-          // level 5) or compact patches of a face.
-          std::vector<std::vector<std::pair<uint32_t, int>>> cls(27);
-          auto axis_class = [&](int c) { return c == 0 ? 0 : (c == np - 1 ? 2 : 1); };
-          auto rel = [&](int c) { return uint32_t(axis_class(c) == 1 ? c - 1 : 0); };
-          for (int64_t q = 0; q < parents; ++q) {
-            int x, y, z;
-            hipfmm::demorton3(uint32_t(q), bits, x, y, z);
-            cls[(axis_class(x) * 3 + axis_class(y)) * 3 + axis_class(z)].push_back(
-                {hipfmm::morton3(rel(x), rel(y), rel(z), bits), int(q)});
-          }
-          // Classes in the order inner, faces, edges, corners: the inner
-          // class (most of the work, every offset active) first, so that
-          // its equal-length workgroups start together and walk the offsets
-          // in step, reading one shifted region of sources that L2 holds;
-          // the shorter boundary workgroups follow and fill the tail.
-          auto boundary_axes = [](int k) { return int(k / 9 != 1) + int(k / 3 % 3 != 1) + int(k % 3 != 1); };
-          std::vector<int> class_order(27);
-          for (int k = 0; k < 27; ++k) class_order[k] = k;
-          std::stable_sort(class_order.begin(), class_order.end(),
-                           [&](int a, int b) { return boundary_axes(a) < boundary_axes(b); });
-          for (const int k : class_order) {
-            auto& c = cls[k];
-            std::stable_sort(c.begin(), c.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-            for (const auto& e : c) order.push_back(e.second);
-            order.insert(order.end(), (G - int(c.size()) % G) % G, -1);
-          }
+        for (const auto& c : classes) {
+          order.insert(order.end(), c.begin(), c.end());
+          if (level >= 4) order.insert(order.end(), (G - int(c.size()) % G) % G, -1);
         }
         d.m2l_order_len[g][level] = int(order.size()) - d.m2l_order_base[g][level];
       }
+      if (sparse)
+        for (int side = 0; side < 2; ++side)
+          add_sparse_level(boxes[side], level, classes, [&](int64_t m) { return occupied(level, m, side == 1); });
     }
     d.m2l_order = upload(P, order.data(), order.size());
+    if (sparse) {
+      std::vector<uint32_t> bits[2];
+      for (int side = 0; side < 2; ++side) {
+        bits[side].assign(size_t(d.nodes + 31) / 32, 0u);
+        for (int level = 0; level <= L; ++level)
+          for (int64_t m = 0; m < (int64_t(1) << (3 * level)); ++m) {
+            const int64_t node = hipfmm::level_offset(level) + m;
+            if (occupied(level, m, side == 1)) bits[side][size_t(node >> 5)] |= 1u << (node & 31);
+          }
+      }
+      d.target_bits = upload(P, bits[0].data(), bits[0].size());
+      const bool same = bits[0] == bits[1];
+      d.source_bits = same ? d.target_bits : upload(P, bits[1].data(), bits[1].size());
+      d.sparse_order = upload(P, boxes[0].order.data(), boxes[0].order.size());
+      P->adj_sparse = boxes[1];
+      P->adj_sparse_order = same ? d.sparse_order : upload(P, boxes[1].order.data(), boxes[1].order.size());
+      std::copy(boxes[0].base, boxes[0].base + hipfmm::kMaxLevels, d.sparse_base);
+      std::copy(boxes[0].len, boxes[0].len + hipfmm::kMaxLevels, d.sparse_len);
+      P->adj_sparse.order.clear();
+      P->adj_sparse.order.shrink_to_fit();
+    }
   }
   std::vector<S> ms(size_t(L + 1) * n), lsc(size_t(L + 1) * n);
   for (size_t i = 0; i < ms.size(); ++i) {
@@ -719,29 +839,7 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   P->stats.m2l_unique_matrix_count = uint64_t(desc.m2l_class_count);
   P->stats.m2l_matrix_bytes = uint64_t(desc.m2l_class_count) * nn * sizeof(S);
   // Interaction counts of the canonical plan (non-empty pairs only).
-  uint64_t m2l_pairs = 0, p2p_pairs = 0, leaf_pairs = 0;
-  for (int level = 2; level <= L; ++level) {
-    const int nb = 1 << level;
-    const int64_t base = hipfmm::level_offset(level);
-    for (int64_t m = 0; m < (int64_t(1) << (3 * level)); ++m) {
-      const int64_t* r = ranges + 4 * (base + m);
-      if (r[3] == r[2]) continue;
-      int x, y, z;
-      hipfmm::demorton3(uint32_t(m), level, x, y, z);
-      for (int ox = (x & 1) - 3; ox <= (x & 1) + 2; ++ox)
-        for (int oy = (y & 1) - 3; oy <= (y & 1) + 2; ++oy)
-          for (int oz = (z & 1) - 3; oz <= (z & 1) + 2; ++oz) {
-            if (std::max({std::abs(ox), std::abs(oy), std::abs(oz)}) <= 1) continue;
-            const int sx = x - ox, sy = y - oy, sz = z - oz;
-            if (sx < 0 || sy < 0 || sz < 0 || sx >= nb || sy >= nb || sz >= nb) continue;
-            const int64_t* sr = ranges + 4 * (base + hipfmm::morton3(sx, sy, sz, level));
-            if (sr[1] != sr[0]) {
-              ++m2l_pairs;
-              if (level == L) ++leaf_pairs;
-            }
-          }
-    }
-  }
+  uint64_t p2p_pairs = 0;
   {
     const int nb = 1 << L;
     for (int64_t m = 0; m < d.leaves; ++m) {
@@ -941,6 +1039,10 @@ DevicePlan role_exchanged(const hipfmm_plan* P) {
   a.blk8_count = P->adj_blk8_count;
   a.nbr_blk_start = P->adj_nbr_blk_start;
   a.nbr_blk = P->adj_nbr_blk;
+  std::swap(a.source_bits, a.target_bits);
+  a.sparse_order = P->adj_sparse_order;
+  std::copy(P->adj_sparse.base, P->adj_sparse.base + hipfmm::kMaxLevels, a.sparse_base);
+  std::copy(P->adj_sparse.len, P->adj_sparse.len + hipfmm::kMaxLevels, a.sparse_len);
   return a;
 }
 
@@ -959,6 +1061,64 @@ void install_identity(hipfmm_plan* P, const int* self) {
   } else if (!std::equal(self, self + f.nt, P->fixed_self.begin())) {
     throw hipfmm::invalid_argument("HipFull identity map changed; rebuild the static plan");
   }
+}
+
+// The plan in harmonic-subspace form, where it has one: the operands are the
+// compressed multipoles and locals (the level scalings are in the transforms).
+DevicePlan compressed_view(const DevicePlan& d) {
+  DevicePlan c = d;
+  if (d.nc == 0 || d.L < 2) return c;
+  c.n = d.nc;
+  c.M = d.Mc;
+  c.Lc = d.Lcc;
+  c.state_major = d.compressed_state_major;
+  c.m2m_dense = d.m2m_dense_c;
+  c.l2l_dense = d.l2l_dense_c;
+  c.m2m_x3 = d.m2m_x3_c;
+  c.l2l_x3 = d.l2l_x3_c;
+  return c;
+}
+bool harmonic_passes(const DevicePlan& d) { return d.m2m_dense_c != nullptr && d.nc > 0 && d.L >= 3; }
+// Layout of the compressed coefficients (DevicePlan::compressed_state_major).
+template <class S>
+bool state_major(const DevicePlan& d, int K) {
+  return d.nc > 0 && (sizeof(S) == 8 || K % 32 != 0);
+}
+
+template <class S>
+void launch_m2l(const DevicePlan& compressed, M2lPath path, int mode, int K, hipStream_t s) {
+  switch (path) {
+    case kTileM2l: hipfmm::launch_m2l_mfma(compressed, K, mode, s); break;
+    case kDirectM2l: hipfmm::launch_m2l_bf16_direct(compressed, K, s); break;
+    case kFullM2l: hipfmm::launch_m2l_full<S>(compressed, K, s); break;
+    case kVectorM2l: hipfmm::launch_m2l_valu<S>(compressed, K, s); break;
+  }
+}
+// L2L, and the leaf level's expansion where the passes are harmonic.
+template <class S>
+void launch_downward(const DevicePlan& d, const DevicePlan& compressed, int K, hipStream_t s) {
+  const bool harmonic = harmonic_passes(d);
+  for (int level = 3; level <= d.L; ++level) hipfmm::launch_l2l<S>(harmonic ? compressed : d, level, K, s);
+  if (harmonic) hipfmm::launch_m2l_expand<S>(d, K, d.L, s);
+}
+
+// The last evaluate's locals of a box that its M2L left out (DevicePlan::
+// target_bits): the M2L and the downward pass again, over every box.
+template <class S>
+void complete_locals(hipfmm_plan* P, int node) {
+  DevicePlan d = P->last_adjoint ? role_exchanged(P) : P->d;
+  if (d.target_bits == nullptr) return;
+  uint32_t word = 0;
+  HIPFMM_CHECK(hipMemcpy(&word, d.target_bits + (node >> 5), sizeof(word), hipMemcpyDeviceToHost));
+  if ((word >> (node & 31)) & 1u) return;
+  d.source_bits = d.target_bits = nullptr;
+  d.sparse_order = nullptr;
+  d.compressed_state_major = state_major<S>(d, P->last_K);
+  const DevicePlan c = compressed_view(d);
+  launch_m2l<S>(c, P->last_path, P->last_mode, P->last_K, P->s_near);
+  if (d.nc > 0 && !harmonic_passes(d)) hipfmm::launch_m2l_expand<S>(d, P->last_K, 2, P->s_near);
+  launch_downward<S>(d, c, P->last_K, P->s_near);
+  HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
 }
 
 // One evaluate.  The near field runs on a stream of the plan's.  The rest of a
@@ -995,7 +1155,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   (void)hipGetLastError();
   ensure_capacity<S>(P, K, want_pot, want_grad);
   DevicePlan d = adjoint ? role_exchanged(P) : P->d;
-  d.compressed_state_major = d.nc > 0 && (sizeof(S) == 8 || K % 32 != 0);
+  d.compressed_state_major = state_major<S>(d, K);
   const bool host = memspace == HIPFMM_HOST;
   const hipStream_t s = host || fork != nullptr ? far_stream(P) : user;
   hipEvent_t* e = P->ev;
@@ -1081,17 +1241,9 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   mark(kEvP2M, s);
   // Harmonic passes: leaf multipoles compressed once, M2M and (below) L2L on
   // the compressed coefficients, the expansion at the leaf level only.
-  const bool harmonic = d.m2m_dense_c != nullptr && d.nc > 0 && d.L >= 3;
-  DevicePlan dc = d;
+  const bool harmonic = harmonic_passes(d);
+  const DevicePlan dc = compressed_view(d);
   if (harmonic) {
-    dc.n = d.nc;
-    dc.M = d.Mc;
-    dc.Lc = d.Lcc;
-    dc.state_major = d.compressed_state_major;
-    dc.m2m_dense = d.m2m_dense_c;
-    dc.l2l_dense = d.l2l_dense_c;
-    dc.m2m_x3 = d.m2m_x3_c;
-    dc.l2l_x3 = d.l2l_x3_c;
     hipfmm::launch_m2l_compress<S>(d, K, d.L, s);
     for (int level = d.L - 1; level >= 2; --level) hipfmm::launch_m2m<S>(dc, level, K, s);
   } else {
@@ -1122,15 +1274,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const int64_t size = d.nodes * K * d.nc;
   const bool small = d.nc > 0 && K % 32 != 0 && size <= (K < 9 ? (bf16 ? 3500000 : 1800000) : 700000);
   const bool mfma = sixteen && !small;
-  // The M2L kernels see the plan through `dm`: in harmonic-subspace form the
-  // operands are the compressed multipoles/locals (the level scalings are in
-  // the transforms).
-  DevicePlan dm = d;
   if (d.nc > 0 && d.L >= 2) {
-    dm.n = d.nc;
-    dm.M = d.Mc;
-    dm.Lc = d.Lcc;
-    dm.state_major = d.compressed_state_major;
     if (!harmonic) hipfmm::launch_m2l_compress<S>(d, K, 2, s);
     if (mfma && P->m2l_mode == HIPFMM_M2L_MFMA_FP16X3)
       hipfmm::launch_m2l_fp16_split(d, K, s);
@@ -1154,14 +1298,10 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const int ring_slot = int(P->m2l_launch_count % hipfmm_plan::kRing);
   drain_m2l_slot(P, ring_slot);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][0], s));
-  if (mfma)
-    hipfmm::launch_m2l_mfma(dm, K, P->m2l_mode, s);
-  else if (sixteen && bf16 && small)
-    hipfmm::launch_m2l_bf16_direct(dm, K, s);
-  else if (d.nc > 0)
-    hipfmm::launch_m2l_full<S>(dm, K, s);
-  else
-    hipfmm::launch_m2l_valu<S>(dm, K, s);
+  P->last_path = mfma ? kTileM2l : sixteen && bf16 && small ? kDirectM2l : d.nc > 0 ? kFullM2l : kVectorM2l;
+  P->last_mode = P->m2l_mode;
+  P->last_adjoint = adjoint;
+  launch_m2l<S>(dc, P->last_path, P->last_mode, K, s);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][1], s));
   P->m2l_ring_pending[ring_slot] = true;
   P->last_ring_slot = ring_slot;
@@ -1171,12 +1311,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     hipfmm::launch_m2l_expand<S>(d, K, 2, s);
     mark(kEvM2L, s);
   }
-  if (harmonic) {
-    for (int level = 3; level <= d.L; ++level) hipfmm::launch_l2l<S>(dc, level, K, s);
-    hipfmm::launch_m2l_expand<S>(d, K, d.L, s);
-  } else {
-    for (int level = 3; level <= d.L; ++level) hipfmm::launch_l2l<S>(d, level, K, s);
-  }
+  launch_downward<S>(d, dc, K, s);
   mark(kEvL2L, s);
   if (!after_near) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
   if (want_grad)
@@ -1540,6 +1675,8 @@ int hipfmm_plan_coefficients(hipfmm_plan* plan, int which, int node, int state, 
       std::fill(out, out + d.n, 0.0);
       return;
     }
+    if (which != 0 && d.precision == 32) complete_locals<float>(plan, node);
+    if (which != 0 && d.precision != 32) complete_locals<double>(plan, node);
     std::vector<unsigned char> buf(size_t(d.n) * K * elem);
     const void* base = which == 0 ? d.M : d.Lc;
     HIPFMM_CHECK(hipMemcpy(buf.data(), static_cast<const unsigned char*>(base) + size_t(node) * d.n * K * elem,
