@@ -18,6 +18,9 @@
 // (62-167), compression 40 (199), expansion 19 (97); FP64, 2^18 points, p = 8,
 // depth 4, L2P 59 (682), L2L 16-18 (320).  131,075 points, p = 8, 20 states:
 // P2M 103 (1870), L2P and unsort 102 (353).
+// Where many boxes hold no points, workgroups of empty boxes end at once
+// (262,144 points of a slab, p = 6, one state: compression 18 -> 8, the pass of
+// four evaluates 1218 -> 1136).
 //
 // Reference operations restated here:
 //   P2M   M_a = (-1)^|a| sum_j sum_{c: a_c>0} m_jc d_j^(a-e_c)/(a-e_c)!
@@ -84,6 +87,12 @@ struct Product {
   Strides out_at;
   int K;
   int64_t cols;
+  // Where bits is set, a workgroup none of whose boxes has a point (node bit0 +
+  // box bit_box + blockIdx.z) stores zeros, or nothing (idle_stores).
+  const uint32_t* bits;
+  int64_t bit0;
+  int bit_box;
+  bool idle_stores;
   int row_waves;  // waves side by side over the rows; blockDim / 64 / row_waves groups share the segments
   bool add;
 };
@@ -111,6 +120,13 @@ __global__ void __launch_bounds__(1024) product_kernel(const Product<S> p) {
   const int64_t first = int64_t(blockIdx.x) * (16 * CT), box0 = first / p.K;
   const uint32_t K = uint32_t(p.K), rem = uint32_t(first - box0 * p.K);
   const uint32_t left = uint32_t(min(p.cols - first, int64_t(16 * CT)));  // columns of this workgroup
+  bool idle = false;  // the same for every wave
+  if (p.bits != nullptr) {
+    const uint32_t last = (rem + left - 1) / K;  // at most 16 CT boxes
+    idle = __any(uint32_t(lane) <= last &&
+                 bit_of(p.bits, p.bit0 + (box0 + lane) * p.bit_box + int64_t(blockIdx.z))) == 0;
+    if (idle && !p.idle_stores) return;
+  }
   const S* in = p.in + box0 * p.in_box;
   S* out = p.out + box0 * p.out_box + int64_t(blockIdx.z) * p.out_z;
   uint32_t in_at[CT], out_at[CT];
@@ -131,7 +147,7 @@ __global__ void __launch_bounds__(1024) product_kernel(const Product<S> p) {
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[t][c] = typename M::Acc{};
   const int per_group = p.segments / groups;
-  const int batches = (p.D + 4 * kU - 1) / (4 * kU);
+  const int batches = idle ? 0 : (p.D + 4 * kU - 1) / (4 * kU);
   for (int g = group * per_group; g < (group + 1) * per_group; ++g) {
     const S* A = p.A + int64_t(blockIdx.z) * p.a_z + g * p.a_seg;
     const int64_t seg = g * p.in_seg;
@@ -581,6 +597,7 @@ void launch_m2m_columns(const DevicePlan& d, int parent_level, int K, hipStream_
   p.out_box = box;
   p.in_at = p.out_at = strides(d.state_major, K, n);
   p.K = K, p.cols = parents * K;
+  p.bits = d.source_bits, p.bit0 = level_offset(parent_level), p.bit_box = 1, p.idle_stores = true;
   launch_product<S>(p, 1, s);
 }
 
@@ -600,6 +617,7 @@ void launch_l2l_columns(const DevicePlan& d, int child_level, int K, hipStream_t
   p.in_at = p.out_at = strides(d.state_major, K, n);
   p.K = K, p.cols = parents * K;
   p.add = true;
+  p.bits = d.target_bits, p.bit0 = level_offset(child_level), p.bit_box = 8;
   launch_product<S>(p, 8, s);
 }
 
@@ -615,6 +633,7 @@ void launch_compress_columns(const DevicePlan& d, int level, int K, hipStream_t 
   p.out = static_cast<S*>(d.Mc) + node0 * p.out_box;
   p.in_at = strides(false, K, d.n), p.out_at = strides(d.compressed_state_major, K, d.nc);
   p.K = K, p.cols = boxes * K;
+  p.bits = d.source_bits, p.bit0 = node0, p.bit_box = 1, p.idle_stores = true;
   launch_product<S>(p, 1, s);
 }
 
@@ -630,6 +649,7 @@ void launch_expand_columns(const DevicePlan& d, int level, int K, hipStream_t s)
   p.out = static_cast<S*>(d.Lc) + node0 * p.out_box;
   p.in_at = strides(d.compressed_state_major, K, d.nc), p.out_at = strides(false, K, d.n);
   p.K = K, p.cols = boxes * K;
+  p.bits = d.target_bits, p.bit0 = node0, p.bit_box = 1;
   launch_product<S>(p, 1, s);
 }
 

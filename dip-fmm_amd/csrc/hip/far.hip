@@ -172,6 +172,11 @@ __global__ void __launch_bounds__(256) p2m_mfma_kernel(const DevicePlan d, int K
   const int leaf = blockIdx.x, kc0 = int(blockIdx.y) * kCols;
   const int2 range = d.leaf_src[leaf];
   const int64_t node = level_offset(d.L) + leaf;
+  if (range.x == range.y) {
+    float* o = static_cast<float*>(d.M) + node * int64_t(n) * K + kc0;
+    for (int w = tid; w < n * kCols; w += 256) o[int64_t(w / kCols) * K + w % kCols] = 0.0f;
+    return;
+  }
   const auto* rel = static_cast<const float4*>(d.src_rel);
   const float* sm = static_cast<const float*>(d.sm);
   int4 ex[kTW];
@@ -877,9 +882,19 @@ template <int RTW, bool kX3>
 __global__ void __launch_bounds__(256)
 box_mfma_kernel(const void* __restrict__ A, int lda, int R, int D,
                                                        const float* __restrict__ in, int64_t in_stride,
-                                                       float* __restrict__ out, int64_t out_stride, int K) {
+                                                       float* __restrict__ out, int64_t out_stride, int K,
+                                                       const uint32_t* __restrict__ bits, int64_t node0, bool zeros) {
   extern __shared__ __align__(16) float box_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
+  // A box without points: its compressed multipole is zero, its local unread
+  // (2^20 points in blobs, depth 6, 32 states: with the P2M, L2L and operand
+  // split alike 66.3 -> 61.7 ms per evaluate).
+  if (bits != nullptr && !bit_of(bits, node0 + blockIdx.x)) {
+    float* o = out + int64_t(blockIdx.x) * out_stride + int(blockIdx.y) * 32;
+    if (zeros)
+      for (int w = threadIdx.x; w < R * 32; w += 256) o[int64_t(w >> 5) * K + (w & 31)] = 0.0f;
+    return;
+  }
   const int kc0 = int(blockIdx.y) * 32, D4 = (D + 3) / 4 * 4, RT = (R + 15) / 16;
   f32x4 acc[RTW][2];
   box_mfma_zero<RTW>(acc);
@@ -944,7 +959,13 @@ l2l_mfma_kernel(const DevicePlan d, int child_level, int K) {
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int n = d.n, NP = round_up(n, 8), D4 = (n + 3) / 4 * 4, RT = (n + 15) / 16;
   const int kc0 = int(blockIdx.y) * 32;
-  const int64_t parent = blockIdx.x;
+  const int64_t parent = blockIdx.x, child0 = level_offset(child_level) + parent * 8;
+  uint32_t wanted = 0xffu;  // the children with targets
+  if (d.target_bits != nullptr) {
+    wanted = 0;
+    for (int c = 0; c < 8; ++c) wanted |= uint32_t(bit_of(d.target_bits, child0 + c)) << c;
+    if (wanted == 0) return;
+  }
   float* Lc = static_cast<float*>(d.Lc) + kc0;
   uint16_t* Bx = reinterpret_cast<uint16_t*>(box_lds);
   if constexpr (kX3)
@@ -954,7 +975,6 @@ l2l_mfma_kernel(const DevicePlan d, int child_level, int K) {
   __syncthreads();
   // The child's own local (from the M2L) is the accumulators' start, and the
   // next child's is loaded during this child's products.
-  const int64_t child0 = level_offset(child_level) + parent * 8;
   f32x4 next[RTW][2];
   box_mfma_load<RTW>(Lc + child0 * int64_t(n) * K, n, RT, K, wave, lane, next);
   for (int c = 0; c < 8; ++c) {
@@ -963,6 +983,7 @@ l2l_mfma_kernel(const DevicePlan d, int child_level, int K) {
 #pragma unroll
     for (int t = 0; t < RTW; ++t) acc[t][0] = next[t][0], acc[t][1] = next[t][1];
     if (c + 1 < 8) box_mfma_load<RTW>(Lc + (child + 1) * int64_t(n) * K, n, RT, K, wave, lane, next);
+    if (((wanted >> c) & 1u) == 0) continue;
     if constexpr (kX3)
       box_x3_tiles<RTW>(static_cast<const uint16_t*>(d.l2l_x3) + (child_level * 8 + c) * box_x3_elems(n, n), n, n,
                         Bx, wave, lane, acc);
@@ -1095,7 +1116,7 @@ void launch_m2l_compress(const DevicePlan& d, int K, int first_level, hipStream_
           const size_t l2 = box_x3_lds_bytes(d.n);
           const uint16_t* A = static_cast<const uint16_t*>(d.cmp_x3) + level * box_x3_elems(d.nc, d.n);
 #define HIPFMM_CMP(R) box_mfma_kernel<R, true><<<g2, 256, l2, s>>>(A, 0, d.nc, d.n, in, int64_t(d.n) * K, out, \
-                                                                    int64_t(d.nc) * K, K)
+                                                                    int64_t(d.nc) * K, K, d.source_bits, node0, true)
           HIPFMM_BOX_RTW(rtw, HIPFMM_CMP)
 #undef HIPFMM_CMP
         } else {
@@ -1103,7 +1124,7 @@ void launch_m2l_compress(const DevicePlan& d, int K, int first_level, hipStream_
           const int NPc = round_up(d.nc, 16);
           const float* A = static_cast<const float*>(d.cmp_op) + size_t(level) * d.n * NPc;
 #define HIPFMM_CMP(R) box_mfma_kernel<R, false><<<g2, 256, l2, s>>>(A, NPc, d.nc, d.n, in, int64_t(d.n) * K, out, \
-                                                                     int64_t(d.nc) * K, K)
+                                                                     int64_t(d.nc) * K, K, d.source_bits, node0, true)
           HIPFMM_BOX_RTW(rtw, HIPFMM_CMP)
 #undef HIPFMM_CMP
         }
@@ -1128,7 +1149,7 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
           const size_t l2 = box_x3_lds_bytes(d.nc);
           const uint16_t* A = static_cast<const uint16_t*>(d.exp_x3) + level * box_x3_elems(d.n, d.nc);
 #define HIPFMM_EXP(R) box_mfma_kernel<R, true><<<g2, 256, l2, s>>>(A, 0, d.n, d.nc, in, int64_t(d.nc) * K, out, \
-                                                                    int64_t(d.n) * K, K)
+                                                                    int64_t(d.n) * K, K, d.target_bits, node0, false)
           HIPFMM_BOX_RTW(rtw, HIPFMM_EXP)
 #undef HIPFMM_EXP
         } else {
@@ -1136,7 +1157,7 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
           const int NP = round_up(d.n, 8);
           const float* A = static_cast<const float*>(d.exp_op) + size_t(level) * d.nc * NP;
 #define HIPFMM_EXP(R) box_mfma_kernel<R, false><<<g2, 256, l2, s>>>(A, NP, d.n, d.nc, in, int64_t(d.nc) * K, out, \
-                                                                     int64_t(d.n) * K, K)
+                                                                     int64_t(d.n) * K, K, d.target_bits, node0, false)
           HIPFMM_BOX_RTW(rtw, HIPFMM_EXP)
 #undef HIPFMM_EXP
         }

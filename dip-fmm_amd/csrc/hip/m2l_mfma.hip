@@ -745,9 +745,10 @@ __global__ void __launch_bounds__(256) level_max_kernel(const DevicePlan d, int 
 // FP16 hi/lo split of 2^e_l Mc / sigma into the MFMA B layout
 // mt[node][ks][KO][16] (KO >= K columns, zeros from K on); each thread packs 8
 // consecutive coefficients of one column (16-byte stores).
-__global__ void __launch_bounds__(256) split_f16_kernel(const DevicePlan d, int K, int KO) {
+__global__ void __launch_bounds__(256) split_f16_kernel(const DevicePlan d, int K, int KO, const uint32_t* bits) {
   const int nc = d.nc, AP = d.apad, KS = AP / 16;
   const int64_t node = level_offset(2) + blockIdx.x;
+  if (bits != nullptr && !bit_of(bits, node)) return;
   const int level = level_of_node(node);
   const float scale = ldexpf(1.0f, fp16_level_exponent(d.lvl_max_bits[level]));
   const float* Mc = static_cast<const float*>(d.Mc) + node * int64_t(nc) * K;
@@ -773,9 +774,10 @@ __global__ void __launch_bounds__(256) split_f16_kernel(const DevicePlan d, int 
 // bf16 hi/lo split of Mc into the MFMA B layout mt[node][ks][KO][16] (levels
 // 2..L, KO as above); each thread packs 8 consecutive coefficients of one
 // column.
-__global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int K, int KO) {
+__global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int K, int KO, const uint32_t* bits) {
   const int nc = d.nc, AP = d.apad, KS = AP / 16;
   const int64_t node = level_offset(2) + blockIdx.x;
+  if (bits != nullptr && !bit_of(bits, node)) return;
   const float* Mc = static_cast<const float*>(d.Mc) + node * int64_t(nc) * K;
   const int row = d.compressed_state_major ? 1 : K, state = d.compressed_state_major ? nc : 1;
   for (int w = threadIdx.x; w < KO * (AP / 8); w += blockDim.x) {
@@ -806,10 +808,17 @@ int m2l_operand_states(const DevicePlan& d, int K) {
   return d.nc == 0 || K < 9 ? K : (K + 31) / 32 * 32;
 }
 
+// The boxes whose operands the tiles read: of one box per tile, those with
+// sources (holds_sources); of several, all.
+static const uint32_t* split_bits(const DevicePlan& d, int KO) {
+  return uniform_box(d, KO) ? d.source_bits : nullptr;
+}
+
 void launch_m2l_bf16_split(const DevicePlan& d, int K, hipStream_t s) {
   if (d.L < 2) return;
   const unsigned boxes = unsigned(d.nodes - level_offset(2));
-  split_bf16_kernel<<<boxes, 256, 0, s>>>(d, K, m2l_operand_states(d, K));
+  const int KO = m2l_operand_states(d, K);
+  split_bf16_kernel<<<boxes, 256, 0, s>>>(d, K, KO, split_bits(d, KO));
   HIPFMM_CHECK(hipGetLastError());
 }
 
@@ -819,7 +828,8 @@ void launch_m2l_fp16_split(const DevicePlan& d, int K, hipStream_t s) {
   launch_zero<float>(reinterpret_cast<float*>(d.lvl_max_bits), size_t(d.L + 1), s);
   level_max_kernel<<<boxes, 256, 0, s>>>(d, K);
   HIPFMM_CHECK(hipGetLastError());
-  split_f16_kernel<<<boxes, 256, 0, s>>>(d, K, m2l_operand_states(d, K));
+  const int KO = m2l_operand_states(d, K);
+  split_f16_kernel<<<boxes, 256, 0, s>>>(d, K, KO, split_bits(d, KO));
   HIPFMM_CHECK(hipGetLastError());
 }
 

@@ -1111,7 +1111,7 @@ void complete_locals(hipfmm_plan* P, int node) {
   uint32_t word = 0;
   HIPFMM_CHECK(hipMemcpy(&word, d.target_bits + (node >> 5), sizeof(word), hipMemcpyDeviceToHost));
   if ((word >> (node & 31)) & 1u) return;
-  d.source_bits = d.target_bits = nullptr;
+  d.target_bits = nullptr;
   d.sparse_order = nullptr;
   d.compressed_state_major = state_major<S>(d, P->last_K);
   const DevicePlan c = compressed_view(d);
