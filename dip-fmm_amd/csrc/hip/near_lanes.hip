@@ -10,8 +10,8 @@
 // D = (3 r r^T/|r|^5 - I/|r|^3)/(4 pi) of src/cuboid.cpp:293-307 and the
 // potential (m.r)/(4 pi |r|^3) of src/static_operators.cpp:455-463.
 //
-// What bounds it: the pair arithmetic, 33 vector instructions per pair and
-// state at one state (25 for the geometry, 10 per further state).  So the
+// What bounds it: the pair arithmetic, 33 vector instructions per pair at
+// one state (24 for the geometry, 9 per state, 10 with the potential).  So the
 // lanes of a wave are sources and its targets are wave-uniform: a lane keeps
 // one source and its moments in registers for T targets of one leaf, whose
 // coordinates sit in scalar registers, and nothing is staged in LDS.  A batch
@@ -32,7 +32,10 @@
 // leaf, FP32: K = 1 .88 (1.77), 2 1.08 (2.70), 4 1.87 (4.61), 8 3.06 (8.01);
 // fields and potentials K = 4 2.08 (4.72); gradients K = 1 1.25 (2.05).
 // 512 per leaf, 2^18 points: K = 8 6.5.  FP64, 2^18 points, 64 per leaf:
-// K = 1 .60 (1.43).
+// K = 1 .60 (1.43).  With sqrt(3) in the unit vector (whole evaluates of 2^20
+// points, p = 4; before: the 3 and the potential's r.m once per state): K = 8
+// 3.94 (4.02), with potentials 4.63 (5.09); 512 per leaf, 2^18 points, K = 8
+// 6.24 (6.51), with potentials 8.07 (9.07).
 #include "common.hpp"
 
 namespace hipfmm {
@@ -222,10 +225,10 @@ __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePla
       const S rx = tp[i].minus(sp, 0), ry = tp[i].minus(sp, 1), rz = tp[i].minus(sp, 2);
       const S r2 = rx * rx + ry * ry + rz * rz;
       const S rinv = near_rsqrt(r2);
-      const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
       S* a = acc + i * C * KS;
       if constexpr (kWhat == kGradient) {
         // dH_c/dx_j, 3/(4 pi |r|^4) (delta_cj w + u_c m_j + m_c u_j - 5 u_c u_j w), w = u.m.
+        const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
         const S g = S(0.23873241463784300365332564505877154) * rinv * rinv * rinv * rinv;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
@@ -240,18 +243,22 @@ __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePla
           a[5 * KS + k] += g * (w + S(2) * uz * mz - w5 * uz * uz);
         }
       } else {
-        // f (3 (u.m) u - m) with f = |r|^-3 / (4 pi) avoids the |r|^-5
-        // overflow of close pairs in FP32.
-        const S f = rinv * rinv * rinv * S(0.079577471545947667884441881686257181);
+        // f ((v.m) v - m) with f = |r|^-3 / (4 pi) and v = sqrt(3) u: no |r|^-5,
+        // which overflows for close pairs in FP32, and the 3 costs a pair one
+        // instruction instead of one per state.  The potential f r.m is
+        // f / (sqrt(3) / |r|) v.m.
+        const S vinv = S(1.7320508075688772935274463415058724) * rinv;
+        const S vx = rx * vinv, vy = ry * vinv, vz = rz * vinv;
+        const S rinv2 = rinv * rinv, f = rinv2 * rinv * S(0.079577471545947667884441881686257181);
+        const S fp = rinv2 * S(0.045944074618482676297581119891486868);  // 1 / (4 pi sqrt 3)
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
           const S mx = m[0][k], my = m[1][k], mz = m[2][k];
-          const S w = ux * mx + uy * my + uz * mz, w3 = S(3) * w;
-          a[0 * KS + k] += f * (w3 * ux - mx);
-          a[1 * KS + k] += f * (w3 * uy - my);
-          a[2 * KS + k] += f * (w3 * uz - mz);
-          if constexpr (kWhat == kFieldAndPotential)
-            a[3 * KS + k] += f * (rx * mx + ry * my + rz * mz);
+          const S w = vx * mx + vy * my + vz * mz;
+          a[0 * KS + k] += f * (w * vx - mx);
+          a[1 * KS + k] += f * (w * vy - my);
+          a[2 * KS + k] += f * (w * vz - mz);
+          if constexpr (kWhat == kFieldAndPotential) a[3 * KS + k] += fp * w;
         }
       }
     }
