@@ -766,10 +766,11 @@ void create_impl(hipfmm_plan* P, const hipfmm_plan_desc& desc) {
   // less there.
   // Where a tenth or more of the list-2 pairs have a box without points, the
   // M2L takes boxes with targets only, and sources with points only: 2^20
-  // points in blobs, depth 6, 32 states, M2L 52.6 -> 35.9 ms; 262,144 points of a slab
-  // seen from a plane, depth 5, one state, 296 -> 46 us.  Below that line the empty
-  // boxes are scattered singly, and the lists and bits would save less than
-  // their lookups cost.
+  // points in blobs, depth 6, 32 states (63% of the pairs), M2L 52.6 -> 35.9
+  // ms; 262,144 points of a slab seen from a plane, depth 5, one state (all but
+  // a few), 296 -> 46 us.  The line keeps trees of uniform points on the full
+  // order: at 5 points per leaf under 2% of their pairs have an empty side, in
+  // boxes scattered singly, which saves no tile and few steps.
   const auto occupied = [&](int level, int64_t m, bool sources) {
     const int64_t* r = ranges + 4 * (hipfmm::level_offset(level) + m) + (sources ? 0 : 2);
     return r[1] > r[0];
