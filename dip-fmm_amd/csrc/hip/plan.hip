@@ -1122,6 +1122,21 @@ void complete_locals(hipfmm_plan* P, int node) {
   HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
 }
 
+// Kernels of an evaluate that failed half-way, which no event marks: they end
+// before the error is reported, so that the next evaluate finds the plan's
+// buffers free whatever stream it runs on.  (Not within a capture, where nothing
+// runs yet.)
+struct SettleOnFailure {
+  hipStream_t far, near;
+  bool armed;
+  ~SettleOnFailure() {
+    if (!armed) return;
+    (void)hipStreamSynchronize(far);
+    (void)hipStreamSynchronize(near);
+    (void)hipGetLastError();
+  }
+};
+
 // One evaluate.  The near field runs on a stream of the plan's.  The rest of a
 // device-resident evaluate runs on the caller's stream `user`, which then needs
 // no fork and no join (1,000 points, p = 4, depth 2: 97 us per evaluate, with
@@ -1170,6 +1185,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const bool captured = capture != hipStreamCaptureStatusNone;
   if (captured ? P->capture_id == capture_id : P->done_recorded)
     HIPFMM_CHECK(hipStreamWaitEvent(s, e[captured ? kEvCaptured : kEvL2P], 0));
+  SettleOnFailure settle{s, P->s_near, !captured};
   auto mark = [&](int ev, hipStream_t on) {
     HIPFMM_CHECK(hipEventRecord(e[ev], on));
   };
@@ -1341,6 +1357,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
     if (grad_bytes) std::memcpy(field_gradients, P->pinned_grad, grad_bytes);
     finalize_timings(P);
   }
+  settle.armed = false;
 }
 
 }  // namespace
