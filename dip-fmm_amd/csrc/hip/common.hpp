@@ -304,8 +304,9 @@ std::vector<double> m2l_fragments_f64(int n, const std::vector<double>& C, int c
 int4 m2l_step(int ox, int oy, int oz, int cls);
 template <class S>
 void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s);
-// State counts from which FP32 batches that are no multiple of 32 take the
-// matrix cores (near.hip): fields with and without potentials, and gradients.
+// State counts from which FP32 batches that are no multiple of 32 may take the
+// matrix cores (near.hip gives the whole rule): fields with and without
+// potentials, and gradients.
 constexpr int kNearBf16States = 9, kNearGradBf16States = 7;
 // The vector-ALU near field (near_lanes.hip): any K, FP32 and FP64.
 template <class S>

@@ -659,18 +659,44 @@ p2p_bf16_kernel(const DevicePlan d, const int2* __restrict__ tiles, int tile_cou
   }
 }
 
-// Batches that are no multiple of 32 take the bf16 kernels from the state count
-// at which a whole 32-state (or 16-state) tile costs less than the vector ALUs'
-// pass per group of states (the near-field variants choose among the kernels of
-// the multiples of 32).  Near field alone, ms, vector ALUs / bf16 tiles:
-//   fields, 2^20 points, 32 per leaf: K = 8 3.06 / 3.39, 9 4.45 / 3.38,
-//     16 6.44 / 3.58, 31 13.7 / 5.1; 512 per leaf, 2^18 points: K = 8 6.5 / 7.5,
-//     9 10.4 / 7.6; 20,000 points: K = 8 .074 / .123, 9 .097 / .124;
-//   fields and potentials, 2^20 points: K = 8 4.07 / 4.12, 9 5.24 / 4.1;
-//   gradients, 2^20 points: K = 6 5.6 / 5.2, 7 6.85 / 5.3; 20,000 points:
-//     K = 6 .114 / .17, 8 .139 / .17.
-static bool near_on_matrix_cores(int K, bool gradient) {
-  return K >= (gradient ? kNearGradBf16States : kNearBf16States);
+// State tiles of 32, and a last one of 16 where at most 16 states are left:
+// launch(halves, first tile, tiles).
+template <class F>
+void for_state_tiles(int K, F&& launch) {
+  const int rest = K % 32, whole = K / 32 + (rest > 16 ? 1 : 0);
+  if (whole > 0) launch(std::integral_constant<int, 2>{}, 0, whole);
+  if (rest > 0 && rest <= 16) launch(std::integral_constant<int, 1>{}, K / 32, 1);
+  HIPFMM_CHECK(hipGetLastError());
+}
+
+// Batches that are no multiple of 32 take the bf16 kernels where a 32-state
+// (or 16-state) tile costs less than the vector ALUs' passes per group of states
+// (the near-field variants choose among the kernels of the multiples of 32).
+//   * From 9 states on (gradients: 7).  Near field alone, ms, vector ALUs / bf16
+//     tiles: fields, 2^20 points, 32 per leaf: K = 8 2.59 / 3.00, 9 3.92 / 3.04,
+//     16 5.51 / 3.19, 31 12.6 / 4.8; fields and potentials: K = 8 3.20 / 3.68,
+//     9 4.12 / 3.69; gradients: K = 6 5.6 / 5.2, 7 6.19 / 4.88.
+//   * Where the tiles fill the chip: a wave of 16 targets and 32 states is one
+//     long chain, so a launch of few takes a wave's time however many states it
+//     holds, and the vector ALUs' shorter waves end sooner.  The line is at
+//     target tiles x states per launch (33 to 48 states are two).  Whole
+//     evaluates, p = 2, ms, vector ALUs / bf16 tiles:
+//       fields: K = 9 2792 tiles .368 / .359, 1256 .147 / .180; 16 2792
+//         .477 / .376, 1256 .182 / .198; 24 1256 .238 / .236, 523 .131 / .147;
+//         40 2792 1.18 / .78, 1256 .325 / .352;
+//       fields and potentials: K = 9 4186 .229 / .243, 10054 .639 / .616; 16 2792
+//         .656 / .446, 523 .126 / .135; 31 1031 1.74 / .78, 523 .174 / .174;
+//       gradients: K = 8 2792 .524 / .536, 1256 .181 / .215; 16 1256 .294 / .245,
+//         523 .143 / .144; 33 1031 1.97 / 1.69, 523 .210 / .228.
+//     Over 64 to 32,768 leaves of 10 to 250 points and 9 to 63 states the line
+//     is within .1% of the faster kernel on average (potentials .4%), bf16 tiles
+//     alone 9 to 12%.
+// rows: outputs per target and state (3, with the potential 4, gradient 6).
+static bool near_on_matrix_cores(const DevicePlan& d, int K, int rows) {
+  int launches = 0;
+  for_state_tiles(K, [&](auto, int, int) { ++launches; });
+  const int64_t line = rows == 3 ? 26000 : rows == 4 ? 16000 : 14000;
+  return K >= (rows == 6 ? kNearGradBf16States : kNearBf16States) && int64_t(d.p2p_tile16_count) * K >= line * launches;
 }
 
 // The moments' bf16 pieces for the near-field kernels on bf16 operands.
@@ -681,16 +707,6 @@ void launch_split_moments(const DevicePlan& d, int K, hipStream_t s) {
   const int KP = (K + 31) / 32 * 32;
   const int64_t threads = int64_t(d.blk8_count) * KP;
   split_moments_kernel<<<unsigned((threads + 255) / 256), 256, 0, s>>>(d, K, KP);
-  HIPFMM_CHECK(hipGetLastError());
-}
-
-// State tiles of 32, and a last one of 16 where at most 16 states are left:
-// launch(halves, first tile, tiles).
-template <class F>
-void for_state_tiles(int K, F&& launch) {
-  const int rest = K % 32, whole = K / 32 + (rest > 16 ? 1 : 0);
-  if (whole > 0) launch(std::integral_constant<int, 2>{}, 0, whole);
-  if (rest > 0 && rest <= 16) launch(std::integral_constant<int, 1>{}, K / 32, 1);
   HIPFMM_CHECK(hipGetLastError());
 }
 
@@ -720,7 +736,7 @@ void launch_p2p(const DevicePlan& d, int K, bool potential, hipStream_t s) {
   if (d.leaves == 0 || d.nt == 0) return;
   if (potential && d.Pn == nullptr) throw invalid_argument("near-field potential buffer is not allocated");
   if constexpr (sizeof(S) == 4) {
-    if (K % 32 == 0 ? d.p2p_variant == 4 || d.p2p_variant == 0 : near_on_matrix_cores(K, false)) {
+    if (K % 32 == 0 ? d.p2p_variant == 4 || d.p2p_variant == 0 : near_on_matrix_cores(d, K, potential ? 4 : 3)) {
       launch_p2p_bf16(d, K, potential, s);
       return;
     }
@@ -994,7 +1010,7 @@ void launch_p2p_grad(const DevicePlan& d, int K, hipStream_t s) {
   if constexpr (sizeof(S) == 4) {
     const int count = d.p2p_tile16_count;
     const unsigned blocks = unsigned((count + kP2PWaves - 1) / kP2PWaves);
-    if (count > 0 && (K % 32 == 0 ? d.p2p_variant == 0 || d.p2p_variant == 4 : near_on_matrix_cores(K, true))) {
+    if (count > 0 && (K % 32 == 0 ? d.p2p_variant == 0 || d.p2p_variant == 4 : near_on_matrix_cores(d, K, 6))) {
       launch_split_moments(d, K, s);
       for_state_tiles(K, [&](auto halves, int tile0, int tiles) {
         constexpr int H = decltype(halves)::value;
