@@ -395,6 +395,14 @@ __global__ void __launch_bounds__(64 * kP2PWaves) p2p_mfma16_kernel(const Device
 // wave's 18 operand loads of one block then sit at fixed offsets from one
 // address.  Thread = (block, state of the KP = 32-padded tiles); reads are
 // coalesced over the states, writes are 16-byte rows.
+// The low pieces of a value x reach down to 2^-23 |x|, and below 2^-126 they
+// lose bits.  So in batches that are no multiple of 32, whose sums are repaired
+// where they are not finite (p2p_repair), the moments of a block and state
+// that are all below 2^-100 (not all zero) enter as NaN: the sums they take part
+// in are formed again in FP32, one pair at a time.  A block with a larger
+// moment loses at most 2^-26 of it.
+constexpr float kSmallestSplitMoment = 0x1p-100f;
+
 __global__ void __launch_bounds__(256) split_moments_kernel(const DevicePlan d, int K, int KP) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= int64_t(d.blk8_count) * KP) return;
@@ -402,13 +410,19 @@ __global__ void __launch_bounds__(256) split_moments_kernel(const DevicePlan d, 
   const int2 bs = d.blk8_src[b];
   const float* sm = static_cast<const float*>(d.sm);
   uint4* out = static_cast<uint4*>(d.smb) + ((int64_t(b) * (KP / 32) + k / 32) * 9) * 32 + k % 32;
+  float x[3][8], most = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[c][e] = e < bs.y && k < K ? sm[(int64_t(bs.x + e) * 3 + c) * K + k] : 0.0f;
+      most = fmaxf(most, fabsf(x[c][e]));
+    }
+  if (K != KP && most > 0.0f && most < kSmallestSplitMoment) x[0][0] = __builtin_nanf("");
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = e < bs.y && k < K ? sm[(int64_t(bs.x + e) * 3 + c) * K + k] : 0.0f;
     uint4 h, m, l;
-    split3_bf16(x, h, m, l);
+    split3_bf16(x[c], h, m, l);
     out[(3 * c) * 32] = h;
     out[(3 * c + 1) * 32] = m;
     out[(3 * c + 2) * 32] = l;
@@ -440,7 +454,9 @@ __device__ __forceinline__ void p2p_bf16_products(f32x4 (&part)[kH], const uint4
 // them is not finite (rare): those of that lane's target and state again, one
 // pair at a time.  In the products a source that is left out (a target's own,
 // a padding slot) has weight zero, and zero times a moment that is not finite
-// is NaN; here it is left out.  kRows: 3 the field, 4 with the potential, 6 the
+// is NaN; here it is left out.  Pairs closer than 3e-8 of the box, whose |r|^-5
+// overflows in the products, and moments too small for the products' pieces
+// (split_moments_kernel) come here too.  kRows: 3 the field, 4 with the potential, 6 the
 // gradient; acc[c][h][i] is row c of state k0 + 16 h, target t0 + i.
 template <int kRows, int kH>
 __device__ __forceinline__ void p2p_repair(const DevicePlan& d, f32x4 (&acc)[kRows][kH], int leaf, int t0, int cnt,
