@@ -1086,6 +1086,35 @@ bool state_major(const DevicePlan& d, int K) {
   return d.nc > 0 && (sizeof(S) == 8 || K % 32 != 0);
 }
 
+// The M2L kernel of a batch of K states.
+//
+// The 16-bit modes split the multipoles in a pass of their own and run in
+// workgroups of 256 columns whose chain of up to 189 offsets takes 0.23-0.6
+// ms however few there are.  A small batch runs on the direct kernels
+// instead, whose waves share the offsets and which need no split: the bf16
+// mode in its own arithmetic, the FP16 mode in full FP32 (24 bits per
+// operand against 22, and no pass over the level maxima).  The line is at
+// the batch's size in boxes x states x coefficients.  Whole evaluates (ms,
+// workgroups of 256 / direct), bf16: p = 8, 4681 boxes 0.92 / 0.49 at K = 1,
+// 1.24 / 1.06 at 6, 1.32 / 1.26 at 8 (3.0e6); 37449 boxes 2.07 / 1.96 at
+// K = 1 (3.0e6), 2.92 / 3.04 at 2; p = 6 1.49 / 1.40 at 1, 2.03 / 2.00 at 2
+// (3.7e6), 2.58 / 2.80 at 3.  FP16: p = 8, 4681 boxes 1.12 / 1.06 at K = 4,
+// 1.24 / 1.36 at 6 (2.3e6); p = 6 0.82 / 0.76 at 6, 0.86 / 0.89 at 8 (1.8e6).
+// From 9 states on the operands are padded to whole 32-column boxes (see
+// m2l_operand_states) and the line is lower: bf16 p = 6, 585 boxes
+// 0.48 / 0.45 at K = 24 (6.9e5), 0.55 / 0.58 at 31.
+template <class S>
+M2lPath m2l_path(const hipfmm_plan* P, int K) {
+  const DevicePlan& d = P->d;
+  const bool sixteen = sizeof(S) == 4 && P->m2l_mode != HIPFMM_M2L_VALU && P->mfma_ready;
+  const bool bf16 = P->m2l_mode == HIPFMM_M2L_MFMA_BF16X3;
+  const int64_t size = d.nodes * K * d.nc;
+  const bool small = d.nc > 0 && K % 32 != 0 && size <= (K < 9 ? (bf16 ? 3500000 : 1800000) : 700000);
+  if (sixteen && !small) return kTileM2l;
+  if (sixteen && bf16) return kDirectM2l;
+  return d.nc > 0 ? kFullM2l : kVectorM2l;
+}
+
 template <class S>
 void launch_m2l(const DevicePlan& compressed, M2lPath path, int mode, int K, hipStream_t s) {
   switch (path) {
@@ -1271,26 +1300,8 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   // them here.
   if (d.L < 2) hipfmm::launch_zero<S>(static_cast<S*>(d.Lc), size_t(d.nodes) * d.n * K, s);
   mark(kEvM2M, s);
-  // The 16-bit modes split the multipoles in a pass of their own and run in
-  // workgroups of 256 columns whose chain of up to 189 offsets takes 0.23-0.6
-  // ms however few there are.  A small batch runs on the direct kernels
-  // instead, whose waves share the offsets and which need no split: the bf16
-  // mode in its own arithmetic, the FP16 mode in full FP32 (24 bits per
-  // operand against 22, and no pass over the level maxima).  The line is at
-  // the batch's size in boxes x states x coefficients.  Whole evaluates (ms,
-  // workgroups of 256 / direct), bf16: p = 8, 4681 boxes 0.92 / 0.49 at K = 1,
-  // 1.24 / 1.06 at 6, 1.32 / 1.26 at 8 (3.0e6); 37449 boxes 2.07 / 1.96 at
-  // K = 1 (3.0e6), 2.92 / 3.04 at 2; p = 6 1.49 / 1.40 at 1, 2.03 / 2.00 at 2
-  // (3.7e6), 2.58 / 2.80 at 3.  FP16: p = 8, 4681 boxes 1.12 / 1.06 at K = 4,
-  // 1.24 / 1.36 at 6 (2.3e6); p = 6 0.82 / 0.76 at 6, 0.86 / 0.89 at 8 (1.8e6).
-  // From 9 states on the operands are padded to whole 32-column boxes (see
-  // m2l_operand_states) and the line is lower: bf16 p = 6, 585 boxes
-  // 0.48 / 0.45 at K = 24 (6.9e5), 0.55 / 0.58 at 31.
-  const bool sixteen = sizeof(S) == 4 && P->m2l_mode != HIPFMM_M2L_VALU && P->mfma_ready;
-  const bool bf16 = P->m2l_mode == HIPFMM_M2L_MFMA_BF16X3;
-  const int64_t size = d.nodes * K * d.nc;
-  const bool small = d.nc > 0 && K % 32 != 0 && size <= (K < 9 ? (bf16 ? 3500000 : 1800000) : 700000);
-  const bool mfma = sixteen && !small;
+  const M2lPath path = m2l_path<S>(P, K);
+  const bool mfma = path == kTileM2l;
   if (d.nc > 0 && d.L >= 2) {
     if (!harmonic) hipfmm::launch_m2l_compress<S>(d, K, 2, s);
     if (mfma && P->m2l_mode == HIPFMM_M2L_MFMA_FP16X3)
@@ -1315,10 +1326,10 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const int ring_slot = int(P->m2l_launch_count % hipfmm_plan::kRing);
   drain_m2l_slot(P, ring_slot);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][0], s));
-  P->last_path = mfma ? kTileM2l : sixteen && bf16 && small ? kDirectM2l : d.nc > 0 ? kFullM2l : kVectorM2l;
+  P->last_path = path;
   P->last_mode = P->m2l_mode;
   P->last_adjoint = adjoint;
-  launch_m2l<S>(dc, P->last_path, P->last_mode, K, s);
+  launch_m2l<S>(dc, path, P->last_mode, K, s);
   HIPFMM_CHECK(hipEventRecord(P->m2l_ring[ring_slot][1], s));
   P->m2l_ring_pending[ring_slot] = true;
   P->last_ring_slot = ring_slot;
@@ -1627,8 +1638,9 @@ int hipfmm_plan_autotune(hipfmm_plan* plan, int batch) {
       set(best);
       return best;
     };
-    const bool mfma = P->d.precision == 32 && P->m2l_mode != HIPFMM_M2L_VALU && P->mfma_ready && P->d.L >= 2;
-    if (mfma && P->d.bpad / 32 <= 3) {
+    // The tile shapes matter where this batch runs on them.
+    const bool tiles = P->d.precision == 32 && m2l_path<float>(P, batch) == kTileM2l;
+    if (tiles && P->d.bpad / 32 <= 3) {
       std::vector<int> shapes(std::begin(hipfmm::kM2LShapes), std::end(hipfmm::kM2LShapes));
       best_of([&](int c) { P->d.m2l_shape = c; }, shapes, [&] { return P->timings.m2l_kernel_seconds; });
     }

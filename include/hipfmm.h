@@ -49,7 +49,10 @@ enum hipfmm_memspace { HIPFMM_HOST = 0, HIPFMM_DEVICE = 1 };
 /* M2L arithmetic.  VALU is the plain path (FP32 plans: FP32 FMA; FP64 plans:
  * FP64 FMA).  The MFMA modes exist for FP32 plans only: operands are split
  * into two 16-bit halves (hi + lo) and three products are accumulated in FP32
- * on the matrix cores. */
+ * on the matrix cores.  A small batch that is no multiple of 32 states does not
+ * pay for the split: up to 3.5e6 boxes x states x (p+1)^2 with 8 or fewer
+ * states (FP16 1.8e6), 7e5 with more, the bf16 mode forms the same products
+ * without a pass of its own for it and the FP16 mode runs as VALU does. */
 enum hipfmm_m2l_mode {
   HIPFMM_M2L_VALU = 0,
   HIPFMM_M2L_MFMA_BF16X3 = 1,
@@ -269,9 +272,10 @@ int hipfmm_plan_set_m2l_mode(hipfmm_plan* plan, int mode);
 /* Launch autotuner; no counterpart in the reference (whose CudaFull launch
  * shapes are fixed, src/cuda_fmm.cu:3500-3600).  Times, on the plan's own
  * state buffers at `batch` states and the current M2L mode, every tile shape
- * of the matrix-core M2L (by its kernel time) and the four near-field kernels
- * (FP32 plans, batch a multiple of 32; by the whole evaluate, since the near
- * field overlaps the far chain), keeps the fastest of each for later
+ * of the 16-bit modes' tiled M2L (by its kernel time, where the batch runs on
+ * it: see hipfmm_m2l_mode) and the four near-field kernels (FP32 plans, batch
+ * a multiple of 32; by the whole evaluate, since the near field overlaps the
+ * far chain), keeps the fastest of each for later
  * evaluates of this plan and reports them in hipfmm_stats.  Results are unchanged in value
  * class: every candidate meets the same accuracy bars.  Overwrites the
  * plan's coefficients of the last evaluate. */
