@@ -1311,17 +1311,26 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   } else if (mfma) {
     hipfmm::launch_m2l_split(d, K, P->m2l_mode, s);
   }
-  // From K = 32 on, the matrix-core M2L starts once the near field is done,
-  // and the vector-ALU M2L always does.  Both kernels then fill the chip and
-  // are bound by instruction issue, so one after the other they take as long
-  // as side by side (measured within noise), and the M2L runs alone; the
-  // upward pass before this point still runs beside the near field.  The
-  // vector-ALU M2L's few, long workgroups must start on an empty chip: placed
-  // around the near field's last workgroups they crowd some CUs (2^20 points,
-  // p = 6, one state: M2L 2.04 ms beside the near field's tail, 1.24 ms after
-  // it).  A smaller matrix-core batch has too few workgroups to fill the chip
-  // and keeps running beside the near field.
-  const bool after_near = !mfma || K >= 32;
+  // Which M2L starts once the near field is done, and which beside it (whole
+  // evaluates, ms, after / beside; the upward pass before this point always runs
+  // beside the near field).
+  //   * The tiles from K = 32 on, after: both kernels then fill the chip and are
+  //     bound by instruction issue, one after the other takes as long (2^20
+  //     points, depth 5, K = 32: p = 8 14.48 / 14.49, p = 4 6.88 / 7.07), and the
+  //     M2L runs alone.  A smaller batch is too few workgroups to fill it, beside
+  //     (131,072 points, depth 4, p = 4: K = 12 .678 / .630, 31 1.009 / .935).
+  //   * The direct and the full-precision kernels on a small tree (585 boxes and
+  //     fewer), beside: 1024 points, depth 2, p = 4: K = 1 .076 / .067, 20
+  //     .136 / .109; 32,768 points, depth 3: p = 4 K = 1 .123 / .101, FP64 K = 4
+  //     .223 / .191, p = 8 K = 20 .760 / .661; nowhere slower with fewer than 32
+  //     states.
+  //   * On a larger one, after.  Beside it most gain (131,072 points, depth 4,
+  //     p = 4, bf16: K = 4 .405 / .322, 8 .565 / .493; K = 1 and 2 0 to 2%), but
+  //     where a launch is one to three workgroups per CU those placed around the
+  //     near field's last ones crowd some CUs: 65,536 points, K = 7, p = 7 bf16
+  //     .537 / .643, FP32 .880 / .938; 180,000 points, p = 8, bf16 K = 3
+  //     .576 / .661, 4 .781 / .837.
+  const bool after_near = K >= 32 || (!mfma && d.nodes > hipfmm::level_offset(4));
   if (after_near) HIPFMM_CHECK(hipStreamWaitEvent(s, e[kEvNear1], 0));
   const int ring_slot = int(P->m2l_launch_count % hipfmm_plan::kRing);
   drain_m2l_slot(P, ring_slot);
