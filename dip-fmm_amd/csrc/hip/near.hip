@@ -692,27 +692,27 @@ void for_state_tiles(int K, F&& launch) {
 //     tiles: fields, 2^20 points, 32 per leaf: K = 8 2.59 / 3.00, 9 3.92 / 3.04,
 //     16 5.51 / 3.19, 31 12.6 / 4.8; fields and potentials: K = 8 3.20 / 3.68,
 //     9 4.12 / 3.69; gradients: K = 6 5.6 / 5.2, 7 6.19 / 4.88.
-//   * Where the tiles fill the chip: a wave of 16 targets and 32 states is one
-//     long chain, so a launch of few takes a wave's time however many states it
-//     holds, and the vector ALUs' shorter waves end sooner.  The line is at
-//     target tiles x states per launch (33 to 48 states are two).  Whole
-//     evaluates, p = 2, ms, vector ALUs / bf16 tiles:
-//       fields: K = 9 2792 tiles .368 / .359, 1256 .147 / .180; 16 2792
-//         .477 / .376, 1256 .182 / .198; 24 1256 .238 / .236, 523 .131 / .147;
-//         40 2792 1.18 / .78, 1256 .325 / .352;
-//       fields and potentials: K = 9 4186 .229 / .243, 10054 .639 / .616; 16 2792
-//         .656 / .446, 523 .126 / .135; 31 1031 1.74 / .78, 523 .174 / .174;
-//       gradients: K = 8 2792 .524 / .536, 1256 .181 / .215; 16 1256 .294 / .245,
-//         523 .143 / .144; 33 1031 1.97 / 1.69, 523 .210 / .228.
-//     Over 64 to 32,768 leaves of 10 to 250 points and 9 to 63 states the line
-//     is within .1% of the faster kernel on average (potentials .4%), bf16 tiles
-//     alone 9 to 12%.
+//   * On trees of 64 leaves and fewer, where the tiles fill the chip: a
+//     neighbourhood there is a good part of all points, so a wave of 16 targets
+//     and 32 states is one long chain, a launch of few takes a wave's time
+//     however many states it holds, and the vector ALUs' shorter waves end
+//     sooner.  The line is at target tiles x states per launch (33 to 48 states
+//     are two).  Whole evaluates, 64 leaves, p = 6, bf16 M2L, ms, vector ALUs /
+//     bf16 tiles, fields: 154 tiles K = 9 .101 / .123, 30 .126 / .166, 40
+//     .145 / .275; 508 tiles K = 9 .157 / .282, 30 .315 / .372, 50 .552 / .425;
+//     1033 tiles K = 20 .614 / .673, 30 .906 / .689.  p = 4 to 8, 10 to 250 points
+//     per leaf, 7 to 63 states: the line is within .3% of the faster kernel on
+//     average, bf16 tiles alone 18 to 25%.  With 512 leaves and more the tiles
+//     alone are within .7% (9728 points, 871 tiles: K = 9 .151 / .145, 30
+//     .406 / .326).
 // rows: outputs per target and state (3, with the potential 4, gradient 6).
 static bool near_on_matrix_cores(const DevicePlan& d, int K, int rows) {
+  if (K < (rows == 6 ? kNearGradBf16States : kNearBf16States)) return false;
+  if (d.leaves > 64) return true;
   int launches = 0;
   for_state_tiles(K, [&](auto, int, int) { ++launches; });
-  const int64_t line = rows == 3 ? 26000 : rows == 4 ? 16000 : 14000;
-  return K >= (rows == 6 ? kNearGradBf16States : kNearBf16States) && int64_t(d.p2p_tile16_count) * K >= line * launches;
+  const int64_t line = rows == 3 ? 25000 : rows == 4 ? 13000 : 14000;
+  return int64_t(d.p2p_tile16_count) * K >= line * launches;
 }
 
 // The moments' bf16 pieces for the near-field kernels on bf16 operands.
