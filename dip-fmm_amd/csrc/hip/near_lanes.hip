@@ -10,8 +10,9 @@
 // D = (3 r r^T/|r|^5 - I/|r|^3)/(4 pi) of src/cuboid.cpp:293-307 and the
 // potential (m.r)/(4 pi |r|^3) of src/static_operators.cpp:455-463.
 //
-// What bounds it: the pair arithmetic, 33 vector instructions per pair at one
-// state, 26 and 9 per state (10 with the potential) at more.  So the
+// What bounds it: the pair arithmetic, 23 vector instructions per pair and 10
+// per state up to three states, 26 and 9 at more (one more per state with the
+// potential).  So the
 // lanes of a wave are sources and its targets are wave-uniform: a lane keeps
 // one source and its moments in registers for T targets of one leaf, whose
 // coordinates sit in scalar registers, and nothing is staged in LDS.  A batch
@@ -32,14 +33,12 @@
 // leaf, FP32: K = 1 .88 (1.77), 2 1.08 (2.70), 4 1.87 (4.61), 8 3.06 (8.01);
 // fields and potentials K = 4 2.08 (4.72); gradients K = 1 1.25 (2.05).
 // 512 per leaf, 2^18 points: K = 8 6.5.  FP64, 2^18 points, 64 per leaf:
-// K = 1 .60 (1.43).  The tensor's 3 and the potential's u.m once per pair
-// (whole evaluates of 2^20 points, p = 4; in brackets once per state): K = 8
-// 3.99 (4.02), with potentials 4.68 (5.09); 512 per leaf, 2^18 points, K = 8
-// 6.25 (6.51), with potentials 8.07 (9.07).  Taking the 3 as sqrt(3) in both
-// factors saves two instructions per pair (1% at K = 8) and was left for the
-// error it adds (8 sources, 50,000 targets, K = 8, against FP64: median
-// relative error 1.8e-7, mean of the signed errors -0.7e-7; with sqrt(3)
-// 2.0e-7 and -1.0e-7).
+// K = 1 .60 (1.43).  Whole evaluates of 2^20 points, p = 4, K = 8 with the
+// tensor's 3 and the potential's u.m once per pair 4.04, with potentials 4.79
+// (2% and 10% more with both once per state).  Taking the 3 as sqrt(3) in both
+// factors would save two instructions per pair (3.99 and 4.72) for more error
+// (8 sources, 50,000 targets, K = 8, against FP64: median relative error 2.0e-7
+// instead of 1.8e-7, mean of the signed errors -1.0e-7 instead of -0.7e-7).
 #include "common.hpp"
 
 namespace hipfmm {
@@ -249,16 +248,17 @@ __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePla
       } else {
         // f (3 (u.m) u - m) with f = |r|^-3 / (4 pi): no |r|^-5, which overflows
         // for close pairs in FP32.  The 3 is multiplied exactly, once per pair
-        // (with one state, once with u.m); as sqrt(3) in both factors it would be
-        // 3 (1 - 3.6e-8) in FP32, an error of one sign in every pair.  The
-        // potential f r.m is |r|^-2 / (4 pi) u.m.
+        // (three instructions; up to three states, once with each u.m); as
+        // sqrt(3) in both factors it would be 3 (1 - 3.6e-8) in FP32, an error of
+        // one sign in every pair.  The potential f r.m is |r|^-2 / (4 pi) u.m.
+        constexpr bool kWithState = KS <= 3;
         const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
         const S fp = rinv * rinv * S(0.079577471545947667884441881686257181), f = fp * rinv;
-        const S tx = KS == 1 ? ux : S(3) * ux, ty = KS == 1 ? uy : S(3) * uy, tz = KS == 1 ? uz : S(3) * uz;
+        const S tx = kWithState ? ux : S(3) * ux, ty = kWithState ? uy : S(3) * uy, tz = kWithState ? uz : S(3) * uz;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
           const S mx = m[0][k], my = m[1][k], mz = m[2][k];
-          const S w = ux * mx + uy * my + uz * mz, v = KS == 1 ? S(3) * w : w;
+          const S w = ux * mx + uy * my + uz * mz, v = kWithState ? S(3) * w : w;
           a[0 * KS + k] += f * (v * tx - mx);
           a[1 * KS + k] += f * (v * ty - my);
           a[2 * KS + k] += f * (v * tz - mz);
