@@ -127,6 +127,7 @@ struct hipfmm_plan {
   M2lPath last_path = kFullM2l;   // what it ran, for complete_locals
   int last_mode = 0;
   bool last_adjoint = false;
+  bool locals_complete = false;   // complete_locals has run since
   bool last_m2l_expands = false;  // its M2L ends at kEvM2L, after its kernel
   uint64_t m2l_launch_count = 0;
   double m2l_total_seconds = 0.0;
@@ -1133,7 +1134,9 @@ void launch_downward(const DevicePlan& d, const DevicePlan& compressed, int K, h
 }
 
 // The last evaluate's locals of a box that its M2L left out (DevicePlan::
-// target_bits): the M2L and the downward pass again, over every box.
+// target_bits): the M2L and the downward pass again, over every box, once per
+// evaluate.  (A captured evaluate's replays change the locals unseen: after a
+// capture they are formed on every read.)
 template <class S>
 void complete_locals(hipfmm_plan* P, int node) {
   DevicePlan d = P->last_adjoint ? role_exchanged(P) : P->d;
@@ -1141,6 +1144,7 @@ void complete_locals(hipfmm_plan* P, int node) {
   uint32_t word = 0;
   HIPFMM_CHECK(hipMemcpy(&word, d.target_bits + (node >> 5), sizeof(word), hipMemcpyDeviceToHost));
   if ((word >> (node & 31)) & 1u) return;
+  if (P->locals_complete) return;
   d.target_bits = nullptr;
   d.sparse_order = nullptr;
   d.compressed_state_major = state_major<S>(d, P->last_K);
@@ -1149,6 +1153,7 @@ void complete_locals(hipfmm_plan* P, int node) {
   if (d.nc > 0 && !harmonic_passes(d)) hipfmm::launch_m2l_expand<S>(d, P->last_K, 2, P->s_near);
   launch_downward<S>(d, c, P->last_K, P->s_near);
   HIPFMM_CHECK(hipStreamSynchronize(P->s_near));
+  P->locals_complete = P->capture_id == 0;
 }
 
 // Kernels of an evaluate that failed half-way, which no event marks: they end
@@ -1215,6 +1220,7 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   if (captured ? P->capture_id == capture_id : P->done_recorded)
     HIPFMM_CHECK(hipStreamWaitEvent(s, e[captured ? kEvCaptured : kEvL2P], 0));
   SettleOnFailure settle{s, P->s_near, !captured};
+  P->locals_complete = false;
   auto mark = [&](int ev, hipStream_t on) {
     HIPFMM_CHECK(hipEventRecord(e[ev], on));
   };
