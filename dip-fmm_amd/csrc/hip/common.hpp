@@ -382,9 +382,10 @@ void launch_m2l_expand(const DevicePlan& d, int K, int first_level, hipStream_t 
 // operand layout, for plans whose upper levels are formed in compressed form.
 void launch_m2l_bf16_split(const DevicePlan& d, int K, hipStream_t s);
 void launch_m2l_mfma(const DevicePlan& d, int K, int mode, hipStream_t s);   // all levels 2..L
-// Columns per box of the 16-bit M2L operands at K states (the mt buffers hold
-// this many at the largest batch).
+// Columns per box of the 16-bit M2L operands at K states, given the mt buffers,
+// and of buffers for batches of up to K.
 int m2l_operand_states(const DevicePlan& d, int K);
+int m2l_operand_capacity(const DevicePlan& d, int K);
 void prepare_mfma_operators(DevicePlan& d, int n, const std::vector<double>& matrices, int classes,
                             const std::vector<double>& local_scaling, std::vector<void*>& allocations, size_t& bytes);
 // FP16 operators of the harmonic form (n = nc); call after prepare_mfma_operators.

@@ -803,9 +803,19 @@ __global__ void __launch_bounds__(256) split_bf16_kernel(const DevicePlan d, int
 // of 32, so that every 32-column tile is one box and its step runs on the
 // uniform-box path: at 4681 boxes of p = 6 a batch of 12 to 31 states takes
 // 0.41 ms padded and 0.77-1.38 ms with several boxes per tile; up to 8 states
-// (four or more boxes per tile) it takes 0.37 ms.
+// (four or more boxes per tile) it takes 0.37 ms.  Not where the padded columns
+// would not fit that path's 32-bit offsets (or, for a batch below the capacity,
+// the operand buffer): several boxes per tile would then walk the padding too.
+static bool padding_fits(const DevicePlan& d, int K, int64_t bytes) {
+  return d.nc > 0 && K >= 9 && int64_t(d.nodes) * ((K + 31) / 32 * 32) * d.apad * 2 <= bytes &&
+         bytes + 1024 <= int64_t(0xffffffffu);
+}
 int m2l_operand_states(const DevicePlan& d, int K) {
-  return d.nc == 0 || K < 9 ? K : (K + 31) / 32 * 32;
+  return padding_fits(d, K, d.mt_zero_offset) ? (K + 31) / 32 * 32 : K;
+}
+int m2l_operand_capacity(const DevicePlan& d, int K) {
+  const int padded = (K + 31) / 32 * 32;
+  return padding_fits(d, K, int64_t(d.nodes) * padded * d.apad * 2) ? padded : K;
 }
 
 // The boxes whose operands the tiles read: of one box per tile, those with

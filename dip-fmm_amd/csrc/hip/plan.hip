@@ -963,7 +963,7 @@ void ensure_capacity(hipfmm_plan* P, int K, bool potential, bool gradient = fals
     HIPFMM_CHECK(hipMemset(d.Lcc, 0, cc * sizeof(S)));
   }
   if (sizeof(S) == 4 && P->mfma_ready) {
-    const size_t ms = size_t(d.nodes) * hipfmm::m2l_operand_states(d, cap) * d.apad;
+    const size_t ms = size_t(d.nodes) * hipfmm::m2l_operand_capacity(d, cap) * d.apad;
     // Each half is followed by a 1 KiB zero block (the operand of sources
     // outside the grid); zeroed once here.
     d.mt_zero_offset = int64_t(ms) * 2;
