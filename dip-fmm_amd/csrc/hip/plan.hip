@@ -3,9 +3,10 @@
 // Replaces the reference's CudaFullPlan (src/cuda_fmm_plan.hpp:95-114,
 // src/cuda_fmm.cu:2636-3665).  Static data is uploaded once at create; each
 // evaluate enqueues
-//   far stream : gather -> P2M -> M2M (levels L-1..2) -> M2L (levels 2..L)
-//                -> L2L (levels 3..L) -> [wait near] -> L2P + combine + unsort
-//   near stream: [wait gather] -> list-1 P2P
+//   far field, on the caller's stream (host operands, groups: a stream of the
+//   plan's): gather -> P2M -> M2M (levels L-1..2) -> M2L (levels 2..L) -> L2L
+//   (levels 3..L) -> [wait near] -> L2P + combine + unsort
+//   near field, on a stream of the plan's: [wait gather] -> list-1 P2P
 // and, for host operands, exactly one H2D (moments) and one D2H (fields),
 // matching the reference's transfer contract (tests/test_cuda_backend.cpp:
 // 102-105 there).
@@ -1209,10 +1210,10 @@ void evaluate_impl(hipfmm_plan* P, const void* moments, void* fields, void* pote
   const bool host = memspace == HIPFMM_HOST;
   const hipStream_t s = host || fork != nullptr ? far_stream(P) : user;
   hipEvent_t* e = P->ev;
-  // The plan's buffers are free once its last evaluate is done.  An event
-  // recorded inside a capture marks nothing outside it, so a captured evaluate
-  // has one of its own, and follows only those of the same capture (a graph's
-  // replays are the caller's to order).
+  // The plan's buffers are free once its last evaluate is done.  On a stream
+  // under capture an event is recorded into the graph and marks nothing outside
+  // it, so a captured evaluate ends at an event of its own and follows only those
+  // of the same capture (a graph's replays are the caller's to order).
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   unsigned long long capture_id = 0;
   HIPFMM_CHECK(hipStreamGetCaptureInfo(host ? s : user, &capture, &capture_id));

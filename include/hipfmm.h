@@ -175,7 +175,7 @@ typedef struct hipfmm_timings {
   double total_seconds;
   double m2l_kernel_seconds; /* the M2L product kernel alone (one launch, all levels) */
   /* Every M2L kernel launch of the plan so far, each timed with its own HIP
-   * events on the plan's stream: summed durations and launch count (callers
+   * events on the evaluate's stream: summed durations and launch count (callers
    * average over a region by differencing two reads). */
   double m2l_kernel_total_seconds;
   uint64_t m2l_kernel_launches;
@@ -211,8 +211,17 @@ int hipfmm_plan_create(const hipfmm_plan_desc* desc, hipfmm_plan** plan);
  *   (src/cuda_fmm.cu:3470-3486).  NULL reuses the fixed map (none = -1).
  *   stream: hipStream_t to order device-memory work after, or NULL.
  * Host-memory calls return when the fields are in host memory; device-memory
- * calls return once the work is enqueued on the plan's streams and ordered
- * before any later work on `stream`. */
+ * calls return once the work is enqueued, the far field on `stream` itself and
+ * the near field on a stream of the plan's, and ordered before any later work
+ * on `stream`.  Calls on one plan take effect in the order they are made,
+ * whatever their streams; after a call that fails, none of its work is left
+ * running.
+ * A device-memory call on a stream under capture is recorded, if an earlier
+ * call allocated the state for its batch and outputs.  It follows the earlier
+ * evaluates of that capture only, marks the end of its work by an event of its
+ * own, so that evaluates outside the capture never wait for a recorded event,
+ * and has no stage times; the order of the graph's replays with other
+ * evaluates of the plan is the caller's.  The tests do not cover captures. */
 int hipfmm_plan_evaluate(hipfmm_plan* plan, const void* moments, void* fields, int batch,
                          const int* sorted_self_indices, int memspace, void* stream);
 
