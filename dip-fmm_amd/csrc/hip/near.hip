@@ -520,8 +520,8 @@ __device__ __forceinline__ void p2p_repair(const DevicePlan& d, f32x4 (&acc)[kRo
 }
 
 // List-1 P2P on the matrix cores with bf16 operands
-// (v_mfma_f32_16x16x32_bf16), for FP32 plans with K a multiple of 32 (the
-// default there).  Both operands are split in three bf16 pieces (hi + mid +
+// (v_mfma_f32_16x16x32_bf16), for FP32 plans: the default with K a multiple of
+// 32, and other batches as near_on_matrix_cores says.  Both operands are split in three bf16 pieces (hi + mid +
 // lo, 24 significant bits) and the six piece products whose orders sum to at
 // most 2 are kept, D m ~ Dh mh + Dh mm + Dm mh + Dh ml + Dl mh + Dm mm: the
 // dropped ones are below 2^-26 |D m|, under the rounding of FP32 operands.
@@ -792,8 +792,8 @@ __device__ __forceinline__ void grad_bf16_products(f32x4 (&acc)[6][kH], const ui
   p2p_bf16_products(acc[E], ph, pm, pl, b[D]);
 }
 
-// Near-field gradient on bf16 three-piece operands (FP32 plans, K a multiple
-// of 32; the default there): the tiles, the neighbourhood's block list and
+// Near-field gradient on bf16 three-piece operands (FP32 plans: the default
+// with K a multiple of 32, other batches as near_on_matrix_cores says): the tiles, the neighbourhood's block list and
 // the operand layout of p2p_bf16_kernel, with the 10 distinct entries of the
 // symmetric 3-tensor W_cjd = g (delta_cj u_d + delta_jd u_c + delta_cd u_j -
 // 5 u_c u_j u_d), g = 3/(4 pi |r|^4), each split once and multiplied by the

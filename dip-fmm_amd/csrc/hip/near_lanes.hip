@@ -36,9 +36,10 @@
 // K = 1 .60 (1.43).  Whole evaluates of 2^20 points, p = 4, K = 8 with the
 // tensor's 3 and the potential's u.m once per pair 4.04, with potentials 4.79
 // (2% and 10% more with both once per state).  Taking the 3 as sqrt(3) in both
-// factors would save two instructions per pair (3.99 and 4.72) for more error
-// (8 sources, 50,000 targets, K = 8, against FP64: median relative error 2.0e-7
-// instead of 1.8e-7, mean of the signed errors -1.0e-7 instead of -0.7e-7).
+// factors would save two instructions per pair (3.99 and 4.72) for more error:
+// 8 sources, 50,000 targets, K = 8, against FP64, median relative error and mean
+// of the signed errors 1.7e-7 and -0.3e-7; with 1 / (4 pi) rounded into each pair
+// 1.8e-7 and -0.7e-7, with sqrt(3) besides 2.0e-7 and -1.0e-7.
 #include "common.hpp"
 
 namespace hipfmm {
@@ -74,6 +75,12 @@ __device__ __forceinline__ double near_rsqrt(double x) {
   const double e = fma(-(x * y), y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
+
+// A sum of pairs times 4 / pi, to within its rounding.
+__device__ __forceinline__ float near_scale(float x) {
+  return fmaf(x, 1.2732395447351626862f, x * float(1.2732395447351626862 - double(1.2732395447351626862f)));
+}
+__device__ __forceinline__ double near_scale(double x) { return x * 1.2732395447351626862; }
 
 // A wave-uniform value moved to scalar registers.
 __device__ __forceinline__ float uniform(float x) {
@@ -251,9 +258,11 @@ __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePla
         // (three instructions; up to three states, once with each u.m); as
         // sqrt(3) in both factors it would be 3 (1 - 3.6e-8) in FP32, an error of
         // one sign in every pair.  The potential f r.m is |r|^-2 / (4 pi) u.m.
+        // Likewise 1 / (4 pi), which is 4e-8 short in FP32: a pair carries 1 / 16
+        // of it, the sums 4 / pi (near_scale).
         constexpr bool kWithState = KS <= 3;
         const S ux = rx * rinv, uy = ry * rinv, uz = rz * rinv;
-        const S fp = rinv * rinv * S(0.079577471545947667884441881686257181), f = fp * rinv;
+        const S fp = rinv * rinv * S(0.0625), f = fp * rinv;
         const S tx = kWithState ? ux : S(3) * ux, ty = kWithState ? uy : S(3) * uy, tz = kWithState ? uz : S(3) * uz;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
@@ -277,9 +286,9 @@ __global__ void __launch_bounds__(64 * kWaves) near_lanes_kernel(const DevicePla
     if constexpr (kWhat == kGradient)
       static_cast<S*>(d.Gn)[(t * 6 + c) * K + k] = acc[v];
     else if (c < 3)
-      static_cast<S*>(d.Hn)[(t * 3 + c) * K + k] = acc[v];
+      static_cast<S*>(d.Hn)[(t * 3 + c) * K + k] = near_scale(acc[v]);
     else
-      static_cast<S*>(d.Pn)[t * K + k] = acc[v];
+      static_cast<S*>(d.Pn)[t * K + k] = near_scale(acc[v]);
   }
 }
 
