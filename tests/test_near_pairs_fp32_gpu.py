@@ -1,5 +1,5 @@
 """Single FP32 near-field pairs, each target with one source (a depth 0 tree has
-no far field), where the arithmetic of a pair shows: the tensor's factor 3.
+no far field), where the arithmetic of a pair shows: its constant factors.
 """
 
 import numpy as np
@@ -44,3 +44,25 @@ def test_the_axial_field_is_twice_the_transverse(axis, K):
     for a, b in zip(fields[axis], fields[across]):
         assert (b < 0).all()
         np.testing.assert_array_equal(a, -2.0 * b)
+
+
+@pytest.mark.parametrize("K", [1, 3, 8])
+def test_pairs_have_no_common_error(K):
+    # Roundings average out over many pairs; a factor that is off does not.  The
+    # hardware root is 0.7e-8 short on average, thrice in f and once more in each
+    # u of 3 (u.m) u: some 4e-8 of the field, and the roundings' mean over 20,000
+    # targets 1e-9.  One more factor rounded with one sign (1 / (4 pi): 4e-8) is
+    # past 7e-8.
+    rng = np.random.default_rng(K)
+    src = np.array([[0.45, 0.55, 0.5]])
+    tgt = rng.uniform(0, 1, size=(20000, 3))
+    m = rng.normal(size=(K, 1, 3)).astype(np.float32).astype(np.float64)
+    f = plan(src, tgt)
+    r = tgt - src
+    n = np.linalg.norm(r, axis=1, keepdims=True)
+    u = r / n
+    for h in (f.evaluate_batch(m), f.evaluate_batch_outputs(m, output="both")["H"]):
+        for k in range(K):
+            want = (3.0 * (u * m[k]).sum(axis=1, keepdims=True) * u - m[k]) / (4.0 * np.pi * n ** 3)
+            off = ((h[k] - want) * want).sum(axis=1) / (want ** 2).sum(axis=1)
+            assert abs(off.mean()) <= 7e-8
