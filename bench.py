@@ -12,8 +12,9 @@ bf16 hi/lo split operands).  Moments and fields stay in HBM (torch tensors);
 value = N * K * steps / elapsed seconds, the elapsed time between
 synchronisations around the timed steps (the same region timed with HIP
 events on the caller's stream is reported beside it).  The plain path (M2L
-on the vector ALUs in FP32, one moment state per evaluate) is timed on the
-same plan.
+in FP32, on the full-precision matrix instructions, one moment state per
+evaluate) is timed on the same plan; speedup_vs_plain is the batched bf16
+rate over its rate, so it falls as the plain path gets faster.
 
 Accuracy: rel. L2 of the MFMA result (states 0 and K-1) against the FP64 FMM
 at the same (p, depth) (the HipFull FP64 plan, itself checked against
@@ -24,8 +25,8 @@ Roofline: the dominant kernel is the M2L product (one launch over levels
 2..5); its algorithmic work is 2 nc^2 flops per list-2 interaction and moment
 state, nc = 81 at p = 8 (the class matrices factor through the (p+1)^2-
 dimensional harmonic subspace; the reference's form uses n = 165 and is
-reported beside it), timed with HIP events on the plan's stream around that
-launch.
+reported beside it), timed with HIP events on the evaluate's stream around
+that launch.
 
 The other benchmark configurations (C2 plain, C3 precision, C4 batching, C5
 differentiation; dip-fmm_amd/workloads.py) each get a line under "configs":
@@ -248,7 +249,7 @@ def config_c2(hip, torch, stream) -> dict:
     del f64
     e_direct, sample, direct = direct_error(hip, x, x, m0, h0, np.arange(n), W.seed(2))
     res = {
-        "workload": "C2: 2^20 uniform dipoles, targets = sources, p=6, depth 5, FP32, plain HIP path (vector-ALU "
+        "workload": "C2: 2^20 uniform dipoles, targets = sources, p=6, depth 5, FP32, plain HIP path (FP32 "
                     "M2L), 1 state per evaluate, 100 seeded states on a fixed plan, device operands",
         "value": n / sec, "unit": "field evals/s", "ms_per_evaluate": 1e3 * sec, "evaluates": reps,
         "accuracy": {"vs_fp64_fmm_state0": rel_l2(h0, r0), "vs_fp64_fmm_state99": rel_l2(h99, r99),
@@ -260,7 +261,7 @@ def config_c2(hip, torch, stream) -> dict:
 
 def config_c3(hip, torch, stream) -> dict:
     # 2^20 dipoles, 80% in 64 Gaussian blobs, p = 8, depth 6: the four M2L
-    # arithmetics (FP64 plan; FP32 plan with vector-ALU FP32, bf16 hi/lo and
+    # arithmetics (FP64 plan; FP32 plan with full FP32, bf16 hi/lo and
     # fp16 level-scaled hi/lo on the matrix cores) against the FP64 direct
     # sum on 4096 seeded targets.  The matrix-core modes run K = 32 states.
     n, p, depth, K = 1 << 20, 8, 6, 32
@@ -537,12 +538,12 @@ def main() -> int:
         plain = {"value": N / plain_s, "ms_per_evaluate": 1e3 * plain_s, "m2l_kernel_ms": 1e3 * pt["m2l_kernel"]}
         plain_fields = one_f[0].cpu().numpy()
         # The plain path at the headline's batch: the same K = 32 states in
-        # one evaluate with the vector-ALU M2L.
+        # one evaluate with the FP32 M2L.
         s32 = time_device(torch, step, max(1, min(args.plain_steps, 3)))
         plain["k32"] = {"value": N * K / s32, "ms_per_step": 1e3 * s32,
                         "m2l_kernel_ms": 1e3 * fmm.device_timings()["m2l_kernel"]}
         fmm.set_m2l_mode(hip.HipM2LMode.MFMA_BF16X3)
-        log(f"plain VALU K=1: {1e3 * plain_s:.2f} ms/evaluate, {N / plain_s:.3e} evals/s; "
+        log(f"plain FP32 K=1: {1e3 * plain_s:.2f} ms/evaluate, {N / plain_s:.3e} evals/s; "
             f"K={K}: {1e3 * s32:.2f} ms/step")
 
     # The same step with the level-scaled FP16 hi/lo M2L (same MFMA rate,

@@ -46,8 +46,9 @@ enum hipfmm_status {
 
 enum hipfmm_memspace { HIPFMM_HOST = 0, HIPFMM_DEVICE = 1 };
 
-/* M2L arithmetic.  VALU is the plain path (FP32 plans: FP32 FMA; FP64 plans:
- * FP64 FMA).  The MFMA modes exist for FP32 plans only: operands are split
+/* M2L arithmetic.  VALU is the plain path: FMA chains in the plan's own
+ * precision, on the full-precision matrix instructions (on the vector ALUs for
+ * class matrices that do not factor).  The MFMA modes exist for FP32 plans only: operands are split
  * into two 16-bit halves (hi + lo) and three products are accumulated in FP32
  * on the matrix cores.  A small batch that is no multiple of 32 states does not
  * pay for the split: up to 3.5e6 boxes x states x (p+1)^2 with 8 or fewer
