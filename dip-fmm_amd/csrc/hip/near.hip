@@ -704,14 +704,19 @@ void for_state_tiles(int K, F&& launch) {
 //     per leaf, 7 to 63 states: the line is within .3% of the faster kernel on
 //     average, bf16 tiles alone 18 to 25%.  With 512 leaves and more the tiles
 //     alone are within .7% (9728 points, 871 tiles: K = 9 .151 / .145, 30
-//     .406 / .326).
+//     .406 / .326).  On 8 leaves and one, whose vector-ALU waves read every
+//     source, the line is lower: 8 leaves, p = 4, fields: 303 tiles K = 30
+//     .400 / .574, 50 .740 / .617, 1005 tiles K = 12 1.16 / 1.41, 20 2.10 / 1.86;
+//     with potentials 303 tiles K = 16 .280 / .431, 30 .668 / .514; gradients 303
+//     tiles K = 20 .449 / .742, 1005 K = 7 1.56 / 1.51, 9 1.90 / 1.51.
 // rows: outputs per target and state (3, with the potential 4, gradient 6).
 static bool near_on_matrix_cores(const DevicePlan& d, int K, int rows) {
   if (K < (rows == 6 ? kNearGradBf16States : kNearBf16States)) return false;
   if (d.leaves > 64) return true;
   int launches = 0;
   for_state_tiles(K, [&](auto, int, int) { ++launches; });
-  const int64_t line = rows == 3 ? 25000 : rows == 4 ? 13000 : 14000;
+  const bool few = d.leaves <= 8;
+  const int64_t line = rows == 3 ? (few ? 15000 : 25000) : rows == 4 ? (few ? 5500 : 13000) : few ? 7000 : 14000;
   return int64_t(d.p2p_tile16_count) * K >= line * launches;
 }
 

@@ -17,8 +17,8 @@ from test_near_lanes_gpu import direct, gradient, hip  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 SOURCES = 61
-# tiles x states per launch where the line lies on small trees, by output
-LINE = {"field": 25000, "both": 13000, "gradient": 14000}
+# tiles x states per launch where the line lies on trees of 8 leaves, by output
+LINE = {"field": 15000, "both": 5500, "gradient": 7000}
 
 
 def plan(hip, src, tgt, ids):  # noqa: F811
